@@ -282,6 +282,20 @@ int ks_mhc_post(const uint16_t *x, const uint16_t *f, const float *res_logits,
                 const float *post_logits, uint16_t *out, int64_t N, int64_t C,
                 int32_t sinkhorn_iters, float eps, void *stream);
 
+/* The layer input of an mHC block from the streams themselves: the logits
+ *   z = (x[t] flattened, RMS-normalised with norm_eps) @ phi,
+ *   pre = alpha[0] z[0..3] + base[0..3], post = alpha[1] z[4..7] + base[4..7],
+ *   res = alpha[2] z[8..23] + base[8..23],
+ * then h as ks_mhc_pre.  phi: f32 [4 C, 24]; alpha: f32 [3]; base: f32 [24];
+ * post_logits f32 [N, 4] and res_logits f32 [N, 4, 4] are written for
+ * ks_mhc_post.  fp32 sums of exact products; x and h 16-byte aligned.
+ * workspace: ks_mhc_input_workspace_size(N, C) bytes. */
+size_t ks_mhc_input_workspace_size(int64_t N, int64_t C);
+int ks_mhc_input(const uint16_t *x, const float *phi, const float *alpha,
+                 const float *base, uint16_t *h, float *post_logits,
+                 float *res_logits, int64_t N, int64_t C, float norm_eps,
+                 void *workspace, size_t workspace_bytes, void *stream);
+
 /* ------------------------------------------------------------------------
  * ks_sparse_attn without a workspace: allocates nothing.
  *

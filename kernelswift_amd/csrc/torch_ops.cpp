@@ -261,6 +261,31 @@ at::Tensor mhc_pre(const at::Tensor& x, const at::Tensor& pre_logits) {
   return h;
 }
 
+std::tuple<at::Tensor, at::Tensor, at::Tensor> mhc_input(const at::Tensor& x, const at::Tensor& phi,
+                                                         const at::Tensor& alpha, const at::Tensor& base,
+                                                         double norm_eps) {
+  check_streams(x);
+  check_gpu(phi, "phi");
+  check_gpu(alpha, "alpha");
+  check_gpu(base, "base");
+  const int64_t N = x.size(0), C = x.size(2);
+  TORCH_CHECK(phi.scalar_type() == at::kFloat && phi.dim() == 2 && phi.size(0) == 4 * C && phi.size(1) == 24,
+              "phi must be float32 [4 C, 24]");
+  TORCH_CHECK(alpha.scalar_type() == at::kFloat && alpha.dim() == 1 && alpha.size(0) == 3, "alpha must be float32 [3]");
+  TORCH_CHECK(base.scalar_type() == at::kFloat && base.dim() == 1 && base.size(0) == 24, "base must be float32 [24]");
+  const auto f32 = x.options().dtype(at::kFloat);
+  at::Tensor h = at::empty({N, C}, x.options());
+  at::Tensor post = at::empty({N, 4}, f32), res = at::empty({N, 4, 4}, f32);
+  const size_t need = ks_mhc_input_workspace_size(N, C);
+  at::Tensor ws = at::empty({static_cast<int64_t>(need)}, x.options().dtype(at::kByte));
+  check_rc(ks_mhc_input(reinterpret_cast<const uint16_t*>(x.data_ptr()), phi.data_ptr<float>(), alpha.data_ptr<float>(),
+                        base.data_ptr<float>(), reinterpret_cast<uint16_t*>(h.data_ptr()), post.data_ptr<float>(),
+                        res.data_ptr<float>(), N, C, static_cast<float>(norm_eps), ws.data_ptr(), need,
+                        current_stream(x)),
+           "ks_mi355x::mhc_input");
+  return {h, post, res};
+}
+
 at::Tensor mhc_post(const at::Tensor& x, const at::Tensor& f, const at::Tensor& res_logits,
                     const at::Tensor& post_logits, int64_t sinkhorn_iters, double eps) {
   check_streams(x);
@@ -303,6 +328,8 @@ TORCH_LIBRARY(ks_mi355x, m) {
   m.def("indexer_fp8(Tensor q, Tensor q_scale, Tensor k, Tensor k_scale, Tensor weights, int k_top, bool causal, "
         "int start_pos, int ratio=1, int offset=0, bool out_i64=False, int? T=None) -> Tensor");
   m.def("mhc_pre(Tensor x, Tensor pre_logits) -> Tensor");
+  m.def("mhc_input(Tensor x, Tensor phi, Tensor alpha, Tensor base, float norm_eps=1e-06) -> "
+        "(Tensor, Tensor, Tensor)");
   m.def("mhc_post(Tensor x, Tensor f, Tensor res_logits, Tensor post_logits, int sinkhorn_iters=20, "
         "float eps=1e-06) -> Tensor");
 }
@@ -317,5 +344,6 @@ TORCH_LIBRARY_IMPL(ks_mi355x, CUDA, m) {
   m.impl("fp8_quant", &fp8_quant);
   m.impl("indexer_fp8", &indexer_fp8);
   m.impl("mhc_pre", &mhc_pre);
+  m.impl("mhc_input", &mhc_input);
   m.impl("mhc_post", &mhc_post);
 }

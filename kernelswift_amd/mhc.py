@@ -8,13 +8,15 @@ x [N, 4, C], and computes per token, from the RMS-normalised flattened streams,
 the layer input h = sigmoid(pre) . x runs in ks_mhc_pre, and the residual update
     x' = Sinkhorn(res) x + 2 sigmoid(post) f(h)
 in ks_mhc_post, whose kernel normalises each token's 4x4 logits in registers (the Sinkhorn of
-torch.ops.ks_mi355x.sinkhorn, repeat = hc_sinkhorn_iters) and mixes the streams in the same pass.  The
-logit projection stays a torch GEMM, as the reference keeps its projections in torch.
+torch.ops.ks_mi355x.sinkhorn, repeat = hc_sinkhorn_iters) and mixes the streams in the same pass.  Where nothing
+has to be differentiated or traced, the logits are formed on the way too (ks_mhc_input); otherwise they stay torch
+operations (`logits`), through which gradients reach phi, alpha and base.
 """
 from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -43,8 +45,26 @@ class HyperConnection(nn.Module):
         res = (self.alpha[2] * z[:, 2 * n:] + self.base[2 * n:]).view(-1, n, n)
         return pre.contiguous(), post.contiguous(), res.contiguous()
 
+    def _fused(self, x: torch.Tensor) -> bool:
+        """Whether `pre` may form the logits inside the kernel: plain contiguous tensors of the kernel's types on one
+        GPU, with no gradient (reverse or forward mode), autocast, vmap or trace that has to see the torch operations."""
+        ts = (x, self.phi, self.alpha, self.base)
+        if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.maybe_current_level() is not None:
+            return False
+        if torch.is_autocast_enabled() or forward_ad._current_level >= 0:
+            return False
+        if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+            return False
+        return (all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.device == x.device and t.is_contiguous()
+                    for t in ts)
+                and x.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[0] > 0 and x.shape[1:] == (4, self.dim)
+                and self.dim % 8 == 0 and all(t.dtype == torch.float32 for t in ts[1:])
+                and self.phi.shape == (4 * self.dim, 24) and self.alpha.shape == (3,) and self.base.shape == (24,))
+
     def pre(self, x: torch.Tensor):
         """The layer input h bf16 [N, C] and the logits the residual update needs."""
+        if self._fused(x):
+            return _lib.torch_ops().mhc_input(x, self.phi, self.alpha, self.base, self.norm_eps)
         pre, post, res = self.logits(x)
         return _lib.torch_ops().mhc_pre(x, pre), post, res
 
