@@ -10,10 +10,9 @@
 // per key row), which measured twice as slow as the separate pass.
 //
 // With 64 heads, D = 128 and fp32 weights the scores are computed with bounds instead of exactly: the
-// score kernel keeps the canonical score of the lower interval ends plus a per-score bound, and the top-k
-// kernel recomputes exactly only the scores whose interval reaches its selection threshold.  The selected
-// indices are identical to those of the exact path (same intervals, same exact recomputation, same
-// canonical sums wherever a score can matter); the exact path runs every other shape.
+// score kernel keeps an approximate score and a bound on its error, and the top-k kernel recomputes exactly only the
+// scores whose interval reaches its selection threshold.  The selected indices are identical to those of the exact
+// path (the same canonical sums wherever a score can matter); the exact path runs every other shape.
 #include "common.h"
 #include "indexer_common.h"
 
@@ -128,7 +127,8 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
     const int64_t kbs = direct ? f8.kbs : T;
     rc = ks::launch_indexer_scores(ws.q_rot, krows, w, 0, ws.q_norm, ws.q_span, ws.k_norm, ws.k_span, ws.scores, B, S,
                                    H, D, T, kbs, causal ? 1 : 0, start_pos, ratio, bound_c, nullptr, st, ws.bounds,
-                                   ws.kmax, counted ? ks::topk_bounded_counts(ws.part, B * S, T) : nullptr, f8.ks);
+                                   ws.kmax, counted ? ks::topk_bounded_counts(ws.part, B * S, T) : nullptr,
+                                   ks::topk_bounded_state(ws.part, B * S, T, counted), f8.ks);
     if (rc != KS_OK) return rc;
     ks::TopkRecompute trc{ws.bounds, ws.kmax, ws.q_rot, ws.k_rot, static_cast<const float *>(w), ws.q_norm,
                           ws.q_span, ws.k_norm, ws.k_span, kbs, bound_c, stats, path == 3 ? 1 : 0, ws.part,
@@ -143,7 +143,7 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
   const ks::QSplit qs{rot_hi > rot_lo ? ws.q_rot : nullptr, rot_lo, rot_hi};
   rc = ks::launch_indexer_scores(q_unrot != nullptr ? q_unrot : ws.q_rot, ws.k_rot, w, w_bf16 ? 1 : 0, ws.q_norm,
                                  ws.q_span, ws.k_norm, ws.k_span, ws.scores, B, S, H, D, T, T, causal ? 1 : 0,
-                                 start_pos, ratio, bound_c, stats, st, nullptr, nullptr, nullptr, nullptr,
+                                 start_pos, ratio, bound_c, stats, st, nullptr, nullptr, nullptr, nullptr, nullptr,
                                  q_unrot != nullptr ? &qs : nullptr);
   if (rc != KS_OK) return rc;
   // bf16 weights: the exact scores are rounded to bf16, so the top-k may take them as bf16 values

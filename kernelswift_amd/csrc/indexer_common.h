@@ -12,6 +12,26 @@ __device__ __forceinline__ uint32_t score_key(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// Buckets of the bounded selection's threshold histogram: 2048, monotone in score_key, logarithmic in the magnitude m
+// (bits without the sign) with 64 per octave over the 16 octaves below the row's scale M (bits of a magnitude that the
+// row's scores rarely exceed; any value is correct): positive values 1024 .. 2047, negative ones 1023 .. 0, larger
+// magnitudes clamped to the outermost bucket, smaller ones to the two middle ones.  The key's own top bits would give
+// 4 buckets per octave in 11 bits, which at N(0, 1) inputs puts a tenth more keys above the threshold.
+__device__ __forceinline__ uint32_t bound_digit(float lo, uint32_t M) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, lo), m = u & 0x7FFFFFFFu;
+  const uint32_t d = min(M > m ? (M - m) >> 17 : 0u, 1023u);
+  return (u >> 31) ? d : 2047u - d;
+}
+// The smallest nonzero key that a value of bucket d can have (so that no value of bucket d or above lies below it).
+__device__ __forceinline__ uint32_t bound_digit_edge(uint32_t d, uint32_t M) {
+  if (d >= 1024u) {  // m > M - ((dd + 1) << 17), or any m down to zero in the last bucket
+    const uint32_t dd = 2047u - d, low = (dd + 1u) << 17;
+    return 0x80000000u | (dd < 1023u && M >= low ? M - low + 1u : 0u);
+  }
+  // m <= M - (d << 17), or any m in the first bucket
+  return d == 0u ? 1u : ~(0x80000000u | (M >= (d << 17) ? M - (d << 17) : 0u));
+}
+
 // Exponent of the least significant bit of a nonzero bf16 value: value = m * 2^lsb, m integer.
 __host__ __device__ inline int bf16_lsb_exponent(uint16_t b) {
   const int e = (b >> 7) & 0xFF;
@@ -287,13 +307,11 @@ struct Fp8RowJob {
 int launch_fp8_rows(const Fp8RowJob &job0, const Fp8RowJob &job1, int D, hipStream_t stream, void *zero = nullptr,
                     int64_t zero16 = 0);
 
-// Exact scores (bounds == nullptr), or, with bounds (H = 64, D = 128, fp32 weights), the canonical score from
-// the lower interval end of every dot plus a per-score bound U: the exact score lies in [score - U,
-// score + U], both ends also after rounding to nearest, and U = 0 exactly when the score is exact.  kmax
-// [B][ceil(T / kScoreKeyBlock)] then receives each key block's key-norm maximum (the interval half-width
-// of a dot is bound_c 2^-23 ||q_h|| kmax), for an exact recomputation with the same intervals, and
-// row_counts [B S][2048] (zero on entry; may be null) is incremented by each row's counts of the first 11-bit
-// digit of score_key(lower end) over its valid columns (the bounded selection's threshold histogram).  With
+// Exact scores (bounds == nullptr), or, with bounds (H = 64, D = 128), a score and a bound U: the exact score lies in
+// [score - U, score + U], both ends also after rounding to nearest.  kmax [B][ceil(T / kScoreKeyBlock)] then receives
+// each key block's key-norm maximum (the interval half-width of a dot is bound_c 2^-23 ||q_h|| kmax), for the exact
+// recomputation, row_state [B S][4] the scale of each row's threshold histogram (word 3), and row_counts [B S][2048]
+// (zero on entry; may be null) is incremented by each row's counts of bound_digit(lower end) over its valid columns.  With
 // ksc (bound mode, 64 heads, D = 128), k holds e4m3 codes with those row scales (FP8 keys), read directly; kn /
 // ksp are the statistics of the dequantised rows.
 constexpr int kScoreKeyBlock = 256;
@@ -314,8 +332,8 @@ int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, i
                           const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B,
                           int64_t S, int64_t H, int64_t D, int64_t T, int64_t kbs, int causal, int64_t start_pos,
                           int ratio, float bound_c, uint32_t *stats, hipStream_t stream, float *bounds = nullptr,
-                          float *kmax = nullptr, uint32_t *row_counts = nullptr, const float *ksc = nullptr,
-                          const QSplit *qsplit = nullptr);
+                          float *kmax = nullptr, uint32_t *row_counts = nullptr, uint32_t *row_state = nullptr,
+                          const float *ksc = nullptr, const QSplit *qsplit = nullptr);
 
 // Sorted exact top-k of rows of bounded scores (the bound-emitting score kernel's output): a threshold from the
 // lower ends, exact recomputation of the scores that may reach the top k (interval test with the score kernel's
@@ -354,6 +372,9 @@ int64_t topk_bounded_part_capacity(int64_t rows, int64_t T);
 // ([rows][4] 32-bit), kTopkCountWords 32-bit words per row in all, to be cleared before the score kernel.
 constexpr int64_t kTopkCountWords = 2048 + 4;
 uint32_t *topk_bounded_counts(uint64_t *part, int64_t rows, int64_t T);
+// The row states in part ([rows][4]: list length, tau, largest key bound, histogram scale), for the counted form or
+// the one whose histogram launch counts column slices.  The score kernel writes the scale.
+uint32_t *topk_bounded_state(uint64_t *part, int64_t rows, int64_t T, bool counted);
 // ks_indexer_topk with the caller's guarantee that every score is a bf16 value (bf16_vals = 1), which spares the
 // one-wave-per-row form its check of the keys' low halves.
 int indexer_topk_impl(const float *scores, int64_t ld, int64_t B, int64_t S, int64_t T, int64_t k, int32_t causal,

@@ -29,10 +29,10 @@
 // accumulator (exact_dot_wide_bf16) computes the dot.  A wave whose norms could overflow inside the MFMA
 // ((||q|| ||k|| >= 2^126) treats every dot as a near tie.
 //
-// Bound mode (BOUND) keeps the interval test but writes, instead of recomputing near ties, the canonical score
-// of the lower interval ends and a bound U on its distance from the exact score; its counting form (COUNT) also
-// builds each row's histogram of the first 11-bit digit of the lower ends' keys for the bounded top-k's
-// threshold (per-wave LDS counts, flushed with one global atomic per nonzero bucket).
+// Bound mode (BOUND, bounded_scores) writes an approximate score and a bound U on its distance from the exact one, for a
+// selection that needs only the scores of its top k exactly; its counting form (COUNT) also builds each row's histogram
+// of the lower ends for the bounded top-k's threshold (per-wave LDS counts, flushed with one global atomic per nonzero
+// bucket).
 //
 // FP8 keys (F8, bound mode): k holds e4m3 codes with one fp32 scale per row, read directly (half the bytes of
 // bf16 rows) and dequantised in registers to the bf16 rows the contract defines, bf16(fp32(value * scale)), before
@@ -313,30 +313,284 @@ __device__ void flush_entries(ScoresLds<KD, HT> &L, int wave, int lane, int nent
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Shared memory of the bound-emitting variant: the key block and the per-wave norm maxima only (no
-// deferred-key entries, no dot lists, no row statistics), and in the counting form each wave's counts of its
-// row's lower ends (2048 buckets as 16-bit halves: a wave counts at most kKR keys).  The counts take the LDS
-// of a second workgroup per CU, so the counting form is for grids of one round.
+// Shared memory of the bound-emitting form: the key block, each wave's head weights as bf16 values (high part, low part,
+// upper bound of |w|), and in the counting form each wave's counts of its row's lower ends (2048 buckets as 16-bit
+// halves: a wave counts at most kKR keys).  The counts take the LDS of a second workgroup per CU, so the counting form
+// is for grids of one round.
 template <int KD, bool COUNT>
 struct ScoresLdsBound {
   uint4 k[kKR * KD / 8];
   uint32_t cnt[COUNT ? kQW : 0][1024];
-  float knorm[kKR];
-  int32_t kspan[kKR];
-  int32_t qspan[kQW][64];
-  float qnorm[kQW][64];
-  float dl[kQW][64];
-  float w[kQW][64];
-  uint16_t wup[kQW][64];  // |w| rounded up to bf16, for the bound MFMAs
+  uint16_t wf[kQW][4][64];  // rows hi, lo, |w| up, zero
 };
 
-// Waves per SIMD a kernel form is built for.  The non-counting bound kernel runs grids of several workgroups per
-// CU: at most 168 VGPRs (three waves per SIMD) let the next workgroup start as soon as one wave per SIMD of the
-// current one has finished.  The exact kernel at 16 heads of 64 dims (the drop-in shape: 4 dots per lane and tile,
-// a tile one chain of dependent steps) at up to 128 VGPRs and 57 KiB of LDS holds two workgroups per CU: four waves per
-// SIMD hide each other's tile latency, and one workgroup's prologue loads overlap the other's tiles.
+// Waves per SIMD a kernel form is built for.  The non-counting bound kernel runs grids of several workgroups per CU: at
+// up to 128 VGPRs and 70 KiB of LDS two of them share a CU, so that one's prologue loads overlap the other's tiles (64
+// queries x 32768 keys: 40.7 us, against 49.1 at 147 VGPRs with the next tile's MFMAs issued a tile ahead).  The exact
+// kernel at 16 heads of 64 dims (the drop-in shape: 4 dots per lane and tile, a tile one chain of dependent steps) at
+// up to 128 VGPRs and 57 KiB of LDS does the same: four waves per SIMD hide each other's tile latency.
 template <int HT, int KD, bool BOUND, bool COUNT>
-constexpr int score_waves() { return (BOUND && !COUNT) ? 3 : (!BOUND && HT == 1 && KD == 64) ? 4 : 1; }
+constexpr int score_waves() { return (BOUND && !COUNT) ? 4 : (!BOUND && HT == 1 && KD == 64) ? 4 : 1; }
+
+// e4m3 key chunks of the staging loop, dequantised to the contract's bf16 rows: 16 codes per load, rows past nk zero.
+template <int KD, int NV>
+__device__ __forceinline__ void stage_fp8_keys(uint4 *kl, const uint4 (&kv)[NV], const float (&ksv)[NV], int tid, int nk) {
+  constexpr int kC = KD / 8;
+  // one conversion form for the whole wave: the one-instruction form when every scale it holds allows it
+  bool p2 = true;
+#pragma unroll
+  for (int it = 0; it < NV; ++it) p2 = p2 & fp8_scale_pow2(ksv[it]);  // no short-circuit: no branches
+  p2 = __builtin_amdgcn_ballot_w64(!p2) == 0ull;
+  auto stage = [&](auto POW2) {
+#pragma unroll
+    for (int it = 0; it < NV; ++it) {
+      const int lin = it * kThreads + tid;
+      const int kr = lin / (kC / 2), ch = 2 * (lin % (kC / 2));
+      const uint32_t msk = kr < nk ? 0xFFFFFFFFu : 0u;
+      const uint4 lo = fp8_dequant8<decltype(POW2)::value>(make_uint2(kv[it].x, kv[it].y), ksv[it]);
+      const uint4 hi = fp8_dequant8<decltype(POW2)::value>(make_uint2(kv[it].z, kv[it].w), ksv[it]);
+      kl[kr * kC + (ch ^ (kr & (kC - 1)))] = make_uint4(lo.x & msk, lo.y & msk, lo.z & msk, lo.w & msk);
+      kl[kr * kC + ((ch + 1) ^ (kr & (kC - 1)))] = make_uint4(hi.x & msk, hi.y & msk, hi.z & msk, hi.w & msk);
+    }
+  };
+  if (p2)
+    stage(std::true_type{});
+  else
+    stage(std::false_type{});
+}
+
+// Sum of a value over the 64 lanes (the same bits in every lane: each exchange adds the same two values).
+__device__ __forceinline__ float wave_sum_f32(float x) {
+#define KS_ADD(S_) x += __builtin_bit_cast(float, lane_xor<S_>(__builtin_bit_cast(uint32_t, x)));
+  KS_ADD(32) KS_ADD(16) KS_ADD(8) KS_ADD(4) KS_ADD(2) KS_ADD(1)
+#undef KS_ADD
+  return x;
+}
+
+// The bound-emitting form (64 heads): per (query, key) a score S and a bound U with |exact score - S| <= U, for a
+// selection that computes exactly only the scores that can reach its top k.  No dot is certified here: with A the MFMA
+// sum of a dot, p = max(bf16(A), 0) is within one bf16 rounding of each side of the exact relu'd value r,
+//   |p - r| <= delta + 2^-8 |A| + 2^-8 (|A| + delta) <= 2^-7 (1 + 2^-7) p + (1 + 2^-7) delta      (delta: dot_halfwidth;
+// for A <= 0, p = 0 and r <= (1 + 2^-8) delta), so that
+//   S = sum_h w_h p_h,   U = c1 sum_h w_up p_h + sum_h w_up delta_h + c2 |S|,
+// w_up a bf16 value >= |w_h| (and >= 2^-110 where w_h != 0, so that the low part of a tiny weight, lost below the bf16
+// range, stays under 2^-24 w_up).  The head sums run on the MFMA too: p packs into the B operand as it is (lane (key, g)
+// holds the heads of k-slots 8 g .. + 7), and the A operand's rows hold w's high and low bf16 parts and w_up.  Products
+// are exact and the sums lose under 2^-19 of w_up p; w - hi - lo is under 2^-16 |w|.
+//   c1 = 2^-7 (1 + 2^-4) covers (1 + 2^-7) with those and the canonical sum's own roundings (2^-18 of |w| r);
+//   bf16 weights: each product and the score are rounded to bf16, 2^-8 of |w| r and of |S| + U more:
+//   c1 = (2^-7 + 2^-8)(1 + 2^-4), c2 = 2^-8 (1 + 2^-4) in place of c2 = 2^-21 (the ends S -/+ U may be rounded).
+// Four 16-key tiles share one accumulator: tile j's A operand holds the weight rows at 4 j .. 4 j + 2 and zeros
+// elsewhere, so that lane (l16, g) ends with the sums of key 16 g + l16 and the epilogue serves 64 keys at once.
+// Against certifying every dot (two interval ends per dot, a rounding test and the canonical sum in VALU: ~105 VALU
+// instructions per tile, VALU-bound: 71.9 us at 64 queries x 32768 keys), this takes ~45; 40.7 us, 844 TFLOP/s, the
+// matrix cores busy ~45% of it (18 MFMAs per tile, 17.7 us of them) and the rest the workgroups' prologues (the block's
+// 64 KiB of keys and 128 KiB of query rows).  128 queries x 4096 keys, one workgroup per CU: 23.7 -> 21.0 us.
+template <bool WBF, bool COUNT, bool F8>
+__device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, const uint16_t *__restrict__ q,
+                                               const uint16_t *__restrict__ k, const void *__restrict__ w,
+                                               const float *__restrict__ qn, const float *__restrict__ kn,
+                                               float *__restrict__ scores, int64_t S, int T, int64_t kbs, int causal,
+                                               int64_t start_pos, int ratio, float bound_c, float *__restrict__ bounds,
+                                               float *__restrict__ kmax, uint32_t *__restrict__ row_counts,
+                                               uint32_t *__restrict__ row_state, const float *__restrict__ ksc, int kblk,
+                                               int qgrp) {
+  constexpr int KD = 128, HT = 4, H = 64, kC = KD / 8;
+  const uint8_t *__restrict__ k8 = reinterpret_cast<const uint8_t *>(k);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int64_t b = blockIdx.z;
+  const int kb0 = kblk * kKR;
+  const int nk = min(kKR, T - kb0);
+  const int64_t s = static_cast<int64_t>(qgrp) * kQW + wave;
+  const bool s_ok = s < S;
+  const int64_t krow0 = b * kbs + kb0;  // first key row of this workgroup
+
+  // Every prologue load goes out before the first wait, the key block ahead of every q load of the workgroup (the
+  // memory pipeline serves a CU's loads in issue order); indices are clamped, values masked afterwards.
+  const int64_t qrow0 = (b * S + (s_ok ? s : 0)) * H;
+  const float *__restrict__ knb = kn + krow0;
+  float kn4[kKR / 64];
+#pragma unroll
+  for (int j = 0; j < kKR / 64; ++j) {
+    const int kj = lane + 64 * j;
+    kn4[j] = knb[static_cast<uint32_t>(kj < nk ? kj : nk - 1)];
+  }
+  // 64 norms spread over the batch's keys: the scale of the row's histogram (the same for every key block)
+  const float kns = (kn + b * kbs)[static_cast<uint32_t>((static_cast<int64_t>(lane) * T) >> 6)];
+  const float qn_v = (qn + qrow0)[static_cast<uint32_t>(lane)];
+  const float w_v = WBF ? bf16_to_f32((static_cast<const uint16_t *>(w) + qrow0)[static_cast<uint32_t>(lane)])
+                        : (static_cast<const float *>(w) + qrow0)[static_cast<uint32_t>(lane)];
+  constexpr int kKL = kKR * kC / kThreads;  // 16-byte key chunks per thread (F8: kKL / 2 loads of 16 codes)
+  constexpr int kKV = F8 ? kKL / 2 : kKL;
+  uint4 kv[kKV];
+  float ksv[F8 ? kKV : 1];
+#pragma unroll
+  for (int it = 0; it < kKV; ++it) {
+    const int lin = it * kThreads + tid;
+    if constexpr (F8) {
+      const int kr = lin / (kC / 2), ch2 = lin % (kC / 2);
+      const int64_t row = krow0 + (kr < nk ? kr : nk - 1);
+      kv[it] = *reinterpret_cast<const uint4 *>(k8 + row * KD + ch2 * 16);
+      ksv[it] = ksc[row];
+    } else {
+      const int kr = lin / kC, ch = lin % kC;
+      kv[it] = *reinterpret_cast<const uint4 *>(k + krow0 * KD + static_cast<uint32_t>((kr < nk ? kr : nk - 1) * KD + ch * 8));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  uint4 qa[HT][KD / 32];  // query rows as MFMA A-fragments, loaded in the order the first tile uses them
+#pragma unroll
+  for (int kk = 0; kk < KD / 32; ++kk)
+#pragma unroll
+    for (int m = 0; m < HT; ++m)
+      qa[m][kk] = *reinterpret_cast<const uint4 *>(q + qrow0 * KD + static_cast<uint32_t>((16 * m + l16) * KD + 32 * kk + 8 * g));
+
+  float knm = 0.f;
+#pragma unroll
+  for (int j = 0; j < kKR / 64; ++j) knm = fmaxf(knm, lane + 64 * j < nk ? kn4[j] : 0.f);
+  knm = wave_max_f32(knm);
+  // lane h: head h's weight parts and its share of the row's bound
+  const uint16_t up16 = w_v == 0.f ? 0 : max(bf16_abs_round_up(w_v), static_cast<uint16_t>(17 << 7));  // 2^-110
+  const float up = bf16_to_f32(up16);
+  const float hi = bf16_to_f32(static_cast<uint16_t>(cvt_pk_bf16(w_v, w_v) & 0xFFFFu));
+  L.wf[wave][0][lane] = static_cast<uint16_t>(__builtin_bit_cast(uint32_t, hi) >> 16);
+  L.wf[wave][1][lane] = WBF ? 0 : static_cast<uint16_t>(cvt_pk_bf16(w_v - hi, 0.f) & 0xFFFFu);
+  L.wf[wave][2][lane] = up16;
+  L.wf[wave][3][lane] = 0;
+  const float dl = dot_halfwidth(qn_v, knm, bound_c);
+  const bool forced = __builtin_amdgcn_ballot_w64(dl == __builtin_inff()) != 0ull;
+  const float dsum = wave_sum_f32(up * dl) * 1.03125f;  // sum_h w_up delta_h, (1 + 2^-7) and the fp32 sums covered
+  const uint32_t mrow = __builtin_bit_cast(uint32_t, wave_sum_f32(up * qn_v) * wave_max_f32(kns)) & 0x7FFFFFFFu;
+
+  if constexpr (F8) {
+    stage_fp8_keys<KD>(L.k, kv, ksv, tid, nk);
+  } else {
+    // rows past T are zeroed: with the loaded values used only by the LDS stores, the compiler would sink their loads
+    // below the q loads and the load-ordering barrier (a CPU test checks the placement in the compiled code)
+#pragma unroll
+    for (int it = 0; it < kKL; ++it) {
+      const int lin = it * kThreads + tid;
+      const int kr = lin / kC, ch = lin % kC;
+      const uint32_t msk = kr < nk ? 0xFFFFFFFFu : 0u;
+      L.k[kr * kC + (ch ^ (kr & (kC - 1)))] = make_uint4(kv[it].x & msk, kv[it].y & msk, kv[it].z & msk, kv[it].w & msk);
+    }
+  }
+  if constexpr (COUNT) {  // this wave's lower-end counts start at zero
+#pragma unroll
+    for (int i = 0; i < 4; ++i) reinterpret_cast<uint4 *>(L.cnt[wave])[lane + 64 * i] = make_uint4(0, 0, 0, 0);
+  }
+  // the only barrier past the load ordering: LDS writes done, no wait for the q loads
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  // the block's key-norm maximum for the exact recomputation (every query group writes the same value)
+  if (tid == 0) kmax[b * gridDim.x + kblk] = knm;
+  if (!s_ok) return;
+  if (kblk == 0 && lane == 0) row_state[4 * (b * S + s) + 3] = mrow;
+
+  const int64_t limit = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
+  const int limit32 = static_cast<int>(limit < INT32_MAX ? limit : INT32_MAX);  // keys are below T < 2^31
+  float *orow = scores + (b * S + s) * T;
+  float *urow = bounds + (b * S + s) * T;
+  const int64_t lim_rel = limit - kb0;
+  const int nlk = lim_rel <= 0 ? 0 : (lim_rel < nk ? static_cast<int>(lim_rel) : nk);  // live keys of the block
+  const int nlive = (nlk + 15) / 16;
+
+  // the head-sum A operand before its rows are masked per tile: row l16 holds part l16 & 3 of the weights of heads
+  // 16 m + 4 g + 0 .. 3 (m = 2 hh, 2 hh + 1)
+  uint4 wa[2];
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    const uint32_t *wr = reinterpret_cast<const uint32_t *>(L.wf[wave][l16 & 3]);
+    const int h0 = 32 * hh + 4 * g, h1 = h0 + 16;
+    wa[hh] = make_uint4(wr[h0 / 2], wr[h0 / 2 + 1], wr[h1 / 2], wr[h1 / 2 + 1]);
+  }
+  auto tile_b = [&](int t, uint4(&bv)[KD / 32]) {
+    const int key_l = 16 * t + l16;
+#pragma unroll
+    for (int kk = 0; kk < KD / 32; ++kk) bv[kk] = L.k[key_l * kC + ((4 * kk + g) ^ (key_l & (kC - 1)))];
+  };
+  auto tile_mfma = [&](const uint4(&bv)[KD / 32], f32x4_t(&acc)[HT]) {
+#pragma unroll
+    for (int m = 0; m < HT; ++m) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KD / 32; ++kk)
+#pragma unroll
+      for (int m = 0; m < HT; ++m) acc[m] = mfma16(qa[m][kk], bv[kk], acc[m]);
+  };
+  constexpr float kC1 = WBF ? (0x1p-7f + 0x1p-8f) * 1.0625f : 0x1p-7f * 1.0625f;
+  constexpr float kC2 = WBF ? 0x1p-8f * 1.0625f : 0x1p-21f;
+  // the sums of 64 keys (lane: key key_l) stored, masked and counted
+  auto emit = [&](int key_l, f32x4_t sums) {
+    const int key = kb0 + key_l;
+    float sc = sums[0] + sums[1];
+    float u = __builtin_fmaf(kC2, fabsf(sc), __builtin_fmaf(kC1, sums[2], dsum)) + 0x1p-120f;
+    if (forced || !(fabsf(sc) + u < 3e38f)) {  // no statement about the score: it is always recomputed
+      sc = 0.f;
+      u = __builtin_inff();
+    }
+    const bool live = key_l < nlk;
+    if (key_l < nk) {
+      orow[static_cast<uint32_t>(key)] = live ? sc : -INFINITY;
+      urow[static_cast<uint32_t>(key)] = live ? u : 0.f;
+    }
+    if (COUNT && live) {
+      const uint32_t d = bound_digit(sc - u, mrow);
+      atomicAdd(&L.cnt[wave][d >> 1], 1u << ((d & 1u) * 16u));
+    }
+  };
+  if (nlive > 0) {
+    // tiles past the last live one repeat it (their keys are masked)
+    const int last = nlive - 1;
+    uint4 bv[KD / 32];
+    tile_b(0, bv);
+    for (int t0 = 0; t0 < nlive; t0 += 4) {
+      f32x4_t sums = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = t0 + j;
+        f32x4_t acc[HT];
+        tile_mfma(bv, acc);
+        tile_b(t + 1 < nlive ? t + 1 : last, bv);
+        uint32_t p[2 * HT];
+#pragma unroll
+        for (int m = 0; m < HT; ++m)
+#pragma unroll
+          for (int rp = 0; rp < 2; ++rp) p[2 * m + rp] = cvt_relu_pk(acc[m][2 * rp], acc[m][2 * rp + 1]);
+        uint64_t rows = 0x000F000F000F000Full << (4 * j);  // lanes with l16 in 4 j .. 4 j + 3
+        asm volatile("" : "+s"(rows));  // the masked operands stay in the loop: hoisted, they would take 32 registers
+        const bool in = __builtin_amdgcn_inverse_ballot_w64(rows);
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          const uint4 wj = make_uint4(in ? wa[hh].x : 0u, in ? wa[hh].y : 0u, in ? wa[hh].z : 0u, in ? wa[hh].w : 0u);
+          sums = mfma16(wj, make_uint4(p[4 * hh], p[4 * hh + 1], p[4 * hh + 2], p[4 * hh + 3]), sums);
+        }
+      }
+      emit(16 * t0 + lane, sums);
+    }
+  }
+  // keys past the last group of live tiles (at or past the causal limit)
+  for (int key_l = 64 * ((nlive + 3) / 4) + lane; key_l < nk; key_l += 64) {
+    orow[static_cast<uint32_t>(kb0 + key_l)] = -INFINITY;
+    urow[static_cast<uint32_t>(kb0 + key_l)] = 0.f;
+  }
+  if constexpr (COUNT) {
+    // the wave's counts into its row's histogram (only the nonzero buckets)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    uint32_t *hrow = row_counts + (b * S + s) * 2048;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int wd = lane + 64 * i;
+      const uint32_t v = L.cnt[wave][wd];
+      if (v & 0xFFFFu) atomicAdd(&hrow[2 * wd], v & 0xFFFFu);
+      if (v >> 16) atomicAdd(&hrow[2 * wd + 1], v >> 16);
+    }
+  }
+}
 
 template <int HT, int KD, bool WBF, bool BOUND, bool COUNT = false, bool F8 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(score_waves<HT, KD, BOUND, COUNT>()))) void
@@ -346,21 +600,19 @@ indexer_scores_kernel(
     const int32_t *__restrict__ ksp, float *__restrict__ scores, int64_t S, int T, int64_t kbs, int causal,
     int64_t start_pos, int ratio, float bound_c, uint32_t *__restrict__ stats, int xcd_pk,
     float *__restrict__ bounds, float *__restrict__ kmax, uint32_t *__restrict__ row_counts,
-    const float *__restrict__ ksc, float bound_r, const uint16_t *__restrict__ qsplit_rot, int qsplit_lo,
+    uint32_t *__restrict__ row_state, const float *__restrict__ ksc, float bound_r, const uint16_t *__restrict__ qsplit_rot, int qsplit_lo,
     int qsplit_hi) {
   constexpr int H = HT * 16;
   constexpr int kC = KD / 8;  // 16-byte chunks per key row
-  static_assert(!BOUND || (HT == 4 && !WBF), "the bound-emitting variant is built for 64 heads, fp32 weights");
+  static_assert(!BOUND || (HT == 4 && KD == 128), "the bound-emitting form is built for 64 heads of 128 dims");
   static_assert(BOUND || !COUNT, "counts of lower ends need the bounds");
   static_assert(!F8 || BOUND, "FP8 keys are read by the bound-emitting variant");
   // per-dot interval half-widths (step_halfwidth_scale: the step-weighted magnitude sum and the step exponents, on
   // the MFMA) instead of the per-head bound_c 2^-23 ||q_h|| max ||k||: under half as wide on typical rows, so
   // under half the near ties and their exact recomputation, for three more MFMAs per 16-key tile (D = 64).  Built
   // where the registers allow it (16 heads).
-  constexpr bool PDD = !BOUND && HT == 1;
+  constexpr bool PDD = HT == 1;
   constexpr int kSteps = KD / 8;  // accumulation steps of a dot
-  // F8: k points at e4m3 codes (KD bytes per row) with row scales ksc
-  const uint8_t *__restrict__ k8 = reinterpret_cast<const uint8_t *>(k);
   __shared__ std::conditional_t<BOUND, ScoresLdsBound<KD, COUNT>, ScoresLds<KD, HT>> L;
   // the wave index is uniform per wave; readfirstlane lets the compiler keep the query row, the causal limit
   // and the tile loop in scalar registers
@@ -398,6 +650,11 @@ indexer_scores_kernel(
       return;
     }
   }
+  if constexpr (BOUND) {  // a body of its own; the rest is the exact kernel
+    bounded_scores<WBF, COUNT, F8>(L, q, k, w, qn, kn, scores, S, T, kbs, causal, start_pos, ratio, bound_c, bounds, kmax,
+                                   row_counts, row_state, ksc, kblk, qgrp);
+    return;
+  } else {
 
   // Every prologue load is issued before the first wait (loads complete in order, so each later wait is a
   // partial one): the key statistics and this wave's query statistics and head weights, then the key
@@ -428,22 +685,13 @@ indexer_scores_kernel(
   const int32_t qs_v = (qsp + qrow0)[hlu];
   const float w_v = WBF ? bf16_to_f32((static_cast<const uint16_t *>(w) + qrow0)[hlu])
                         : (static_cast<const float *>(w) + qrow0)[hlu];
-  constexpr int kKL = kKR * kC / kThreads;  // 16-byte key chunks per thread (F8: kKL / 2 loads of 16 codes)
-  constexpr int kKV = F8 ? kKL / 2 : kKL;
-  uint4 kv[kKV];
-  float ksv[F8 ? kKV : 1];
+  constexpr int kKL = kKR * kC / kThreads;  // 16-byte key chunks per thread
+  uint4 kv[kKL];
 #pragma unroll
-  for (int it = 0; it < kKV; ++it) {
+  for (int it = 0; it < kKL; ++it) {
     const int lin = it * kThreads + tid;
-    if constexpr (F8) {
-      const int kr = lin / (kC / 2), ch2 = lin % (kC / 2);
-      const int64_t row = krow0 + (kr < nk ? kr : nk - 1);
-      kv[it] = *reinterpret_cast<const uint4 *>(k8 + row * KD + ch2 * 16);
-      ksv[it] = ksc[row];
-    } else {
-      const int kr = lin / kC, ch = lin % kC;
-      kv[it] = *reinterpret_cast<const uint4 *>(k + krow0 * KD + static_cast<uint32_t>((kr < nk ? kr : nk - 1) * KD + ch * 8));
-    }
+    const int kr = lin / kC, ch = lin % kC;
+    kv[it] = *reinterpret_cast<const uint4 *>(k + krow0 * KD + static_cast<uint32_t>((kr < nk ? kr : nk - 1) * KD + ch * 8));
   }
   // Every wave's key-block loads are queued ahead of every q load: the memory pipeline serves a CU's loads in
   // issue order, and the waves that issued last would otherwise wait behind the others' q rows (8 x 16 KiB)
@@ -464,7 +712,7 @@ indexer_scores_kernel(
     {
       // (the exact kernel may read its q rows from two buffers, QSplit: the rotated dims from qsplit_rot)
       const uint16_t *qsrc =
-          (!BOUND && qsplit_rot != nullptr && 32 * kk >= qsplit_lo && 32 * kk < qsplit_hi) ? qsplit_rot : q;
+          (qsplit_rot != nullptr && 32 * kk >= qsplit_lo && 32 * kk < qsplit_hi) ? qsplit_rot : q;
       qa[m][kk] = *reinterpret_cast<const uint4 *>(qsrc + qrow0 * KD + static_cast<uint32_t>((16 * m + l16) * KD + 32 * kk + 8 * g));
     }
   auto abs8 = [](uint4 v) {  // |x| of 8 packed bf16
@@ -482,32 +730,9 @@ indexer_scores_kernel(
   // per-head data formed once per head (lane h), not by each of the 16 lanes that use it.  PDD (the exact kernel
   // at 16 heads): per-dot half-widths from the MFMA sum of the magnitudes, dl then holds their additive part
   L.dl[wave][hl] = PDD ? step_halfwidth_add(qn_v, knm, bound_r) : dot_halfwidth(qn_v, knm, bound_c);
-  if constexpr (BOUND) L.wup[wave][hl] = bf16_abs_round_up(w_v);
   L.w[wave][hl] = w_v;
   // the workgroup's whole key block into LDS
-  if constexpr (F8) {
-    // one conversion form for the whole wave: the one-instruction form when every scale it holds allows it
-    bool p2 = true;
-#pragma unroll
-    for (int it = 0; it < kKV; ++it) p2 = p2 & fp8_scale_pow2(ksv[it]);  // no short-circuit: no branches
-    p2 = __builtin_amdgcn_ballot_w64(!p2) == 0ull;
-    auto stage = [&](auto POW2) {
-#pragma unroll
-      for (int it = 0; it < kKV; ++it) {
-        const int lin = it * kThreads + tid;
-        const int kr = lin / (kC / 2), ch = 2 * (lin % (kC / 2));
-        const uint32_t msk = kr < nk ? 0xFFFFFFFFu : 0u;
-        const uint4 lo = fp8_dequant8<decltype(POW2)::value>(make_uint2(kv[it].x, kv[it].y), ksv[it]);
-        const uint4 hi = fp8_dequant8<decltype(POW2)::value>(make_uint2(kv[it].z, kv[it].w), ksv[it]);
-        L.k[kr * kC + (ch ^ (kr & (kC - 1)))] = make_uint4(lo.x & msk, lo.y & msk, lo.z & msk, lo.w & msk);
-        L.k[kr * kC + ((ch + 1) ^ (kr & (kC - 1)))] = make_uint4(hi.x & msk, hi.y & msk, hi.z & msk, hi.w & msk);
-      }
-    };
-    if (p2)
-      stage(std::true_type{});
-    else
-      stage(std::false_type{});
-  } else {
+  {
     // Rows past T hold copies of the last key, loaded from the clamped row: finite operands whose columns are
     // neither stored nor listed.  The 32- and 64-head kernels still zero them: with the loaded values used only by
     // the LDS stores, the compiler sinks their loads below the q loads (and the load-ordering barrier above),
@@ -522,19 +747,10 @@ indexer_scores_kernel(
       if constexpr (PDD) L.kstep[kr][ch] = static_cast<uint16_t>(step_exponent_pow2(kv[it]));
     }
   }
-  if constexpr (COUNT) {  // this wave's lower-end counts start at zero
-#pragma unroll
-    for (int i = 0; i < 4; ++i) reinterpret_cast<uint4 *>(L.cnt[wave])[lane + 64 * i] = make_uint4(0, 0, 0, 0);
-  }
   // the only barrier (from here on every wave runs independently): LDS writes done, no wait for the q loads
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  // BOUND: the block's key-norm maximum for the exact recomputation of candidate scores, which must use
-  // the same interval width (every query group writes the same value)
-  if constexpr (BOUND) {
-    if (tid == 0) kmax[b * gridDim.x + kblk] = knm;
-  }
   if (!s_ok) return;
   float wv[HT][4], dl[HT][4];
 #pragma unroll
@@ -552,42 +768,9 @@ indexer_scores_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) any_inf = any_inf || dl[m][r] == __builtin_inff();
   const bool forced = __builtin_amdgcn_ballot_w64(any_inf) != 0ull;
-  // BOUND: the tile MFMAs start from -delta instead of 0, so that they return the lower interval end A - delta
-  // without a subtraction, and the upper end is fl((A - delta) + 2 delta).  The accumulation model above applies
-  // to any initial value: the running values now carry -delta, which adds at most 16 (2^-31 + 2^-24) delta
-  // (< 2^-19 delta) to its loss; the lower end needs no fp32 rounding of its own, and the upper end's single
-  // rounding loses at most 2^-24 (|A - delta| + 2 delta), as forming A + delta did.  The constant 13 still
-  // covers the sum (12.07 + 0.5 + 2^-19 + the constant's 3 ulps).
-  // (each -delta passes through an empty asm, so that the compiler cannot rewrite the upper end's fma in terms of
-  // +delta and keep both sets of 16 registers live)
-  f32x4_t negd[HT];
-#pragma unroll
-  for (int m = 0; m < HT; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float x = -dl[m][r];
-      asm("" : "+v"(x));
-      negd[m][r] = x;
-    }
-
-  // BOUND: A-fragments holding bf16 upper bounds of |w| for the two 32-head halves.  With the relu'd
-  // interval ends of a tile as B-fragments (lane (l16, g) holds heads 4g + 0..3 and 16 + 4g + 0..3 of
-  // each half, exactly the k-slots 8g .. 8g + 7 of a 16x16x32 B operand), one MFMA per half sums
-  // w_up * r over the 32 heads for every key, in every output row.
-  uint4 wa[2] = {};
-  if constexpr (BOUND) {
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      // heads 16 m + 4 g + (0, 1) and (2, 3) of m = 2 hh and 2 hh + 1, as packed pairs
-      const uint32_t *up = reinterpret_cast<const uint32_t *>(L.wup[wave]);
-      const int h0 = 16 * (2 * hh) + 4 * g, h1 = h0 + 16;
-      wa[hh] = make_uint4(up[h0 / 2], up[h0 / 2 + 1], up[h1 / 2], up[h1 / 2 + 1]);
-    }
-  }
   const int64_t limit = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
   const int limit32 = static_cast<int>(limit < INT32_MAX ? limit : INT32_MAX);  // keys are below T < 2^31
   float *orow = scores + (b * S + s) * T;
-  float *urow = BOUND ? bounds + (b * S + s) * T : nullptr;
   uint32_t n_exact = 0, n_unres = 0;
   int nent = 0;
   // tiles of 16 keys; tiles at or past the causal limit are masked without MFMA work
@@ -644,25 +827,10 @@ indexer_scores_kernel(
       }
     }
   };
-  // the same in two halves (BOUND, from -delta): the B fragments of a tile are read one tile ahead of its MFMAs
-  auto tile_b = [&](int t, uint4(&bv)[KD / 32]) {
-    const int key_l = 16 * t + l16;
-#pragma unroll
-    for (int kk = 0; kk < KD / 32; ++kk) bv[kk] = L.k[key_l * kC + ((4 * kk + g) ^ (key_l & (kC - 1)))];
-  };
-  auto tile_mfma_b = [&](const uint4(&bv)[KD / 32], f32x4_t(&acc)[HT]) {
-#pragma unroll
-    for (int m = 0; m < HT; ++m) acc[m] = negd[m];  // lower ends A - delta
-#pragma unroll
-    for (int kk = 0; kk < KD / 32; ++kk)
-#pragma unroll
-      for (int m = 0; m < HT; ++m) acc[m] = mfma16(qa[m][kk], bv[kk], acc[m]);
-  };
 
   const float dsc = PDD ? step_halfwidth_scale(bound_r) : 0.f;
   // the exact kernel's interval test (the tile epilogue's, below) on the 16 keys of a resolution round: pl, ph and the
-  // ballot of the lanes holding a near-tie dot.  (The tile epilogue keeps its own copy: sharing this lambda with
-  // the bound kernels' epilogue made the compiler spill registers in their tile loop.)
+  // ballot of the lanes holding a near-tie dot.
   auto interval_ends = [&](const f32x4_t(&acc)[HT], const f32x4_t(&accs)[HT], uint32_t(&pl)[2 * HT],
                            uint32_t(&ph)[2 * HT]) {
     uint64_t anyr = 0;
@@ -709,16 +877,10 @@ indexer_scores_kernel(
 #pragma unroll
       for (int rp = 0; rp < 2; ++rp) {
         const float A0 = acc[m][2 * rp], A1 = acc[m][2 * rp + 1];
-        if constexpr (BOUND) {  // A0, A1 are already the lower ends A - delta
-          const float n0 = negd[m][2 * rp], n1 = negd[m][2 * rp + 1];
-          pl[2 * m + rp] = cvt_relu_pk(A0, A1);
-          ph[2 * m + rp] = cvt_relu_pk(__builtin_fmaf(-2.f, n0, A0), __builtin_fmaf(-2.f, n1, A1));
-        } else {
-          const float d0 = PDD ? __builtin_fmaf(accs[m][2 * rp], dsc, dl[m][2 * rp]) : dl[m][2 * rp];
-          const float d1 = PDD ? __builtin_fmaf(accs[m][2 * rp + 1], dsc, dl[m][2 * rp + 1]) : dl[m][2 * rp + 1];
-          pl[2 * m + rp] = cvt_relu_pk(A0 - d0, A1 - d1);
-          ph[2 * m + rp] = cvt_relu_pk(A0 + d0, A1 + d1);
-        }
+        const float d0 = PDD ? __builtin_fmaf(accs[m][2 * rp], dsc, dl[m][2 * rp]) : dl[m][2 * rp];
+        const float d1 = PDD ? __builtin_fmaf(accs[m][2 * rp + 1], dsc, dl[m][2 * rp + 1]) : dl[m][2 * rp + 1];
+        pl[2 * m + rp] = cvt_relu_pk(A0 - d0, A1 - d1);
+        ph[2 * m + rp] = cvt_relu_pk(A0 + d0, A1 + d1);
         anyr |= __builtin_amdgcn_ballot_w64(pl[2 * m + rp] != ph[2 * m + rp]);
       }
     if (fcd) {  // wave-uniform and rare: A may not even be finite; the exact values replace everything
@@ -743,17 +905,6 @@ indexer_scores_kernel(
           G = __builtin_fmaf(rv, wv[m][r], G);
         }
     }
-    if constexpr (BOUND) {
-      // the next tile's 16 MFMAs (issued before this epilogue, in the same basic block) spread over the interval
-      // test and the head sum, one per 6 VALU instructions: the wave keeps issuing VALU work while the matrix
-      // core runs, instead of stalling on 16 back-to-back MFMAs
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
-      }
-    }
     float tot = 0.f, outv = 0.f;
     if constexpr (decltype(PAIR)::value) {
       gsum = G;
@@ -762,71 +913,14 @@ indexer_scores_kernel(
       outv = WBF ? round_score_bf16(tot) : tot;
       if (g == 0 && kvalid) orow[key] = (full || key < limit32) ? outv : -INFINITY;
     }
-    // keys past T are not stored and, in the exact kernel, keys past the causal limit are -inf: neither is deferred
-    // (the bound kernel stores bound 0 past the limit, below)
-    if constexpr (!full) anyr &= __builtin_amdgcn_ballot_w64(BOUND ? kvalid : (kvalid && key < limit32));
-    const uint32_t km = key_mask(anyr);
-    if constexpr (BOUND) {
-      // |exact score - tot| <= sum_h |w_h| (ph_h - pl_h) + (rounding of the canonical sum: 38 roundings of
-      // at most 2^-24 of sum_h |w_h| ph_h, < 2^-18 of it) <= dph - dpl + 2^-16 (dph + dpl), dph / dpl the
-      // MFMA sums of w_up * ph / pl (64 nonnegative exact products in 8 accumulation steps: relative error
-      // below (8 + 8) 2^-24 < 2^-19 by the step model of dot_halfwidth, the 2^-100 term covering subnormal
-      // operands).  The 2^-21 |tot| term lets tot -/+ bound be rounded to nearest and stay a bound.  Keys
-      // without a near-tie dot have bound 0 (tot is exact).
-      f32x4_t dph = f32x4_t{0.f, 0.f, 0.f, 0.f}, dpl = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        dph = mfma16(wa[hh], make_uint4(ph[4 * hh], ph[4 * hh + 1], ph[4 * hh + 2], ph[4 * hh + 3]), dph);
-        dpl = mfma16(wa[hh], make_uint4(pl[4 * hh], pl[4 * hh + 1], pl[4 * hh + 2], pl[4 * hh + 3]), dpl);
-      }
-      float u = (dph[0] - dpl[0]) + 0x1p-16f * (dph[0] + dpl[0]) + 0x1p-21f * fabsf(tot) + 0x1p-100f;
-      if (fcd) u = __builtin_inff();  // score 0 with an infinite bound: always recomputed
-      const bool live_key = kvalid && key < limit32;
-      const float us = (live_key && ((km >> l16) & 1u)) ? u : 0.f;
-      if (g == 0 && kvalid) urow[key] = us;
-      // the row's threshold histogram: first 11-bit digit of the lower end's key, counted for the valid columns
-      // (the same arithmetic as the stored score and bound give)
-      if (COUNT && g == 0 && live_key) {
-        const uint32_t kk = score_key(us > 0.f ? outv - us : outv);
-        if (kk != 0u) atomicAdd(&L.cnt[wave][kk >> 22], 1u << ((kk >> 17) & 16u));
-      }
-    }
-    return km;
+    // keys past T are not stored and keys past the causal limit are -inf: neither is deferred
+    if constexpr (!full) anyr &= __builtin_amdgcn_ballot_w64(kvalid && key < limit32);
+    return key_mask(anyr);
   };
-
   // software pipeline: the MFMAs of the next tile are in flight during the current tile's epilogue.
   f32x4_t acc[HT], nxt[HT];
-  if constexpr (BOUND) {
-    // no deferred keys: two tiles per iteration, alternating the accumulator sets (no copy between them) and
-    // the B-fragment sets (read one tile ahead).  The MFMAs and reads past the last live tile repeat that tile
-    // (results unused), so that no branch separates them from the epilogue they are interleaved with.
-    auto run = [&](auto FC) {
-      uint4 ba[KD / 32], bb[KD / 32];
-      const int last = nlive - 1;
-      tile_b(0, ba);
-      tile_mfma_b(ba, acc);
-      tile_b(1 < nlive ? 1 : last, bb);
-      for (int t = 0; t < nlive; t += 2) {
-        uint32_t pl[2 * HT], ph[2 * HT];
-        tile_mfma_b(bb, nxt);
-        tile_b(t + 2 < nlive ? t + 2 : last, ba);
-        float gs;
-        (void)tile_epilogue(FC, std::false_type{}, std::false_type{}, t, acc, acc, pl, ph, gs);
-        if (t + 1 >= nlive) break;
-        tile_mfma_b(ba, acc);
-        tile_b(t + 3 < nlive ? t + 3 : last, bb);
-        (void)tile_epilogue(FC, std::false_type{}, std::false_type{}, t + 1, nxt, nxt, pl, ph, gs);
-      }
-    };
-    if (nlive > 0) {
-      if (forced)
-        run(std::true_type{});
-      else
-        run(std::false_type{});
-    }
-  }
-  if constexpr (!BOUND) {
-    // the exact kernel: the tile loop only lists the keys holding a near-tie dot (their block rows, in LDS); the
+  {
+    // the tile loop only lists the keys holding a near-tie dot (their block rows, in LDS); the
     // listed keys are resolved after it.  Nothing of the recomputation is live in the loop, so the loop keeps its
     // pipeline in few registers.  The next tile's MFMAs past the last live tile repeat that tile (results unused).
     // Two tiles per iteration alternate the accumulator sets (no copies between them); the loop is built twice,
@@ -985,41 +1079,20 @@ indexer_scores_kernel(
       }
     }
   }
-  // masked tiles (at or past the causal limit); the exact kernel stores with every lane (the bound kernel keeps
-  // its tile form, which its register allocation was tuned with)
-  if constexpr (BOUND) {
-    for (int t = nlive; t < ntiles; ++t) {
-      const int key_l = 16 * t + l16;
-      if (g == 0 && key_l < nk) orow[kb0 + key_l] = -INFINITY;
-    }
-  } else {
-    for (int key_l = 16 * nlive + lane; key_l < nk; key_l += 64) orow[static_cast<uint32_t>(kb0 + key_l)] = -INFINITY;
-  }
-  if constexpr (COUNT) {
-    // the wave's counts into its row's histogram (only the nonzero buckets: a block of 256 keys fills a few
-    // dozen of the 2048)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint32_t *hrow = row_counts + (b * S + s) * 2048;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int wd = lane + 64 * i;
-      const uint32_t v = L.cnt[wave][wd];
-      if (v & 0xFFFFu) atomicAdd(&hrow[2 * wd], v & 0xFFFFu);
-      if (v >> 16) atomicAdd(&hrow[2 * wd + 1], v >> 16);
-    }
-  }
+  // masked tiles (at or past the causal limit)
+  for (int key_l = 16 * nlive + lane; key_l < nk; key_l += 64) orow[static_cast<uint32_t>(kb0 + key_l)] = -INFINITY;
   if (stats != nullptr) {
     if (lane == 0 && n_exact) atomicAdd(&stats[0], n_exact);
     if (n_unres) atomicAdd(&stats[1], n_unres);
   }
+  }  // !BOUND
 }
 
 template <int HT, int KD>
 int launch_scores_ht(const uint16_t *q, const uint16_t *k, const void *w, int w_bf16, const float *qn,
                      const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B, int64_t S,
                      int64_t T, int64_t kbs, int causal, int64_t start_pos, int ratio, float bound_c, uint32_t *stats,
-                     float *bounds, float *kmax, uint32_t *row_counts, const float *ksc, hipStream_t stream,
+                     float *bounds, float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc, hipStream_t stream,
                      const QSplit *qsplit) {
   const QSplit qs = qsplit != nullptr ? *qsplit : QSplit{nullptr, 0, 0};
   dim3 grid(static_cast<unsigned>(ceil_div(T, kKR)), static_cast<unsigned>(ceil_div(S, kQW)),
@@ -1046,43 +1119,45 @@ int launch_scores_ht(const uint16_t *q, const uint16_t *k, const void *w, int w_
   if (bounds != nullptr && ksc != nullptr) {
     if constexpr (HT == 4 && KD == 128) {
       if (w_bf16) return fail(KS_ERR_INVALID, "indexer scores: score bounds need fp32 weights");
-      if (kmax == nullptr) return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax buffer");
+      if (kmax == nullptr || row_state == nullptr)
+        return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax and row state buffers");
       if (row_counts != nullptr) {
         hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, true, true>), grid, dim3(kThreads), 0, stream, q,
                            k, w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio,
-                           bound_c, stats, xcd_pk, bounds, kmax, row_counts, ksc, bound_r, qs.rot, qs.lo, qs.hi);
+                           bound_c, stats, xcd_pk, bounds, kmax, row_counts, row_state, ksc, bound_r, qs.rot, qs.lo, qs.hi);
       } else {
         hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, false, true>), grid, dim3(kThreads), 0, stream,
                            q, k, w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio,
-                           bound_c, stats, xcd_pk, bounds, kmax, nullptr, ksc, bound_r, qs.rot, qs.lo, qs.hi);
+                           bound_c, stats, xcd_pk, bounds, kmax, nullptr, row_state, ksc, bound_r, qs.rot, qs.lo, qs.hi);
       }
     } else {
       return fail(KS_ERR_INVALID, "indexer scores: FP8 keys need H = 64 and D = 128");
     }
   } else if (bounds != nullptr) {
-    if constexpr (HT == 4) {
+    if constexpr (HT == 4 && KD == 128) {
       if (w_bf16) return fail(KS_ERR_INVALID, "indexer scores: score bounds need fp32 weights");
-      if (kmax == nullptr) return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax buffer");
+      if (kmax == nullptr || row_state == nullptr)
+        return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax and row state buffers");
       if (row_counts != nullptr) {
         hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, true>), grid, dim3(kThreads), 0, stream, q, k, w,
                            qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c,
-                           stats, xcd_pk, bounds, kmax, row_counts, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                           stats, xcd_pk, bounds, kmax, row_counts, row_state, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
       } else {
         hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, false>), grid, dim3(kThreads), 0, stream, q, k,
                            w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c,
-                           stats, xcd_pk, bounds, kmax, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                           stats, xcd_pk, bounds, kmax, nullptr, row_state, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
       }
     } else {
-      return fail(KS_ERR_INVALID, "indexer scores: score bounds need H = 64");
+      return fail(KS_ERR_INVALID, "indexer scores: score bounds need H = 64 and D = 128");
     }
   } else if (w_bf16) {
     hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, true, false>), grid, dim3(kThreads), 0, stream, q, k, w, qn, qsp,
                        kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c, stats, xcd_pk,
-                       nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                       nullptr, nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
   } else {
     hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, false>), grid, dim3(kThreads), 0, stream, q, k, w, qn,
                        qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c, stats,
-                       xcd_pk, nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                       xcd_pk, nullptr, nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
   }
   KS_CHECK_LAUNCH("indexer_scores_kernel");
   return KS_OK;
@@ -1092,18 +1167,18 @@ template <int KD>
 int launch_scores_d(const uint16_t *q, const uint16_t *k, const void *w, int w_bf16, const float *qn,
                     const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B, int64_t S,
                     int64_t H, int64_t T, int64_t kbs, int causal, int64_t start_pos, int ratio, float bound_c,
-                    uint32_t *stats, float *bounds, float *kmax, uint32_t *row_counts, const float *ksc,
+                    uint32_t *stats, float *bounds, float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc,
                     hipStream_t stream, const QSplit *qsplit) {
   switch (H) {
     case 16:
       return launch_scores_ht<1, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
     case 32:
       return launch_scores_ht<2, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
     case 64:
       return launch_scores_ht<4, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
     default:
       return fail(KS_ERR_INVALID, "indexer scores: H=%lld, supported: 16, 32, 64", (long long)H);
   }
@@ -1119,13 +1194,14 @@ int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, i
                           const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B,
                           int64_t S, int64_t H, int64_t D, int64_t T, int64_t kbs, int causal, int64_t start_pos,
                           int ratio, float bound_c, uint32_t *stats, hipStream_t stream, float *bounds,
-                          float *kmax, uint32_t *row_counts, const float *ksc, const QSplit *qsplit) {
+                          float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc,
+                          const QSplit *qsplit) {
   if (D == 128)
     return launch_scores_d<128>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, H, T, kbs, causal, start_pos, ratio,
-                                bound_c, stats, bounds, kmax, row_counts, ksc, stream, qsplit);
+                                bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
   if (D == 64)
     return launch_scores_d<64>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, H, T, kbs, causal, start_pos, ratio,
-                               bound_c, stats, bounds, kmax, row_counts, ksc, stream, qsplit);
+                               bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
   return fail(KS_ERR_INVALID, "indexer scores: D=%lld, supported: 64, 128", (long long)D);
 }
 
@@ -1206,5 +1282,6 @@ extern "C" int ks_dbg_indexer_scores_bounded(const uint16_t *q, const uint16_t *
   return ks::launch_indexer_scores(q, k, w, 0, q_norm, q_span, k_norm, k_span, scores, B, S, 64, 128, T, T,
                                    causal ? 1 : 0, start_pos, 1, ks::kScoreBoundC, nullptr,
                                    static_cast<hipStream_t>(stream), bounds, kmax,
-                                   ks::scores_count_rows(B, S, T) ? ks::topk_bounded_counts(part, B * S, T) : nullptr);
+                                   ks::scores_count_rows(B, S, T) ? ks::topk_bounded_counts(part, B * S, T) : nullptr,
+                                   ks::topk_bounded_state(part, B * S, T, ks::scores_count_rows(B, S, T)));
 }

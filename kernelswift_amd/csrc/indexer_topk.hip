@@ -841,8 +841,8 @@ __device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow,
   }
 }
 
-// Workgroup (row, slice): counts of the first 11-bit digit (2048 buckets) of the lower ends (score - U; the score
-// itself where U = 0) of slice p's valid columns, stored for the recomputation's threshold.  Workgroup (row, 0)
+// Workgroup (row, slice): counts of the buckets (bound_digit, 2048) of the lower ends score - U of slice p's valid
+// columns, stored for the recomputation's threshold.  Workgroup (row, 0)
 // also clears the row's list length and key maximum (the recomputation appends to the list after this launch).
 template <int KPT>
 __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const float *scores, const float *bounds,
@@ -870,6 +870,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
     sv[j] = src[col < nv ? col : 0];
     uv[j] = ub[col < nv ? col : 0];
   }
+  const uint32_t mrow = rstate[4 * row + 3];
   if (blockIdx.y == 0 && tid == 0) {
     rstate[4 * row] = 0u;
     rstate[4 * row + 2] = 0u;
@@ -879,8 +880,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 #pragma unroll
   for (int j = 0; j < KPT; ++j) {
     if (j * kTopkThreads + tid < nv) {
-      const uint32_t kk = score_key(uv[j] > 0.f ? sv[j] - uv[j] : sv[j]);
-      if (kk != 0) atomicAdd(&hist[kk >> 21], 1u);
+      atomicAdd(&hist[bound_digit(sv[j] - uv[j], mrow)], 1u);
     }
   }
   __syncthreads();
@@ -947,6 +947,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   const int hh = tid & (kRecH - 1);
   const float wv = rc.w[qrow0 + hh], qnv = rc.qn[qrow0 + hh];
   const int32_t qsv = rc.qsp[qrow0 + hh];
+  const uint32_t mrow = rstate[4 * row + 3];
   float sv[KPB], uv[KPB];
 #pragma unroll
   for (int j = 0; j < KPB; ++j) {
@@ -1009,7 +1010,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
           found = true;
         }
       }
-      s_tau = bucket << 21;
+      s_tau = bound_digit_edge(bucket, mrow);
     }
   }
   __syncthreads();
@@ -1361,6 +1362,13 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
 #undef KS_COLL
   KS_CHECK_LAUNCH("topk_collected_kernel");
   return KS_OK;
+}
+
+uint32_t *ks::topk_bounded_state(uint64_t *part, int64_t rows, int64_t T, bool counted) {
+  const int Ti = static_cast<int>(T), np = counted ? 1 : topk_slices(rows, Ti);
+  int W = kTopkThreads;
+  while (W * np < Ti) W <<= 1;
+  return reinterpret_cast<uint32_t *>(part + rows * topk_list_cap(Ti)) + rows * ((Ti + W - 1) / W) * 2048;
 }
 
 uint32_t *ks::topk_bounded_counts(uint64_t *part, int64_t rows, int64_t T) {
