@@ -27,8 +27,7 @@ struct IndexerWs {
   int32_t *k_span;
   float *scores;
   float *bounds;  // per-score bounds of the bounded path
-  float *kmax;    // per key block norm maxima of the bounded path
-  uint64_t *part;  // the bounded selection's lists, bucket counts and list lengths
+  uint64_t *part;  // the bounded selection's lists, bucket counts and states
   int64_t part_cap;
   void *w_scaled;  // the head weights times w_scale (ks_indexer_scaled), in the weights' format
   size_t bytes;
@@ -52,7 +51,6 @@ IndexerWs carve(void *base, int64_t B, int64_t S, int64_t H, int64_t D, int64_t 
   w.k_span = reinterpret_cast<int32_t *>(take(size_t(B * T) * 4));
   w.scores = reinterpret_cast<float *>(take(size_t(B * S * T) * 4));
   w.bounds = reinterpret_cast<float *>(take(size_t(B * S * T) * 4));
-  w.kmax = reinterpret_cast<float *>(take(size_t(B * ((T + ks::kScoreKeyBlock - 1) / ks::kScoreKeyBlock)) * 4));
   // the bounded selection's lists and counts (only shapes that can take the bounded path)
   w.part_cap = (H == 64 && D == 128) ? ks::topk_bounded_part_capacity(B * S, T) : 0;
   w.part = reinterpret_cast<uint64_t *>(take(size_t(w.part_cap) * 8));
@@ -92,12 +90,6 @@ bool takes_bounded(int64_t k_top, int32_t w_bf16, int64_t H, int64_t D, int64_t 
   return H == 64 && D == 128 && !w_bf16 && T <= 32768 && kk <= 2048 && path != 1;
 }
 
-// The bounded path's count region in the workspace, which the row preparation launch clears when the score
-// kernel counts the rows: 16-byte words.
-int64_t count_words16(const IndexerWs &ws, int64_t B, int64_t S, int64_t T) {
-  return ws.part_cap > 0 && ks::scores_count_rows(B, S, T) ? B * S * ks::kTopkCountWords / 4 : 0;
-}
-
 // FP8 keys read directly by the bounded kernels (codes and row scales at batch stride kbs), or none.
 struct Fp8Direct {
   const uint8_t *kc = nullptr;
@@ -106,9 +98,6 @@ struct Fp8Direct {
 };
 
 // Scores of the prepared rows (ws.q_rot / ws.k_rot with their statistics, or the FP8 rows of f8) -> exact top-k.
-// Where the score kernel counts the rows, the bounded path needs the count region cleared by the row preparation
-// launch.
-
 int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w_bf16, int64_t k_top, int32_t causal,
                    int64_t start_pos, int32_t ratio, int64_t offset, void *out, int32_t out_i64, int64_t B, int64_t S,
                    int64_t H, int64_t D, int64_t T, hipStream_t st, float bound_c, uint32_t *stats, int path,
@@ -120,19 +109,17 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
                "%s: the bounded path needs H = 64, D = 128, fp32 weights, T <= 32768 and k <= 2048", fn);
   int rc;
   if (can_bound && path != 1) {
-    const bool counted = ks::scores_count_rows(B, S, T);
     const bool direct = f8.kc != nullptr;
     // FP8 keys: the codes with their row scales (the statistics are indexed like the rows: B == 1 or kbs == T)
     const uint16_t *krows = direct ? reinterpret_cast<const uint16_t *>(f8.kc) : ws.k_rot;
     const int64_t kbs = direct ? f8.kbs : T;
     rc = ks::launch_indexer_scores(ws.q_rot, krows, w, 0, ws.q_norm, ws.q_span, ws.k_norm, ws.k_span, ws.scores, B, S,
                                    H, D, T, kbs, causal ? 1 : 0, start_pos, ratio, bound_c, nullptr, st, ws.bounds,
-                                   ws.kmax, counted ? ks::topk_bounded_counts(ws.part, B * S, T) : nullptr,
-                                   ks::topk_bounded_state(ws.part, B * S, T, counted), f8.ks);
+                                   ks::topk_bounded_state(ws.part, B * S, T), f8.ks);
     if (rc != KS_OK) return rc;
-    ks::TopkRecompute trc{ws.bounds, ws.kmax, ws.q_rot, ws.k_rot, static_cast<const float *>(w), ws.q_norm,
+    ks::TopkRecompute trc{ws.bounds, ws.q_rot, ws.k_rot, static_cast<const float *>(w), ws.q_norm,
                           ws.q_span, ws.k_norm, ws.k_span, kbs, bound_c, stats, path == 3 ? 1 : 0, ws.part,
-                          ws.part_cap, counted ? 1 : 0};
+                          ws.part_cap};
     trc.kc = f8.kc;
     trc.ks = f8.ks;
     return ks::launch_indexer_topk_bounded(ws.scores, T, B, S, T, kk, causal ? 1 : 0, start_pos, ratio, offset, out,
@@ -143,7 +130,7 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
   const ks::QSplit qs{rot_hi > rot_lo ? ws.q_rot : nullptr, rot_lo, rot_hi};
   rc = ks::launch_indexer_scores(q_unrot != nullptr ? q_unrot : ws.q_rot, ws.k_rot, w, w_bf16 ? 1 : 0, ws.q_norm,
                                  ws.q_span, ws.k_norm, ws.k_span, ws.scores, B, S, H, D, T, T, causal ? 1 : 0,
-                                 start_pos, ratio, bound_c, stats, st, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                 start_pos, ratio, bound_c, stats, st, nullptr, nullptr, nullptr,
                                  q_unrot != nullptr ? &qs : nullptr);
   if (rc != KS_OK) return rc;
   // bf16 weights: the exact scores are rounded to bf16, so the top-k may take them as bf16 values
@@ -188,8 +175,7 @@ int indexer_impl(const uint16_t *q, const uint16_t *k, const void *w, int32_t w_
   const bool scaled = w_scale != 1.0f;
   const ks::WeightScale wsc{w, ws.w_scaled, w_scale, w_bf16 ? 1 : 0};
   rc = ks::launch_rope_rows(qjob, kjob, freqs, static_cast<int>(D), static_cast<int>(rope_start), st,
-                            bounded ? ks::topk_bounded_counts(ws.part, B * S, T) : nullptr,
-                            bounded ? count_words16(ws, B, S, T) : 0, scaled ? &wsc : nullptr);
+                            scaled ? &wsc : nullptr);
   if (rc != KS_OK) return rc;
   return indexer_select("ks_indexer", ws, scaled ? ws.w_scaled : w, w_bf16, k_top, causal, start_pos, ratio, offset,
                         out, out_i64, B, S, H, D, T, st, bound_c, stats, path, Fp8Direct{}, split ? q : nullptr,
@@ -221,9 +207,7 @@ int indexer_fp8_impl(const uint8_t *q, const float *q_scale, const uint8_t *k, c
   // q rows (scale per row) and k rows of every batch (stride k_batch_stride, scale per row, same stride)
   const ks::Fp8RowJob qjob{q, q_scale, ws.q_rot, ws.q_norm, ws.q_span, B * S * H, B * S * H, B * S * H};
   const ks::Fp8RowJob kjob{k, k_scale, direct ? nullptr : ws.k_rot, ws.k_norm, ws.k_span, B * T, T, k_batch_stride};
-  rc = ks::launch_fp8_rows(qjob, kjob, static_cast<int>(D), st,
-                           bounded ? ks::topk_bounded_counts(ws.part, B * S, T) : nullptr,
-                           bounded ? count_words16(ws, B, S, T) : 0);
+  rc = ks::launch_fp8_rows(qjob, kjob, static_cast<int>(D), st);
   if (rc != KS_OK) return rc;
   Fp8Direct f8;
   if (direct) {

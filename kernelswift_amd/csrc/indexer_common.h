@@ -274,9 +274,7 @@ struct RowJob {
 };
 
 // Both jobs in one launch (job1.rows may be 0); rows of D in {64, 128} for statistics, any multiple of 8
-// otherwise.  Rotated dims [rope_start, rope_start + job.rope_dim), freqs = (cos, sin) per position.  The
-// launch also clears zero16 16-byte words at zero (the bounded selection's counts, which the score kernel
-// that follows accumulates into).
+// otherwise.  Rotated dims [rope_start, rope_start + job.rope_dim), freqs = (cos, sin) per position.
 // Head weights scaled on the way (the fused indexer's w_scale): out[r] = w[r] * scale for the first job's rows r
 // (one weight per q row), rounded as torch rounds a tensor times a Python float: fp32(w * fp32(scale)), then
 // bf16 (nearest even) for bf16 weights.
@@ -288,7 +286,7 @@ struct WeightScale {
 };
 
 int launch_rope_rows(const RowJob &job0, const RowJob &job1, const float *freqs, int D, int rope_start,
-                     hipStream_t stream, void *zero = nullptr, int64_t zero16 = 0, const WeightScale *wscale = nullptr);
+                     hipStream_t stream, const WeightScale *wscale = nullptr);
 
 // One set of e4m3 rows for the dequantisation / row-statistics launch: row r is source row
 // (r / rows_per_batch) * src_batch_rows + r % rows_per_batch of src (D code bytes) with fp32 scale
@@ -302,25 +300,14 @@ struct Fp8RowJob {
   int64_t rows, rows_per_batch, src_batch_rows;
 };
 
-// Both jobs in one launch (job1.rows may be 0); D in {64, 128}.  Clears zero16 16-byte words at zero, as
-// launch_rope_rows does.
-int launch_fp8_rows(const Fp8RowJob &job0, const Fp8RowJob &job1, int D, hipStream_t stream, void *zero = nullptr,
-                    int64_t zero16 = 0);
+// Both jobs in one launch (job1.rows may be 0); D in {64, 128}.
+int launch_fp8_rows(const Fp8RowJob &job0, const Fp8RowJob &job1, int D, hipStream_t stream);
 
 // Exact scores (bounds == nullptr), or, with bounds (H = 64, D = 128), a score and a bound U: the exact score lies in
-// [score - U, score + U], both ends also after rounding to nearest.  kmax [B][ceil(T / kScoreKeyBlock)] then receives
-// each key block's key-norm maximum (the interval half-width of a dot is bound_c 2^-23 ||q_h|| kmax), for the exact
-// recomputation, row_state [B S][4] the scale of each row's threshold histogram (word 3), and row_counts [B S][2048]
-// (zero on entry; may be null) is incremented by each row's counts of bound_digit(lower end) over its valid columns.  With
-// ksc (bound mode, 64 heads, D = 128), k holds e4m3 codes with those row scales (FP8 keys), read directly; kn /
-// ksp are the statistics of the dequantised rows.
+// [score - U, score + U], both ends also after rounding to nearest; row_state [B S][2] (word 1) then receives the scale of
+// each row's threshold histogram (bound_digit).  With ksc (bound mode), k holds e4m3 codes with those row scales (FP8
+// keys), read directly; kn / ksp are the statistics of the dequantised rows.
 constexpr int kScoreKeyBlock = 256;
-// Whether the fused entry counts the rows in the score kernel: its grid of (key block, 8 queries) workgroups
-// fits the 256 CUs in one round.  The counts' LDS leaves no room for a second workgroup per CU, which a grid
-// of several rounds needs to start its next workgroups in the tails of the running ones; such grids are counted
-// by the selection's own histogram launch instead.
-constexpr int64_t kScoreCountGrid = 256;
-bool scores_count_rows(int64_t B, int64_t S, int64_t T);
 // q rows split over two buffers (the exact path when the row preparation wrote only the rotated dims): dims
 // [lo, hi) (32-aligned) from rot, the others from the q argument; rot == nullptr: all of q from the argument.
 struct QSplit {
@@ -332,18 +319,16 @@ int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, i
                           const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B,
                           int64_t S, int64_t H, int64_t D, int64_t T, int64_t kbs, int causal, int64_t start_pos,
                           int ratio, float bound_c, uint32_t *stats, hipStream_t stream, float *bounds = nullptr,
-                          float *kmax = nullptr, uint32_t *row_counts = nullptr, uint32_t *row_state = nullptr,
-                          const float *ksc = nullptr, const QSplit *qsplit = nullptr);
+                          uint32_t *row_state = nullptr, const float *ksc = nullptr, const QSplit *qsplit = nullptr);
 
 // Sorted exact top-k of rows of bounded scores (the bound-emitting score kernel's output): a threshold from the
 // lower ends, exact recomputation of the scores that may reach the top k (interval test with the score kernel's
-// half-widths, exact double-precision dots for the near ties, canonical head sum; written back with bound 0),
+// half-widths, exact double-precision dots for the near ties, canonical head sum),
 // then a sort of the exact scores at or above the threshold.  q / k: the rotated rows and their statistics
 // (64 heads, D = 128), w fp32 [B, S, 64]; with kc / ks set, the keys are e4m3 codes and row scales (the statistics
 // those of the dequantised rows), read directly and dequantised in registers.
 struct TopkRecompute {
-  float *bounds;  // recomputed scores get bound 0
-  const float *kmax;
+  float *bounds;  // overwritten where a row's list outgrows LDS
   const uint16_t *q;
   const uint16_t *k;
   const float *w;
@@ -355,26 +340,17 @@ struct TopkRecompute {
   float bound_c;
   uint32_t *stats;  // optional: [0] += exact dot recomputations, [1] += dots outside the exact range
   int stats_ext;    // with stats: [2] += recomputed scores
-  // workspace of topk_bounded_part_capacity(rows, T) 64-bit slots: the rows' lists of exact scores at or above
-  // the threshold, the bucket counts of their column slices, the list lengths
+  // workspace of topk_bounded_part_capacity(rows, T) 64-bit slots
   uint64_t *part;
   int64_t part_cap;  // 64-bit slots
-  // nonzero: the score kernel has already counted the rows (one slice per row, at topk_bounded_counts) and the
-  // row states there are clear, so the selection starts with the threshold
-  int counted;
   // FP8 keys (both set, or neither): codes [rows][128] and row scales, kbs rows per batch
   const uint8_t *kc = nullptr;
   const float *ks = nullptr;
 };
 // Slots the bounded selection needs for `rows` rows of T <= 32768 columns (0 outside that range).
 int64_t topk_bounded_part_capacity(int64_t rows, int64_t T);
-// The counted form's region in part: the rows' bucket counts ([rows][2048] 32-bit) followed by their states
-// ([rows][4] 32-bit), kTopkCountWords 32-bit words per row in all, to be cleared before the score kernel.
-constexpr int64_t kTopkCountWords = 2048 + 4;
-uint32_t *topk_bounded_counts(uint64_t *part, int64_t rows, int64_t T);
-// The row states in part ([rows][4]: list length, tau, largest key bound, histogram scale), for the counted form or
-// the one whose histogram launch counts column slices.  The score kernel writes the scale.
-uint32_t *topk_bounded_state(uint64_t *part, int64_t rows, int64_t T, bool counted);
+// The row states in part ([rows][2]: tau, histogram scale); the score kernel writes the scale.
+uint32_t *topk_bounded_state(uint64_t *part, int64_t rows, int64_t T);
 // ks_indexer_topk with the caller's guarantee that every score is a bf16 value (bf16_vals = 1), which spares the
 // one-wave-per-row form its check of the keys' low halves.
 int indexer_topk_impl(const float *scores, int64_t ld, int64_t B, int64_t S, int64_t T, int64_t k, int32_t causal,

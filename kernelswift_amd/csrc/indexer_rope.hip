@@ -53,13 +53,11 @@ RowJobK kernel_job(const RowJob &j) {
 // the statistics forms (CPR = chunks per row, 8 or 16: lane j of the row's CPR / 2 lanes holds chunks j and
 // j + CPR / 2), so that the row and position arithmetic, the statistics' final steps and the weight scaling are
 // shared by twice the bytes.  Blocks [0, blocks0) take job 0 and the rest job 1 (a uniform choice, so each field is
-// selected separately from the kernel arguments, never through a pointer to them).  The grid's threads also clear
-// zero16 16-byte words at zero (grid-strided).
+// selected separately from the kernel arguments, never through a pointer to them).
 template <int CPR>
 __global__ __launch_bounds__(256) void rope_rows_kernel(RowJobK j0, RowJobK j1, uint32_t blocks0,
                                                        const float *__restrict__ freqs, int D, FastDiv cpr,
-                                                       int rope_start, uint4 *__restrict__ zero, uint32_t zero16,
-                                                       WeightScale wsc) {
+                                                       int rope_start, WeightScale wsc) {
   constexpr int NC = CPR == 0 ? 1 : 2;  // chunks per thread
   constexpr int LPR = CPR / NC;         // lanes per row (statistics forms)
   const bool second = blockIdx.x >= blocks0;
@@ -140,16 +138,12 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RowJobK j0, RowJobK j1, 
       static_cast<float *>(wsc.out)[row] = static_cast<const float *>(wsc.w)[row] * wsc.scale;
     }
   }
-  // after the row's own stores, so that its loads do not wait behind these
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < zero16; i += gridDim.x * 256u) zero[i] = make_uint4(0, 0, 0, 0);
 }
 
 }  // namespace
 
 int launch_rope_rows(const RowJob &job0, const RowJob &job1, const float *freqs, int D, int rope_start,
-                     hipStream_t stream, void *zero, int64_t zero16, const WeightScale *wscale) {
-  KS_CHECK_ARG(zero16 >= 0 && zero16 < (int64_t(1) << 31) && (zero16 == 0 || aligned(zero, 16)),
-               "rope rows: clear range of %lld words", (long long)zero16);
+                     hipStream_t stream, const WeightScale *wscale) {
   const bool stats = job0.norm != nullptr;
   const int64_t tpr = stats ? D / 16 : D / 8;  // threads per row: two chunks each with statistics, else one
   const int64_t c0 = job0.rows * tpr, c1 = job1.rows * tpr;
@@ -161,7 +155,6 @@ int launch_rope_rows(const RowJob &job0, const RowJob &job1, const float *freqs,
                    job1.H < (int64_t(1) << 31) && job0.S < (int64_t(1) << 31) && job1.S < (int64_t(1) << 31),
                "rope rows: batch, head or position extent out of range");
   const int64_t b0 = ceil_div(c0, 256), b1 = ceil_div(c1, 256);
-  KS_CHECK_ARG(b0 + b1 > 0 || zero16 == 0, "rope rows: a clear range needs rows");
   if (b0 + b1 == 0) return KS_OK;
   KS_CHECK_ARG((job1.rows == 0 || (job1.norm != nullptr) == stats) && (!stats || D == 64 || D == 128),
                "rope rows: statistics need D in {64, 128} and both jobs alike");
@@ -169,15 +162,13 @@ int launch_rope_rows(const RowJob &job0, const RowJob &job1, const float *freqs,
   const RowJobK k0 = kernel_job(job0), k1 = kernel_job(job1);
   const FastDiv cpr(static_cast<uint32_t>(D / 8));
   const uint32_t n0 = static_cast<uint32_t>(b0);
-  uint4 *zp = static_cast<uint4 *>(zero);
-  const uint32_t zn = static_cast<uint32_t>(zero16);
   const WeightScale ws = wscale != nullptr ? *wscale : WeightScale{nullptr, nullptr, 1.f, 0};
   if (stats && D == 128) {
-    hipLaunchKernelGGL(rope_rows_kernel<16>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, zp, zn, ws);
+    hipLaunchKernelGGL(rope_rows_kernel<16>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, ws);
   } else if (stats) {
-    hipLaunchKernelGGL(rope_rows_kernel<8>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, zp, zn, ws);
+    hipLaunchKernelGGL(rope_rows_kernel<8>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, ws);
   } else {
-    hipLaunchKernelGGL(rope_rows_kernel<0>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, zp, zn, ws);
+    hipLaunchKernelGGL(rope_rows_kernel<0>, grid, dim3(256), 0, stream, k0, k1, n0, freqs, D, cpr, rope_start, ws);
   }
   KS_CHECK_LAUNCH("rope_rows_kernel");
   return KS_OK;

@@ -30,9 +30,8 @@
 // ((||q|| ||k|| >= 2^126) treats every dot as a near tie.
 //
 // Bound mode (BOUND, bounded_scores) writes an approximate score and a bound U on its distance from the exact one, for a
-// selection that needs only the scores of its top k exactly; its counting form (COUNT) also builds each row's histogram
-// of the lower ends for the bounded top-k's threshold (per-wave LDS counts, flushed with one global atomic per nonzero
-// bucket).
+// selection that needs only the scores of its top k exactly; with few queries a batch (FEW) the waves of a workgroup
+// share the keys of one query.
 //
 // FP8 keys (F8, bound mode): k holds e4m3 codes with one fp32 scale per row, read directly (half the bytes of
 // bf16 rows) and dequantised in registers to the bf16 rows the contract defines, bf16(fp32(value * scale)), before
@@ -52,6 +51,8 @@ namespace {
 constexpr int kQW = 8;        // queries (= waves) per workgroup
 constexpr int kThreads = kQW * 64;
 constexpr int kKR = kScoreKeyBlock;  // keys per workgroup
+constexpr int64_t kFewQueries = 4;       // queries a batch up to which the few-queries form runs
+constexpr int64_t kFewTargetWgs = 2048;  // its workgroups, about
 constexpr int kEntCap = 32;   // deferred key entries per wave (flushed before another 16 could overflow them)
 static_assert(kEntCap >= 16, "16 listed keys are resolved at a time");
 static_assert(4 * kEntCap <= 255, "list entries hold the (entry, group) pair in 8 bits");
@@ -313,24 +314,21 @@ __device__ void flush_entries(ScoresLds<KD, HT> &L, int wave, int lane, int nent
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Shared memory of the bound-emitting form: the key block, each wave's head weights as bf16 values (high part, low part,
-// upper bound of |w|), and in the counting form each wave's counts of its row's lower ends (2048 buckets as 16-bit
-// halves: a wave counts at most kKR keys).  The counts take the LDS of a second workgroup per CU, so the counting form
-// is for grids of one round.
-template <int KD, bool COUNT>
+// Shared memory of the bound-emitting form: the key block (few queries: the query's rows instead), and the head weights
+// of each wave's query (few: of the one query) as bf16 values: high part, low part, upper bound of |w|, zero.
+template <int KD, bool FEW>
 struct ScoresLdsBound {
-  uint4 k[kKR * KD / 8];
-  uint32_t cnt[COUNT ? kQW : 0][1024];
-  uint16_t wf[kQW][4][64];  // rows hi, lo, |w| up, zero
+  uint4 k[(FEW ? 64 : kKR) * KD / 8];
+  uint16_t wf[FEW ? 1 : kQW][4][64];
 };
 
-// Waves per SIMD a kernel form is built for.  The non-counting bound kernel runs grids of several workgroups per CU: at
+// Waves per SIMD a kernel form is built for.  The bound kernel runs grids of several workgroups per CU: at
 // up to 128 VGPRs and 70 KiB of LDS two of them share a CU, so that one's prologue loads overlap the other's tiles (64
 // queries x 32768 keys: 40.7 us, against 49.1 at 147 VGPRs with the next tile's MFMAs issued a tile ahead).  The exact
 // kernel at 16 heads of 64 dims (the drop-in shape: 4 dots per lane and tile, a tile one chain of dependent steps) at
 // up to 128 VGPRs and 57 KiB of LDS does the same: four waves per SIMD hide each other's tile latency.
-template <int HT, int KD, bool BOUND, bool COUNT>
-constexpr int score_waves() { return (BOUND && !COUNT) ? 4 : (!BOUND && HT == 1 && KD == 64) ? 4 : 1; }
+template <int HT, int KD, bool BOUND, bool FEW>
+constexpr int score_waves() { return BOUND ? (FEW ? 2 : 4) : (!BOUND && HT == 1 && KD == 64) ? 4 : 1; }
 
 // e4m3 key chunks of the staging loop, dequantised to the contract's bf16 rows: 16 codes per load, rows past nk zero.
 template <int KD, int NV>
@@ -367,6 +365,68 @@ __device__ __forceinline__ float wave_sum_f32(float x) {
   return x;
 }
 
+// What a row's bounds are made of (the derivation is below): bf16 parts of the head weights, U = kC1 sum(w_up p) +
+// (the dots' own errors) + kC2 |S|, and the store of 64 keys' scores and bounds.
+struct WeightParts {
+  float up;  // w_up
+  uint16_t hi, lo, up16;
+};
+template <bool WBF>
+__device__ __forceinline__ WeightParts weight_parts(float w) {
+  WeightParts p;
+  p.up16 = w == 0.f ? 0 : max(bf16_abs_round_up(w), static_cast<uint16_t>(17 << 7));  // 2^-110
+  p.up = bf16_to_f32(p.up16);
+  const float hi = bf16_to_f32(static_cast<uint16_t>(cvt_pk_bf16(w, w) & 0xFFFFu));
+  p.hi = static_cast<uint16_t>(__builtin_bit_cast(uint32_t, hi) >> 16);
+  p.lo = WBF ? 0 : static_cast<uint16_t>(cvt_pk_bf16(w - hi, 0.f) & 0xFFFFu);
+  return p;
+}
+template <bool WBF>
+__device__ __forceinline__ void store_bounded(float *__restrict__ orow, float *__restrict__ urow, int key, bool in,
+                                              bool live, f32x4_t sums, float dsum, bool forced) {
+  constexpr float kC1 = WBF ? (0x1p-7f + 0x1p-8f) * 1.0625f : 0x1p-7f * 1.0625f;
+  constexpr float kC2 = WBF ? 0x1p-8f * 1.0625f : 0x1p-21f;
+  float sc = sums[0] + sums[1];
+  float u = __builtin_fmaf(kC2, fabsf(sc), __builtin_fmaf(kC1, sums[2], dsum)) + 0x1p-120f;
+  if (forced || !(fabsf(sc) + u < 3e38f)) {  // no statement about the score: it is always recomputed
+    sc = 0.f;
+    u = __builtin_inff();
+  }
+  if (in) {
+    orow[static_cast<uint32_t>(key)] = live ? sc : -INFINITY;
+    urow[static_cast<uint32_t>(key)] = live ? u : 0.f;
+  }
+}
+// The head-sum A operand of tile j: the lanes of rows 4 j .. 4 j + 3 keep wa (row l16 holds part l16 & 3 of the weights),
+// the others are zero.  Made in the loop: hoisted, the four forms would take 32 registers.
+__device__ __forceinline__ uint4 tile_weights(uint4 wa, int j) {
+  uint64_t rows = 0x000F000F000F000Full << (4 * j);
+  asm volatile("" : "+s"(rows));
+  const bool in = __builtin_amdgcn_inverse_ballot_w64(rows);
+  return make_uint4(in ? wa.x : 0u, in ? wa.y : 0u, in ? wa.z : 0u, in ? wa.w : 0u);
+}
+// wa for heads 32 hh + 4 g + 0 .. 3 and 16 above (the k-slots 8 g .. 8 g + 7 of the relu'd dots packed per lane)
+__device__ __forceinline__ uint4 head_weights(const uint16_t (&wf)[4][64], int hh, int l16, int g) {
+  const uint32_t *wr = reinterpret_cast<const uint32_t *>(wf[l16 & 3]);
+  const int h0 = 32 * hh + 4 * g, h1 = h0 + 16;
+  return make_uint4(wr[h0 / 2], wr[h0 / 2 + 1], wr[h1 / 2], wr[h1 / 2 + 1]);
+}
+// sums += the weighted relu'd bf16 dots of one 16-key tile (tile j of its four), from the tile's MFMA sums
+__device__ __forceinline__ f32x4_t add_tile(const f32x4_t (&acc)[4], const uint4 (&wa)[2], int j, f32x4_t sums) {
+  uint32_t p[8];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int rp = 0; rp < 2; ++rp) p[2 * m + rp] = cvt_relu_pk(acc[m][2 * rp], acc[m][2 * rp + 1]);
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh)
+    sums = mfma16(tile_weights(wa[hh], j), make_uint4(p[4 * hh], p[4 * hh + 1], p[4 * hh + 2], p[4 * hh + 3]), sums);
+  return sums;
+}
+__device__ __forceinline__ uint32_t row_scale(float upqn, float kns) {  // the same bits in every lane and workgroup
+  return __builtin_bit_cast(uint32_t, wave_sum_f32(upqn) * wave_max_f32(kns)) & 0x7FFFFFFFu;
+}
+
 // The bound-emitting form (64 heads): per (query, key) a score S and a bound U with |exact score - S| <= U, for a
 // selection that computes exactly only the scores that can reach its top k.  No dot is certified here: with A the MFMA
 // sum of a dot, p = max(bf16(A), 0) is within one bf16 rounding of each side of the exact relu'd value r,
@@ -386,13 +446,12 @@ __device__ __forceinline__ float wave_sum_f32(float x) {
 // instructions per tile, VALU-bound: 71.9 us at 64 queries x 32768 keys), this takes ~45; 40.7 us, 844 TFLOP/s, the
 // matrix cores busy ~45% of it (18 MFMAs per tile, 17.7 us of them) and the rest the workgroups' prologues (the block's
 // 64 KiB of keys and 128 KiB of query rows).  128 queries x 4096 keys, one workgroup per CU: 23.7 -> 21.0 us.
-template <bool WBF, bool COUNT, bool F8>
-__device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, const uint16_t *__restrict__ q,
+template <bool WBF, bool F8>
+__device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, false> &L, const uint16_t *__restrict__ q,
                                                const uint16_t *__restrict__ k, const void *__restrict__ w,
                                                const float *__restrict__ qn, const float *__restrict__ kn,
                                                float *__restrict__ scores, int64_t S, int T, int64_t kbs, int causal,
                                                int64_t start_pos, int ratio, float bound_c, float *__restrict__ bounds,
-                                               float *__restrict__ kmax, uint32_t *__restrict__ row_counts,
                                                uint32_t *__restrict__ row_state, const float *__restrict__ ksc, int kblk,
                                                int qgrp) {
   constexpr int KD = 128, HT = 4, H = 64, kC = KD / 8;
@@ -453,17 +512,15 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, co
   for (int j = 0; j < kKR / 64; ++j) knm = fmaxf(knm, lane + 64 * j < nk ? kn4[j] : 0.f);
   knm = wave_max_f32(knm);
   // lane h: head h's weight parts and its share of the row's bound
-  const uint16_t up16 = w_v == 0.f ? 0 : max(bf16_abs_round_up(w_v), static_cast<uint16_t>(17 << 7));  // 2^-110
-  const float up = bf16_to_f32(up16);
-  const float hi = bf16_to_f32(static_cast<uint16_t>(cvt_pk_bf16(w_v, w_v) & 0xFFFFu));
-  L.wf[wave][0][lane] = static_cast<uint16_t>(__builtin_bit_cast(uint32_t, hi) >> 16);
-  L.wf[wave][1][lane] = WBF ? 0 : static_cast<uint16_t>(cvt_pk_bf16(w_v - hi, 0.f) & 0xFFFFu);
-  L.wf[wave][2][lane] = up16;
+  const WeightParts wp = weight_parts<WBF>(w_v);
+  L.wf[wave][0][lane] = wp.hi;
+  L.wf[wave][1][lane] = wp.lo;
+  L.wf[wave][2][lane] = wp.up16;
   L.wf[wave][3][lane] = 0;
   const float dl = dot_halfwidth(qn_v, knm, bound_c);
   const bool forced = __builtin_amdgcn_ballot_w64(dl == __builtin_inff()) != 0ull;
-  const float dsum = wave_sum_f32(up * dl) * 1.03125f;  // sum_h w_up delta_h, (1 + 2^-7) and the fp32 sums covered
-  const uint32_t mrow = __builtin_bit_cast(uint32_t, wave_sum_f32(up * qn_v) * wave_max_f32(kns)) & 0x7FFFFFFFu;
+  const float dsum = wave_sum_f32(wp.up * dl) * 1.03125f;  // sum_h w_up delta_h, (1 + 2^-7) and the fp32 sums covered
+  const uint32_t mrow = row_scale(wp.up * qn_v, kns);
 
   if constexpr (F8) {
     stage_fp8_keys<KD>(L.k, kv, ksv, tid, nk);
@@ -478,36 +535,21 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, co
       L.k[kr * kC + (ch ^ (kr & (kC - 1)))] = make_uint4(kv[it].x & msk, kv[it].y & msk, kv[it].z & msk, kv[it].w & msk);
     }
   }
-  if constexpr (COUNT) {  // this wave's lower-end counts start at zero
-#pragma unroll
-    for (int i = 0; i < 4; ++i) reinterpret_cast<uint4 *>(L.cnt[wave])[lane + 64 * i] = make_uint4(0, 0, 0, 0);
-  }
   // the only barrier past the load ordering: LDS writes done, no wait for the q loads
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  // the block's key-norm maximum for the exact recomputation (every query group writes the same value)
-  if (tid == 0) kmax[b * gridDim.x + kblk] = knm;
   if (!s_ok) return;
-  if (kblk == 0 && lane == 0) row_state[4 * (b * S + s) + 3] = mrow;
+  if (kblk == 0 && lane == 0) row_state[2 * (b * S + s) + 1] = mrow;
 
   const int64_t limit = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
-  const int limit32 = static_cast<int>(limit < INT32_MAX ? limit : INT32_MAX);  // keys are below T < 2^31
   float *orow = scores + (b * S + s) * T;
   float *urow = bounds + (b * S + s) * T;
   const int64_t lim_rel = limit - kb0;
   const int nlk = lim_rel <= 0 ? 0 : (lim_rel < nk ? static_cast<int>(lim_rel) : nk);  // live keys of the block
   const int nlive = (nlk + 15) / 16;
 
-  // the head-sum A operand before its rows are masked per tile: row l16 holds part l16 & 3 of the weights of heads
-  // 16 m + 4 g + 0 .. 3 (m = 2 hh, 2 hh + 1)
-  uint4 wa[2];
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    const uint32_t *wr = reinterpret_cast<const uint32_t *>(L.wf[wave][l16 & 3]);
-    const int h0 = 32 * hh + 4 * g, h1 = h0 + 16;
-    wa[hh] = make_uint4(wr[h0 / 2], wr[h0 / 2 + 1], wr[h1 / 2], wr[h1 / 2 + 1]);
-  }
+  const uint4 wa[2] = {head_weights(L.wf[wave], 0, l16, g), head_weights(L.wf[wave], 1, l16, g)};
   auto tile_b = [&](int t, uint4(&bv)[KD / 32]) {
     const int key_l = 16 * t + l16;
 #pragma unroll
@@ -520,27 +562,6 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, co
     for (int kk = 0; kk < KD / 32; ++kk)
 #pragma unroll
       for (int m = 0; m < HT; ++m) acc[m] = mfma16(qa[m][kk], bv[kk], acc[m]);
-  };
-  constexpr float kC1 = WBF ? (0x1p-7f + 0x1p-8f) * 1.0625f : 0x1p-7f * 1.0625f;
-  constexpr float kC2 = WBF ? 0x1p-8f * 1.0625f : 0x1p-21f;
-  // the sums of 64 keys (lane: key key_l) stored, masked and counted
-  auto emit = [&](int key_l, f32x4_t sums) {
-    const int key = kb0 + key_l;
-    float sc = sums[0] + sums[1];
-    float u = __builtin_fmaf(kC2, fabsf(sc), __builtin_fmaf(kC1, sums[2], dsum)) + 0x1p-120f;
-    if (forced || !(fabsf(sc) + u < 3e38f)) {  // no statement about the score: it is always recomputed
-      sc = 0.f;
-      u = __builtin_inff();
-    }
-    const bool live = key_l < nlk;
-    if (key_l < nk) {
-      orow[static_cast<uint32_t>(key)] = live ? sc : -INFINITY;
-      urow[static_cast<uint32_t>(key)] = live ? u : 0.f;
-    }
-    if (COUNT && live) {
-      const uint32_t d = bound_digit(sc - u, mrow);
-      atomicAdd(&L.cnt[wave][d >> 1], 1u << ((d & 1u) * 16u));
-    }
   };
   if (nlive > 0) {
     // tiles past the last live one repeat it (their keys are masked)
@@ -555,21 +576,10 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, co
         f32x4_t acc[HT];
         tile_mfma(bv, acc);
         tile_b(t + 1 < nlive ? t + 1 : last, bv);
-        uint32_t p[2 * HT];
-#pragma unroll
-        for (int m = 0; m < HT; ++m)
-#pragma unroll
-          for (int rp = 0; rp < 2; ++rp) p[2 * m + rp] = cvt_relu_pk(acc[m][2 * rp], acc[m][2 * rp + 1]);
-        uint64_t rows = 0x000F000F000F000Full << (4 * j);  // lanes with l16 in 4 j .. 4 j + 3
-        asm volatile("" : "+s"(rows));  // the masked operands stay in the loop: hoisted, they would take 32 registers
-        const bool in = __builtin_amdgcn_inverse_ballot_w64(rows);
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-          const uint4 wj = make_uint4(in ? wa[hh].x : 0u, in ? wa[hh].y : 0u, in ? wa[hh].z : 0u, in ? wa[hh].w : 0u);
-          sums = mfma16(wj, make_uint4(p[4 * hh], p[4 * hh + 1], p[4 * hh + 2], p[4 * hh + 3]), sums);
-        }
+        sums = add_tile(acc, wa, j, sums);
       }
-      emit(16 * t0 + lane, sums);
+      const int key_l = 16 * t0 + lane;
+      store_bounded<WBF>(orow, urow, kb0 + key_l, key_l < nk, key_l < nlk, sums, dsum, forced);
     }
   }
   // keys past the last group of live tiles (at or past the causal limit)
@@ -577,35 +587,150 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, COUNT> &L, co
     orow[static_cast<uint32_t>(kb0 + key_l)] = -INFINITY;
     urow[static_cast<uint32_t>(kb0 + key_l)] = 0.f;
   }
-  if constexpr (COUNT) {
-    // the wave's counts into its row's histogram (only the nonzero buckets)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint32_t *hrow = row_counts + (b * S + s) * 2048;
+}
+
+// Few queries per batch (generation: one new token a sequence): a workgroup takes one query, and its 8 waves take 64-key
+// groups of their own, so that no wave idles (with a query per wave, one query would leave seven of eight idle).  No key
+// is used twice, so key fragments are read from memory as they are, each tile's registers refilled with the next group's
+// tile once its MFMAs are issued; the query's rows are staged once in LDS for the workgroup.  Scores and bounds as above
+// (the dots' error from the largest norm of the group's 64 keys).
+// 16 queries of one token over 16382 keys: see the launcher.
+template <bool WBF, bool F8>
+__device__ __forceinline__ void bounded_scores_few(ScoresLdsBound<128, true> &L, const uint16_t *__restrict__ q,
+                                                   const uint16_t *__restrict__ k, const void *__restrict__ w,
+                                                   const float *__restrict__ qn, const float *__restrict__ kn,
+                                                   float *__restrict__ scores, int64_t S, int T, int64_t kbs, int causal,
+                                                   int64_t start_pos, int ratio, float bound_c,
+                                                   float *__restrict__ bounds, uint32_t *__restrict__ row_state,
+                                                   const float *__restrict__ ksc) {
+  constexpr int KD = 128, HT = 4, H = 64, kC = KD / 8;
+  const uint8_t *__restrict__ k8 = reinterpret_cast<const uint8_t *>(k);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int64_t b = blockIdx.z, s = blockIdx.y, row = b * S + s;
+  const int ngrp = (T + 63) / 64, gstep = 8 * gridDim.x;  // group of this wave: wave + 8 blockIdx.x, then every gstep
+  const int64_t limit = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
+  const int nlk = limit <= 0 ? 0 : (limit < T ? static_cast<int>(limit) : T);  // live keys of the row
+  float *orow = scores + row * T;
+  float *urow = bounds + row * T;
+  const int64_t qrow0 = row * H;
+
+  // the first group's keys (rows past T read the last one), the query's rows and head data: all in flight together
+  uint4 bv[4][KD / 32];
+  uint2 bc[F8 ? 4 : 1][KD / 32];
+  float bs[F8 ? 4 : 1];
+  auto load_tile = [&](int grp, int j) {
+    const int key = 64 * grp + 16 * j + l16;
+    const int64_t kr = b * kbs + (key < T ? key : T - 1);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int wd = lane + 64 * i;
-      const uint32_t v = L.cnt[wave][wd];
-      if (v & 0xFFFFu) atomicAdd(&hrow[2 * wd], v & 0xFFFFu);
-      if (v >> 16) atomicAdd(&hrow[2 * wd + 1], v >> 16);
+    for (int kk = 0; kk < KD / 32; ++kk) {
+      if constexpr (F8)
+        bc[j][kk] = *reinterpret_cast<const uint2 *>(k8 + kr * KD + 32 * kk + 8 * g);
+      else
+        bv[j][kk] = *reinterpret_cast<const uint4 *>(k + kr * KD + 32 * kk + 8 * g);
     }
+    if constexpr (F8) bs[j] = ksc[kr];
+  };
+  auto load_norm = [&](int grp) {
+    const int key = 64 * grp + lane;
+    return kn[b * kbs + (key < T ? key : T - 1)];
+  };
+  int grp = wave + 8 * static_cast<int>(blockIdx.x);
+  const int grp0 = grp < ngrp ? grp : ngrp - 1;
+  uint4 qv[H * kC / kThreads];
+#pragma unroll
+  for (int i = 0; i < H * kC / kThreads; ++i) {
+    const int idx = tid + i * kThreads;
+    qv[i] = *reinterpret_cast<const uint4 *>(q + (qrow0 + idx / kC) * KD + 8 * (idx % kC));
+  }
+  const float qn_v = (qn + qrow0)[static_cast<uint32_t>(lane)];
+  const float w_v = WBF ? bf16_to_f32((static_cast<const uint16_t *>(w) + qrow0)[static_cast<uint32_t>(lane)])
+                        : (static_cast<const float *>(w) + qrow0)[static_cast<uint32_t>(lane)];
+  const float kns = (kn + b * kbs)[static_cast<uint32_t>((static_cast<int64_t>(lane) * T) >> 6)];
+  float kg = load_norm(grp0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) load_tile(grp0, j);
+  __builtin_amdgcn_sched_barrier(0);  // keep the key loads above the staging's waits
+
+#pragma unroll
+  for (int i = 0; i < H * kC / kThreads; ++i) {
+    const int idx = tid + i * kThreads, h = idx / kC, c = idx % kC;
+    L.k[h * kC + (c ^ (h & (kC - 1)))] = qv[i];
+  }
+  const WeightParts wp = weight_parts<WBF>(w_v);
+  L.wf[0][0][lane] = wp.hi;  // every wave writes the same values
+  L.wf[0][1][lane] = wp.lo;
+  L.wf[0][2][lane] = wp.up16;
+  L.wf[0][3][lane] = 0;
+  // sum_h w_up delta_h = bound_c 2^-23 (knm + pad) sum(w_up (qn + pad)) + 2^-144 sum(w_up), per group's knm
+  const float a1 = wave_sum_f32(wp.up * (qn_v + 0x1p-122f)) * bound_c * 0x1p-23f * 1.03125f;
+  const float a2 = wave_sum_f32(wp.up) * 0x1p-143f;
+  const float qpmax = wave_max_f32(qn_v) + 0x1p-122f;
+  const uint32_t mrow = row_scale(wp.up * qn_v, kns);
+  if (blockIdx.x == 0 && tid == 0) row_state[2 * row + 1] = mrow;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // LDS writes done, no wait for the key loads
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  uint4 qa[HT][KD / 32];
+#pragma unroll
+  for (int kk = 0; kk < KD / 32; ++kk)
+#pragma unroll
+    for (int m = 0; m < HT; ++m) qa[m][kk] = L.k[(16 * m + l16) * kC + ((4 * kk + g) ^ l16)];
+  const uint4 wa[2] = {head_weights(L.wf[0], 0, l16, g), head_weights(L.wf[0], 1, l16, g)};
+
+  for (; grp < ngrp; grp += gstep) {
+    const int nxt = grp + gstep < ngrp ? grp + gstep : grp;
+    const int key = 64 * grp + lane;
+    if (64 * grp >= nlk) {  // uniform: every key of the group is masked (and so are the later ones)
+      if (key < T) {
+        orow[key] = -INFINITY;
+        urow[key] = 0.f;
+      }
+      continue;
+    }
+    const float kp = wave_max_f32(kg) + 0x1p-122f;
+    kg = load_norm(nxt);
+    const bool forced = !(qpmax * kp < 0x1p126f);
+    const float dsum = __builtin_fmaf(a1, kp, a2);
+    f32x4_t sums = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (F8) {
+        if (__builtin_amdgcn_ballot_w64(!fp8_scale_pow2(bs[j])) == 0ull) {
+#pragma unroll
+          for (int kk = 0; kk < KD / 32; ++kk) bv[j][kk] = fp8_dequant8<true>(bc[j][kk], bs[j]);
+        } else {
+#pragma unroll
+          for (int kk = 0; kk < KD / 32; ++kk) bv[j][kk] = fp8_dequant8<false>(bc[j][kk], bs[j]);
+        }
+      }
+      f32x4_t acc[HT];
+#pragma unroll
+      for (int m = 0; m < HT; ++m) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < KD / 32; ++kk)
+#pragma unroll
+        for (int m = 0; m < HT; ++m) acc[m] = mfma16(qa[m][kk], bv[j][kk], acc[m]);
+      load_tile(nxt, j);
+      sums = add_tile(acc, wa, j, sums);
+    }
+    store_bounded<WBF>(orow, urow, key, key < T, key < nlk, sums, dsum, forced);
   }
 }
 
-template <int HT, int KD, bool WBF, bool BOUND, bool COUNT = false, bool F8 = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(score_waves<HT, KD, BOUND, COUNT>()))) void
+template <int HT, int KD, bool WBF, bool BOUND, bool FEW = false, bool F8 = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(score_waves<HT, KD, BOUND, FEW>()))) void
 indexer_scores_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const void *__restrict__ w,
     const float *__restrict__ qn, const int32_t *__restrict__ qsp, const float *__restrict__ kn,
     const int32_t *__restrict__ ksp, float *__restrict__ scores, int64_t S, int T, int64_t kbs, int causal,
     int64_t start_pos, int ratio, float bound_c, uint32_t *__restrict__ stats, int xcd_pk,
-    float *__restrict__ bounds, float *__restrict__ kmax, uint32_t *__restrict__ row_counts,
-    uint32_t *__restrict__ row_state, const float *__restrict__ ksc, float bound_r, const uint16_t *__restrict__ qsplit_rot, int qsplit_lo,
+    float *__restrict__ bounds, uint32_t *__restrict__ row_state, const float *__restrict__ ksc, float bound_r, const uint16_t *__restrict__ qsplit_rot, int qsplit_lo,
     int qsplit_hi) {
   constexpr int H = HT * 16;
   constexpr int kC = KD / 8;  // 16-byte chunks per key row
   static_assert(!BOUND || (HT == 4 && KD == 128), "the bound-emitting form is built for 64 heads of 128 dims");
-  static_assert(BOUND || !COUNT, "counts of lower ends need the bounds");
+  static_assert(BOUND || !FEW, "the few-queries form emits bounds");
   static_assert(!F8 || BOUND, "FP8 keys are read by the bound-emitting variant");
   // per-dot interval half-widths (step_halfwidth_scale: the step-weighted magnitude sum and the step exponents, on
   // the MFMA) instead of the per-head bound_c 2^-23 ||q_h|| max ||k||: under half as wide on typical rows, so
@@ -613,7 +738,12 @@ indexer_scores_kernel(
   // where the registers allow it (16 heads).
   constexpr bool PDD = HT == 1;
   constexpr int kSteps = KD / 8;  // accumulation steps of a dot
-  __shared__ std::conditional_t<BOUND, ScoresLdsBound<KD, COUNT>, ScoresLds<KD, HT>> L;
+  __shared__ std::conditional_t<BOUND, ScoresLdsBound<KD, FEW>, ScoresLds<KD, HT>> L;
+  if constexpr (FEW) {
+    bounded_scores_few<WBF, F8>(L, q, k, w, qn, kn, scores, S, T, kbs, causal, start_pos, ratio, bound_c, bounds,
+                                row_state, ksc);
+    return;
+  } else {
   // the wave index is uniform per wave; readfirstlane lets the compiler keep the query row, the causal limit
   // and the tile loop in scalar registers
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -651,8 +781,8 @@ indexer_scores_kernel(
     }
   }
   if constexpr (BOUND) {  // a body of its own; the rest is the exact kernel
-    bounded_scores<WBF, COUNT, F8>(L, q, k, w, qn, kn, scores, S, T, kbs, causal, start_pos, ratio, bound_c, bounds, kmax,
-                                   row_counts, row_state, ksc, kblk, qgrp);
+    bounded_scores<WBF, F8>(L, q, k, w, qn, kn, scores, S, T, kbs, causal, start_pos, ratio, bound_c, bounds, row_state,
+                            ksc, kblk, qgrp);
     return;
   } else {
 
@@ -1086,13 +1216,14 @@ indexer_scores_kernel(
     if (n_unres) atomicAdd(&stats[1], n_unres);
   }
   }  // !BOUND
+  }  // !FEW
 }
 
 template <int HT, int KD>
 int launch_scores_ht(const uint16_t *q, const uint16_t *k, const void *w, int w_bf16, const float *qn,
                      const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B, int64_t S,
                      int64_t T, int64_t kbs, int causal, int64_t start_pos, int ratio, float bound_c, uint32_t *stats,
-                     float *bounds, float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc, hipStream_t stream,
+                     float *bounds, uint32_t *row_state, const float *ksc, hipStream_t stream,
                      const QSplit *qsplit) {
   const QSplit qs = qsplit != nullptr ? *qsplit : QSplit{nullptr, 0, 0};
   dim3 grid(static_cast<unsigned>(ceil_div(T, kKR)), static_cast<unsigned>(ceil_div(S, kQW)),
@@ -1114,50 +1245,40 @@ int launch_scores_ht(const uint16_t *q, const uint16_t *k, const void *w, int w_
       }
     }
   }
-  if (ksc != nullptr && bounds == nullptr)
-    return fail(KS_ERR_INVALID, "indexer scores: FP8 keys need the bound-emitting kernel");
-  if (bounds != nullptr && ksc != nullptr) {
+  if (bounds != nullptr || ksc != nullptr) {
     if constexpr (HT == 4 && KD == 128) {
-      if (w_bf16) return fail(KS_ERR_INVALID, "indexer scores: score bounds need fp32 weights");
-      if (kmax == nullptr || row_state == nullptr)
-        return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax and row state buffers");
-      if (row_counts != nullptr) {
-        hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, true, true>), grid, dim3(kThreads), 0, stream, q,
-                           k, w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio,
-                           bound_c, stats, xcd_pk, bounds, kmax, row_counts, row_state, ksc, bound_r, qs.rot, qs.lo, qs.hi);
-      } else {
-        hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, false, true>), grid, dim3(kThreads), 0, stream,
-                           q, k, w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio,
-                           bound_c, stats, xcd_pk, bounds, kmax, nullptr, row_state, ksc, bound_r, qs.rot, qs.lo, qs.hi);
+      if (bounds == nullptr) return fail(KS_ERR_INVALID, "indexer scores: FP8 keys need the bound-emitting kernel");
+      if (row_state == nullptr) return fail(KS_ERR_INVALID, "indexer scores: score bounds need the row states");
+      // up to kFewQueries queries a batch: a workgroup per query, its waves over the keys (at most ~4 rounds of
+      // workgroups, each wave then taking several groups)
+      const bool few = S <= kFewQueries;
+      if (few) {
+        const int64_t per_row = ceil_div(T, 64 * kQW), rows = B * S;
+        const int64_t most = ceil_div(kFewTargetWgs, rows);
+        grid = dim3(static_cast<unsigned>(per_row < most ? per_row : most), static_cast<unsigned>(S),
+                    static_cast<unsigned>(B));
       }
-    } else {
-      return fail(KS_ERR_INVALID, "indexer scores: FP8 keys need H = 64 and D = 128");
-    }
-  } else if (bounds != nullptr) {
-    if constexpr (HT == 4 && KD == 128) {
+      auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, q, k, w, qn, qsp, kn, ksp, scores, S,
+                           static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c, stats, xcd_pk, bounds, row_state,
+                           ksc, bound_r, qs.rot, qs.lo, qs.hi);
+      };
       if (w_bf16) return fail(KS_ERR_INVALID, "indexer scores: score bounds need fp32 weights");
-      if (kmax == nullptr || row_state == nullptr)
-        return fail(KS_ERR_INVALID, "indexer scores: score bounds need the kmax and row state buffers");
-      if (row_counts != nullptr) {
-        hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, true>), grid, dim3(kThreads), 0, stream, q, k, w,
-                           qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c,
-                           stats, xcd_pk, bounds, kmax, row_counts, row_state, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
-      } else {
-        hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, true, false>), grid, dim3(kThreads), 0, stream, q, k,
-                           w, qn, qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c,
-                           stats, xcd_pk, bounds, kmax, nullptr, row_state, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
-      }
+      if (ksc != nullptr && few) run(indexer_scores_kernel<HT, KD, false, true, true, true>);
+      else if (ksc != nullptr) run(indexer_scores_kernel<HT, KD, false, true, false, true>);
+      else if (few) run(indexer_scores_kernel<HT, KD, false, true, true, false>);
+      else run(indexer_scores_kernel<HT, KD, false, true, false, false>);
     } else {
       return fail(KS_ERR_INVALID, "indexer scores: score bounds need H = 64 and D = 128");
     }
   } else if (w_bf16) {
     hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, true, false>), grid, dim3(kThreads), 0, stream, q, k, w, qn, qsp,
                        kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c, stats, xcd_pk,
-                       nullptr, nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                       nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
   } else {
     hipLaunchKernelGGL((indexer_scores_kernel<HT, KD, false, false>), grid, dim3(kThreads), 0, stream, q, k, w, qn,
                        qsp, kn, ksp, scores, S, static_cast<int>(T), kbs, causal, start_pos, ratio, bound_c, stats,
-                       xcd_pk, nullptr, nullptr, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
+                       xcd_pk, nullptr, nullptr, nullptr, bound_r, qs.rot, qs.lo, qs.hi);
   }
   KS_CHECK_LAUNCH("indexer_scores_kernel");
   return KS_OK;
@@ -1167,18 +1288,18 @@ template <int KD>
 int launch_scores_d(const uint16_t *q, const uint16_t *k, const void *w, int w_bf16, const float *qn,
                     const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B, int64_t S,
                     int64_t H, int64_t T, int64_t kbs, int causal, int64_t start_pos, int ratio, float bound_c,
-                    uint32_t *stats, float *bounds, float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc,
+                    uint32_t *stats, float *bounds, uint32_t *row_state, const float *ksc,
                     hipStream_t stream, const QSplit *qsplit) {
   switch (H) {
     case 16:
       return launch_scores_ht<1, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, row_state, ksc, stream, qsplit);
     case 32:
       return launch_scores_ht<2, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, row_state, ksc, stream, qsplit);
     case 64:
       return launch_scores_ht<4, KD>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, T, kbs, causal, start_pos,
-                                     ratio, bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
+                                     ratio, bound_c, stats, bounds, row_state, ksc, stream, qsplit);
     default:
       return fail(KS_ERR_INVALID, "indexer scores: H=%lld, supported: 16, 32, 64", (long long)H);
   }
@@ -1186,22 +1307,18 @@ int launch_scores_d(const uint16_t *q, const uint16_t *k, const void *w, int w_b
 
 }  // namespace
 
-bool scores_count_rows(int64_t B, int64_t S, int64_t T) {
-  return ceil_div(T, kKR) * ceil_div(S, kQW) * B <= kScoreCountGrid;
-}
-
 int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, int w_bf16, const float *qn,
                           const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B,
                           int64_t S, int64_t H, int64_t D, int64_t T, int64_t kbs, int causal, int64_t start_pos,
                           int ratio, float bound_c, uint32_t *stats, hipStream_t stream, float *bounds,
-                          float *kmax, uint32_t *row_counts, uint32_t *row_state, const float *ksc,
+                          uint32_t *row_state, const float *ksc,
                           const QSplit *qsplit) {
   if (D == 128)
     return launch_scores_d<128>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, H, T, kbs, causal, start_pos, ratio,
-                                bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
+                                bound_c, stats, bounds, row_state, ksc, stream, qsplit);
   if (D == 64)
     return launch_scores_d<64>(q, k, w, w_bf16, qn, qsp, kn, ksp, scores, B, S, H, T, kbs, causal, start_pos, ratio,
-                               bound_c, stats, bounds, kmax, row_counts, row_state, ksc, stream, qsplit);
+                               bound_c, stats, bounds, row_state, ksc, stream, qsplit);
   return fail(KS_ERR_INVALID, "indexer scores: D=%lld, supported: 64, 128", (long long)D);
 }
 
@@ -1264,10 +1381,9 @@ extern "C" int ks_dbg_indexer_scores(const uint16_t *q, const uint16_t *k, const
 }
 
 // Diagnostic variant of the bounded score kernel (not part of the public header), for timing it alone:
-// as ks_dbg_indexer_scores with fp32 weights, 64 heads and D = 128, plus the per-score bounds [B, S, T],
-// the key-block norm maxima [B, ceil(T / 256)] and the bounded selection's workspace part
-// (ks_dbg_topk_bounded_slots(B S, T) 64-bit slots).  Where the fused entry counts the rows in the score
-// kernel (ks::scores_count_rows), so does this one, into part's count region, which must then be zero.
+// as ks_dbg_indexer_scores with fp32 weights, 64 heads and D = 128, plus the per-score bounds [B, S, T] and the bounded
+// selection's workspace part (ks_dbg_topk_bounded_slots(B S, T) 64-bit slots), whose row states receive the rows'
+// histogram scales.  kmax is not used.
 extern "C" int ks_dbg_indexer_scores_bounded(const uint16_t *q, const uint16_t *k, const float *w,
                                              const float *q_norm, const int32_t *q_span, const float *k_norm,
                                              const int32_t *k_span, float *scores, float *bounds, float *kmax,
@@ -1276,12 +1392,11 @@ extern "C" int ks_dbg_indexer_scores_bounded(const uint16_t *q, const uint16_t *
   ks::last_error().clear();
   int rc = check_scores_args(q, k, w, q_norm, q_span, k_norm, k_span, scores, B, S, 64, 128, T, T, 1, start_pos);
   if (rc != KS_OK) return rc;
-  KS_CHECK_ARG(bounds && kmax && part, "ks_dbg_indexer_scores_bounded: null pointer");
+  KS_CHECK_ARG(bounds && part, "ks_dbg_indexer_scores_bounded: null pointer");
   KS_CHECK_ARG(T <= 32768, "ks_dbg_indexer_scores_bounded: T <= 32768");
   if (B * S == 0) return KS_OK;
   return ks::launch_indexer_scores(q, k, w, 0, q_norm, q_span, k_norm, k_span, scores, B, S, 64, 128, T, T,
                                    causal ? 1 : 0, start_pos, 1, ks::kScoreBoundC, nullptr,
-                                   static_cast<hipStream_t>(stream), bounds, kmax,
-                                   ks::scores_count_rows(B, S, T) ? ks::topk_bounded_counts(part, B * S, T) : nullptr,
-                                   ks::topk_bounded_state(part, B * S, T, ks::scores_count_rows(B, S, T)));
+                                   static_cast<hipStream_t>(stream), bounds,
+                                   ks::topk_bounded_state(part, B * S, T));
 }

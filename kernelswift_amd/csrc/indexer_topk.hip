@@ -575,49 +575,91 @@ inline int topk_slices(int64_t rows, int T) {
   return p;
 }
 
-// Capacity (composites) of a row's list of exact scores >= tau: the power of two >= T up to 8192 (a longer list
-// takes the whole-row fallback; k <= 2048 on this path, and the 11-bit threshold bucket can hold ~2000 more).
-constexpr int kTopkListCap = 8192;
-inline int topk_list_cap(int T) {
+// Composites of a row that the rank store takes in LDS (more take the whole-row fallback): twice the power of two >= k,
+// at least 2048, at most 4096 and the power of two >= T.  A list holds the top k and the scores within the bounds'
+// width of its last one, 1.1 to 1.2 k at N(0, 1) inputs.
+constexpr int kTopkListCap = 4096;
+inline int topk_list_cap(int T, int k) {
   int c = 128;
-  while (c < T && c < kTopkListCap) c <<= 1;
+  while (c < T && c < kTopkListCap && (c < 2048 || c < 2 * k)) c <<= 1;
   return c;
 }
 
-// 64-bit workspace slots of the bounded selection: the rows' lists, their slices' bucket counts (2048 x 32 bits
-// each), the rows' states (list length, threshold, largest key: 4 x 32 bits).
-inline int64_t topk_bounded_slots(int64_t rows, int NP, int cap) { return rows * cap + rows * NP * 1024 + rows * 2; }
+// Rows of at most this many columns are counted by each of their recomputation workgroups (the row's scores and bounds
+// come from L2, 64 KiB at most, counted into LDS); longer rows by a histogram launch over column slices.  128 rows of
+// 4096 columns: the recomputation grew by 0.5 us, against 5.5 us for counting in the score kernel (one global atomic
+// per nonzero bucket of every wave) and ~5 us for a launch.
+constexpr int kTopkSelfCount = 8192;
 
-// Wave-wide minimum and maximum (every lane receives both).
-__device__ __forceinline__ void wave_min_max(uint32_t &mn, uint32_t &mx) {
-#define KS_MM(S)                                             \
-  {                                                          \
-    const uint32_t a = lane_xor<S>(mn), b = lane_xor<S>(mx); \
-    mn = a < mn ? a : mn;                                    \
-    mx = b > mx ? b : mx;                                    \
+// The bounded selection's plan: columns per recomputation thread (8, 4 or 2, the largest that still gives ~512
+// workgroups, two per CU: each wave should own about one tile of candidates, whose chain of dependent steps sets its
+// time, while every workgroup stages the row's query once), segments per row, histogram slices (0: none) and their
+// width.
+struct SelPlan {
+  int kpb, segs, NP, W;
+};
+// Wave-wide maxima of two values (every lane receives both).
+__device__ __forceinline__ void wave_max2(uint32_t &a, uint32_t &b) {
+#define KS_MM(S)                                           \
+  {                                                        \
+    const uint32_t x = lane_xor<S>(a), y = lane_xor<S>(b); \
+    a = x > a ? x : a;                                     \
+    b = y > b ? y : b;                                     \
   }
   KS_MM(1) KS_MM(2) KS_MM(4) KS_MM(8) KS_MM(16) KS_MM(32)
 #undef KS_MM
 }
 
 // ---------------------------------------------------------------- rows of bounded scores
-// Bounded scores S with bounds U (the exact score lies in [S - U, S + U]; U = 0 exactly when S is exact) are
-// selected in three launches (two where the score kernel has counted the rows, TopkRecompute::counted):
-//  1. topk_slice_hist_kernel, workgroup (row, slice): counts of the first 11-bit digit (2048 buckets) of the lower
+// Bounded scores S with bounds U (the exact score lies in [S - U, S + U]) are selected in two launches, three for rows
+// past kTopkSelfCount columns:
+//  1. (long rows) topk_slice_hist_kernel, workgroup (row, slice): counts of the buckets (bound_digit, 2048) of the lower
 //     ends S - U of the slice's columns.
-//  2. topk_recompute_kernel, workgroup (row, segment): the threshold tau from the row's summed counts (the lower
-//     edge of the bucket holding the row's k-th largest lower end, so no exact score of the top k lies below it);
-//     every score of the segment with U > 0 whose upper end reaches tau is recomputed exactly and written back
-//     (S = exact, U = 0); every column whose upper end reaches tau has a slot in the row's list, which receives
-//     the composite (key, ~column) of its exact score, or key 0 (an empty slot) where that score fell below tau.
-//  3. topk_collected_kernel, one workgroup per row: the list holds every column of the top k, each with its exact
-//     score, so sorting its nonempty slots gives the top k.  A list longer than its capacity falls back to the exact selection over
-//     the whole row, whose keys are exact wherever they reach tau (the others enter as upper ends, below tau).
+//  2. topk_recompute_kernel, workgroup (row, segment): the threshold tau from the row's counts (the lower edge of the
+//     bucket holding the row's k-th largest lower end, so no exact score of the top k lies below it); every score of
+//     the segment whose upper end reaches tau is recomputed exactly, and the
+//     segment's list receives the composite (key, ~column) of its exact score, or key 0 (an empty slot) where that
+//     score fell below tau.  Every segment has a list of its own, of its own width: no atomics.
+//  3. topk_collected_kernel, one workgroup per row: the lists hold every column of the top k, each with its exact
+//     score, so sorting their nonempty slots gives the top k.  More slots than LDS takes
+//     fall back to the exact selection over the row, on keys spread from the lists (0 for the columns in none).
 constexpr int kRecD = 128;        // head dim of the recomputation
 constexpr int kRecH = 64;         // heads
 constexpr int kRecC = kRecD / 8;  // 16-byte chunks per row
 constexpr int kRecThreads = 512;  // the recomputation's workgroup
 constexpr int kRecWaves = kRecThreads / 64;
+
+inline SelPlan sel_plan(int64_t rows, int T) {
+  SelPlan p{8, 0, 0, kTopkThreads};
+  while (p.kpb > 2 && rows * ceil_div(T, kRecThreads * p.kpb) < 512) p.kpb >>= 1;
+  p.segs = static_cast<int>(ceil_div(T, kRecThreads * p.kpb));
+  if (T > kTopkSelfCount) {
+    const int np = topk_slices(rows, T);
+    while (p.W * np < T) p.W <<= 1;
+    p.NP = (T + p.W - 1) / p.W;
+  }
+  return p;
+}
+
+// The selection's regions in its workspace of 64-bit slots: the segments' lists (kRecThreads kpb composites each), the
+// slices' bucket counts (2048 x 32 bits each), the segments' states (slots used, largest key) and the rows' (tau, the
+// histogram scale).
+struct SelRegions {
+  uint64_t *lists;
+  uint32_t *hists;
+  uint2 *sstate, *rstate;
+  int64_t slots;
+};
+inline SelRegions sel_regions(uint64_t *part, int64_t rows, const SelPlan &p) {
+  SelRegions r{};
+  const int64_t nl = rows * p.segs * kRecThreads * p.kpb, nh = rows * p.NP * 1024, ns = rows * p.segs;
+  r.slots = nl + nh + ns + rows;
+  r.lists = part;
+  r.hists = reinterpret_cast<uint32_t *>(part + nl);
+  r.sstate = reinterpret_cast<uint2 *>(part + nl + nh);
+  r.rstate = r.sstate + ns;
+  return r;
+}
 
 // The row's query (64 heads) staged once per workgroup: rows in LDS with a 16-byte XOR swizzle (chunk c of
 // head h at c ^ (h & 15): the 16 lanes reading one chunk of 16 heads hit distinct banks), and the head
@@ -642,17 +684,17 @@ struct RecWave {
   int64_t limb[18];        // the integer accumulator of the rare dots beyond the double-precision paths
 };
 
-// Exact scores of the keys list[0 .. n) of one row, by the canonical contract, written over the row's
-// scores (srow, with bound 0 in urow) and over the keys' list slots (bit patterns of the scores).  Each wave takes tiles of 16 keys: four
+// Exact scores of the keys list[0 .. n) of one row, by the canonical contract, written over the keys'
+// list slots (bit patterns of the scores).  Each wave takes tiles of 16 keys: four
 // 16-head MFMA rounds (heads 16m + 4g + r, m = 0..3) with the score kernel's interval test (same
-// half-widths: bound_c 2^-23 ||q_h|| times the key block's norm maximum) keep the relu'd lower ends of all
+// half-widths: bound_c 2^-23 ||q_h|| times the key's norm) keep the relu'd lower ends of all
 // 64 heads; the tile's near-tie dots are then recomputed exactly, 16 at a time with a quad of lanes per dot
 // (q_h and the key row from LDS: exact_dot_bf16's arithmetic), and the fp32 fma head sum runs in the
 // canonical order over the corrected values.  F8: the key rows are e4m3 codes with row scales, dequantised in
 // registers to the contract's bf16 rows (q comes dequantised).
 template <int NW, bool F8>
-__device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow, const TopkRecompute &rc,
-                                 const RecShared &rs, RecWave &rw, int64_t kbrow0, int64_t kmax_row0, float qpmax,
+__device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
+                                 const RecShared &rs, RecWave &rw, int64_t kbrow0, float qpmax,
                                  uint32_t &n_exact, uint32_t &n_unres) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
@@ -662,7 +704,7 @@ __device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow,
     const bool kv = li < n;
     const int col = list[kv ? li : n - 1];
     const int64_t krow = kbrow0 + col;
-    // the tile's loads go out together (one round trip): key rows, key span, key-block norm maximum
+    // the tile's loads go out together (one round trip): key rows, key span and norm
     uint4 kb[kRecD / 32];
     uint2 kc8[F8 ? kRecD / 32 : 1];
     float kscale = 0.f;
@@ -675,7 +717,7 @@ __device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow,
       for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = *reinterpret_cast<const uint4 *>(rc.k + krow * kRecD + 32 * kk + 8 * g);
     }
     const int32_t ksv = rc.ksp[krow];
-    const float knm = rc.kmax[kmax_row0 + col / kScoreKeyBlock];
+    const float knm = rc.kn[krow];
     if constexpr (F8) {
       if (__builtin_amdgcn_ballot_w64(!fp8_scale_pow2(kscale)) == 0ull) {
 #pragma unroll
@@ -693,7 +735,7 @@ __device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow,
     // Interval half-widths: one fma per dot from the per-head factor qd (two roundings, within the three that
     // the bound constant allows for evaluating the width, so the width still bounds the MFMA error; it need not
     // equal the score kernel's, since any valid width certifies the same exact values).  When the query's
-    // largest padded norm times a key block's reaches 2^126 (uniform over the wave, and rare), the MFMA may
+    // largest padded norm times a key's reaches 2^126 (uniform over the wave, and rare), the MFMA may
     // overflow: every dot of the tile is then taken as a near tie and computed exactly.
     const float kp = knm + 0x1p-122f;
     const bool overflow = __builtin_amdgcn_ballot_w64(!(qpmax * kp < 0x1p126f)) != 0ull;
@@ -833,23 +875,18 @@ __device__ void recompute_scores(int32_t *list, int n, float *srow, float *urow,
     const float tot = combine_groups(G);
     // the score replaces its column in the list too (read back from LDS when the batch is the last one):
     // the tile's lanes read their list slots (and lanes past n read slot n - 1, of this same tile) before
-    if (g == 0 && kv) {
-      srow[col] = tot;
-      urow[col] = 0.f;
-      list[li] = __builtin_bit_cast(int32_t, tot);
-    }
+    if (g == 0 && kv) list[li] = __builtin_bit_cast(int32_t, tot);
   }
 }
 
 // Workgroup (row, slice): counts of the buckets (bound_digit, 2048) of the lower ends score - U of slice p's valid
-// columns, stored for the recomputation's threshold.  Workgroup (row, 0)
-// also clears the row's list length and key maximum (the recomputation appends to the list after this launch).
+// columns, stored for the recomputation's threshold.
 template <int KPT>
 __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const float *scores, const float *bounds,
                                                                       int64_t ld, int64_t S, int T, int causal,
                                                                       int64_t start_pos, int ratio, int W,
                                                                       uint32_t *__restrict__ hist_out,
-                                                                      uint32_t *__restrict__ rstate) {
+                                                                      const uint2 *__restrict__ rstate) {
   __shared__ uint32_t hist[2048];
   const int64_t row = blockIdx.x;
   const int64_t s = row % S;
@@ -870,11 +907,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
     sv[j] = src[col < nv ? col : 0];
     uv[j] = ub[col < nv ? col : 0];
   }
-  const uint32_t mrow = rstate[4 * row + 3];
-  if (blockIdx.y == 0 && tid == 0) {
-    rstate[4 * row] = 0u;
-    rstate[4 * row + 2] = 0u;
-  }
+  const uint32_t mrow = rstate[row].y;
   for (int i = tid; i < 2048; i += kTopkThreads) hist[i] = 0;
   __syncthreads();
 #pragma unroll
@@ -890,27 +923,31 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 
 // Workgroup (row, segment) of kRecThreads lanes over columns [c0, c0 + SW) of the row's valid prefix, SW =
 // kRecThreads KPB (column c0 + j kRecThreads + tid in slot j of thread tid):
-//  - tau: the row's NP bucket counts summed (thread t owns the kBPT buckets below 2048 - kBPT t), a block scan
-//    from the top bucket finds the bucket holding the row's k-th largest lower end; tau is its lower edge;
-//  - recomputation of the scores with U > 0 whose upper end reaches tau (recompute_scores), written back with
-//    U = 0;
-//  - the segment's columns whose upper end reaches tau fill a range of the row's list (capacity cap composites)
-//    reserved on the row's length counter: the exact key of each, or 0 where the exact score fell below tau; the
-//    row state also receives tau and an upper bound of its largest key (the largest upper end).
-// Row state (4 x 32 bits per row): list length (slots reserved), tau, largest key bound, unused.
+//  - tau: the row's bucket counts (NP slices of them summed, or, with NP = 0, counted here from the whole row's scores;
+//    thread t owns the kBPT buckets below 2048 - kBPT t), a block scan from the top bucket finds the bucket holding the
+//    row's k-th largest lower end; tau is its lower edge;
+//  - recomputation of the scores whose upper end reaches tau (recompute_scores); the scores and bounds in memory stay as
+//    they are, since the workgroups of the row's other segments may still be counting them;
+//  - these columns fill the segment's list, in column-slot order: the exact key of each, or 0 where the exact score
+//    fell below tau; the segment's state receives the number of slots and an upper bound of the largest key (the
+//    largest upper end), the row's state tau.
 template <int KPB, bool F8>
-__global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *scores, int64_t ld, int64_t S, int T,
+__global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const float *scores, int64_t ld, int64_t S, int T,
                                                                     int k, int causal, int64_t start_pos, int ratio,
                                                                     TopkRecompute rc, int segs, int NP,
                                                                     const uint32_t *__restrict__ hists,
-                                                                    uint64_t *__restrict__ lists, int cap,
-                                                                    uint32_t *__restrict__ rstate) {
+                                                                    uint64_t *__restrict__ lists,
+                                                                    uint2 *__restrict__ sstate,
+                                                                    uint2 *__restrict__ rstate) {
   constexpr int SW = kRecThreads * KPB;
   __shared__ RecShared rs;
   __shared__ RecWave rw[kRecWaves];
   __shared__ int32_t list[SW];
   __shared__ uint32_t wsum[kRecWaves];
-  __shared__ uint32_t s_tau, s_base;
+  __shared__ uint32_t s_tau, s_max[kRecWaves];
+  // the row's counts (NP = 0) share the LDS of the recomputation's scratch, which they precede
+  static_assert(sizeof(RecWave) * kRecWaves >= 2048 * sizeof(uint32_t), "bucket counts fit");
+  uint32_t *hist = reinterpret_cast<uint32_t *>(rw);
   // workgroups are dealt to the 8 XCDs round-robin (block id mod 8): the segments of one row are placed on one
   // XCD, so its L2 serves the row's query rows and bucket counts to all of them
   const int64_t nblk = gridDim.x;
@@ -928,8 +965,8 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   const int c0 = seg * SW;
   const int nv = n_valid - c0 <= 0 ? 0 : (n_valid - c0 < SW ? n_valid - c0 : SW);
   if (k_row == 0 || nv == 0) return;  // uniform, before any barrier: no valid column here
-  float *srow = scores + row * ld;
-  float *urow = rc.bounds + row * ld;
+  const float *srow = scores + row * ld;
+  const float *urow = rc.bounds + row * ld;
 
   // every load goes out before the first wait: the row's query chunks with its head data, the segment's scores
   // and bounds (column c0 stands in past the valid part), and the row's bucket counts (slice 0 stands in for
@@ -947,7 +984,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   const int hh = tid & (kRecH - 1);
   const float wv = rc.w[qrow0 + hh], qnv = rc.qn[qrow0 + hh];
   const int32_t qsv = rc.qsp[qrow0 + hh];
-  const uint32_t mrow = rstate[4 * row + 3];
+  const uint32_t mrow = rstate[row].y;
   float sv[KPB], uv[KPB];
 #pragma unroll
   for (int j = 0; j < KPB; ++j) {
@@ -955,12 +992,14 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
     sv[j] = srow[c0 + (col < nv ? col : 0)];
     uv[j] = urow[c0 + (col < nv ? col : 0)];
   }
-  uint4 hv[kTopkMaxSlices][kBPT / 4];
-  const uint32_t *hr = hists + row * NP * 2048 + (2048 - kBPT * (tid + 1));
-#pragma unroll
-  for (int p = 0; p < kTopkMaxSlices; ++p)
-#pragma unroll
-    for (int u = 0; u < kBPT / 4; ++u) hv[p][u] = *reinterpret_cast<const uint4 *>(hr + (p < NP ? p : 0) * 2048 + 4 * u);
+  static_assert(kBPT == 4, "one 16-byte read of a slice's buckets per thread");
+  uint4 hv0 = make_uint4(0, 0, 0, 0), hv1 = hv0, hv2 = hv0, hv3 = hv0;
+  if (NP > 0) {  // uniform; slice 0 stands in for the slices past NP
+    const uint32_t *hr = hists + row * NP * 2048 + (2048 - kBPT * (tid + 1));
+    auto slice = [&](int p) { return *reinterpret_cast<const uint4 *>(hr + (p < NP ? p : 0) * 2048); };
+    static_assert(kTopkMaxSlices == 4, "four slices");
+    hv0 = slice(0), hv1 = slice(1), hv2 = slice(2), hv3 = slice(3);
+  }
 #pragma unroll
   for (int i = 0; i < kQPT; ++i) {
     const int idx = tid + i * kRecThreads, h = idx / kRecC, c = idx % kRecC;
@@ -977,21 +1016,36 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   qpmax = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int32_t, qpmax)));
 
   // ---- tau: bucket e of the thread's kBPT is 2048 - kBPT (tid + 1) + e (the top one is e = kBPT - 1)
-  uint32_t hc[kBPT];
+  if (NP == 0) {  // uniform
+    reinterpret_cast<uint4 *>(hist)[tid] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    // eight columns per thread at a time, their loads in flight together
+    for (int j0 = 0; j0 * kRecThreads < n_valid; j0 += 8) {
+      float sa[8], ua[8];
 #pragma unroll
-  for (int e = 0; e < kBPT; ++e) hc[e] = 0u;
-#pragma unroll
-  for (int p = 0; p < kTopkMaxSlices; ++p) {
-    if (p < NP) {
-#pragma unroll
-      for (int u = 0; u < kBPT / 4; ++u) {
-        hc[4 * u] += hv[p][u].x;
-        hc[4 * u + 1] += hv[p][u].y;
-        hc[4 * u + 2] += hv[p][u].z;
-        hc[4 * u + 3] += hv[p][u].w;
+      for (int j = 0; j < 8; ++j) {
+        const int col = (j0 + j) * kRecThreads + tid;
+        sa[j] = srow[col < n_valid ? col : 0];
+        ua[j] = urow[col < n_valid ? col : 0];
       }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if ((j0 + j) * kRecThreads + tid < n_valid) atomicAdd(&hist[bound_digit(sa[j] - ua[j], mrow)], 1u);
     }
+    __syncthreads();
+    hv0 = *reinterpret_cast<const uint4 *>(hist + 2048 - kBPT * (tid + 1));
+  } else {
+    auto add = [&](uint4 h, bool in) {
+      hv0.x += in ? h.x : 0u;
+      hv0.y += in ? h.y : 0u;
+      hv0.z += in ? h.z : 0u;
+      hv0.w += in ? h.w : 0u;
+    };
+    add(hv1, NP > 1);
+    add(hv2, NP > 2);
+    add(hv3, NP > 3);
   }
+  const uint32_t hc[kBPT] = {hv0.x, hv0.y, hv0.z, hv0.w};
   uint32_t mine = 0;
 #pragma unroll
   for (int e = 0; e < kBPT; ++e) mine += hc[e];
@@ -1015,13 +1069,10 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   }
   __syncthreads();
   const uint32_t tau = s_tau;
-  if (seg == 0 && tid == 0) rstate[4 * row + 1] = tau;
+  if (seg == 0 && tid == 0) rstate[row].x = tau;
 
-  // ---- the segment's candidates (U > 0, upper end >= tau) and its list slots: every column whose upper end
-  // reaches tau (the candidates, and the exact scores >= tau) gets a slot, counted before the recomputation so
-  // that one block scan counts both (candidates in the low 16 bits, slots in the high 16: at most SW <= 4096 of
-  // each per workgroup) and the reservation is made as soon as a wave's own recomputation ends; a candidate whose
-  // exact score falls below tau leaves its slot empty (key 0, which the rank store skips).
+  // ---- the segment's candidates: every column whose upper end reaches tau, with U > 0 (a score with U = 0 is exact
+  // already and takes its slot as it is); one block scan counts candidates (low 16 bits) and slots (high 16)
   // (few registers stay live across the recomputation: the masks share one word, the bases another, and the
   // largest upper end is taken from hik afterwards)
   uint32_t hik[KPB], masks = 0;  // bit j: column j is a candidate; bit 8 + j: it has a slot
@@ -1052,32 +1103,34 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
   uint32_t n_exact = 0, n_unres = 0;
   if (ncand > 0) {
     const int64_t kbrow0 = b * rc.kbs;
-    const int64_t kmax_row0 = b * ((T + kScoreKeyBlock - 1) / kScoreKeyBlock);
-    recompute_scores<kRecWaves, F8>(list, static_cast<int>(ncand), srow, urow, rc, rs, rw[tid >> 6], kbrow0, kmax_row0, qpmax,
+    recompute_scores<kRecWaves, F8>(list, static_cast<int>(ncand), rc, rs, rw[tid >> 6], kbrow0, qpmax,
                                 n_exact, n_unres);
   }
-  // each wave, its own recomputation done (the atomics wait behind no tile load, and the last wave, which holds
-  // the fewest tiles, makes the reservation while the others finish theirs): the row's largest key, bounded by
-  // the largest upper end, and the workgroup's slots
   {
-    uint32_t umax = 0, unused = 0xFFFFFFFFu;
+    uint32_t umax = 0, unused = 0;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) umax = ((masks >> (8 + j)) & 1u) && hik[j] > umax ? hik[j] : umax;
-    wave_min_max(unused, umax);
-    if ((tid & 63) == 0 && umax != 0u) atomicMax(&rstate[4 * row + 2], umax);
+    wave_max2(unused, umax);
+    if ((tid & 63) == 0) s_max[tid >> 6] = umax;
   }
-  if (tid == kRecThreads - 1) s_base = nres > 0 ? atomicAdd(&rstate[4 * row], nres) : 0u;
-  __syncthreads();  // every recomputed score is in its list slot, and the reservation's base is known
+  __syncthreads();  // every recomputed score is in its list slot
+  const int64_t sg = row * segs + seg;
+  if (tid == 0) {
+    uint32_t m = s_max[0];
+#pragma unroll
+    for (int w = 1; w < kRecWaves; ++w) m = s_max[w] > m ? s_max[w] : m;
+    sstate[sg] = make_uint2(nres, m);
+  }
   if (rc.stats != nullptr) {
     if (n_exact) atomicAdd(&rc.stats[0], n_exact);
     if (n_unres) atomicAdd(&rc.stats[1], n_unres);
     if (rc.stats_ext && tid == 0 && ncand) atomicAdd(&rc.stats[2], ncand);
   }
 
-  // ---- the reserved slots: the exact key, or 0 where a recomputed score fell below tau
+  // ---- the segment's slots: the exact key, or 0 where a recomputed score fell below tau
   const float *listf = reinterpret_cast<const float *>(list);
-  uint64_t *dst = lists + row * cap;
-  uint32_t pos = s_base + (bexcl >> 16), p = bexcl & 0xFFFFu;
+  uint64_t *dst = lists + sg * SW;
+  uint32_t pos = bexcl >> 16, p = bexcl & 0xFFFFu;
 #pragma unroll
   for (int j = 0; j < KPB; ++j) {
     if ((masks >> (8 + j)) & 1u) {
@@ -1086,24 +1139,49 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(float *s
       p += cj ? 1u : 0u;
       if (key < tau) key = 0u;
       const uint32_t col = static_cast<uint32_t>(c0 + j * kRecThreads + tid);
-      if (pos < static_cast<uint32_t>(cap)) dst[pos] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
-      ++pos;
+      dst[pos++] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
     }
   }
 }
 
-// Sorted store of the k_sel largest of n unique composites, entry j * 1024 + tid in v[j] of thread tid, whose keys
-// lie in [kmin, kmax], by ranks from a counting sort: 2048 buckets uniform in the key over [kmin, kmax] (the bucket
-// is a monotone function of the key, so a higher bucket holds only larger composites); bucket starts from a block
+// Sorted store of the k_sel largest of the unique composites held in v (key 0: none; at most cap in all), whose keys
+// lie in [kmin, kmax], by ranks from a counting sort: 2048 buckets over [kmin, kmax] (RankScale: the bucket is a monotone
+// function of the key, so a higher bucket holds only larger composites); bucket starts from a block
 // scan from the top bucket; every entry is scattered into its bucket's range of tmp, and its rank is its bucket's
 // start plus the number of its bucket's entries above it.  Three barriers and O(n) work, against the log2(n)
 // dependent merge rounds of a sort.  Returns false, having stored nothing, when a bucket holds more than
 // kRankBucketMax entries (keys tied or clustered far beyond a smooth distribution); the caller then sorts.  Uses
-// sh.hist (counts, then starts), sh.wsum and tmp[0, n).
+// sh.hist (counts, then starts), sh.wsum and tmp[0, cap).
 constexpr int kRankBuckets = 2048;
 constexpr int kRankBucketMax = 256;
+// Uniform in the key (logarithmic in the score) over a positive range of at most eight octaves; otherwise uniform in the
+// score: a range that reaches down to zero or below it holds so many octaves of tiny magnitudes that uniform keys left
+// all large scores in a few buckets (12000 columns, k = 2048, where a third of the rows' k-th scores lie there:
+// the 128-row launch took 32.6 us, with this 7.7; 64 rows of 32768: 15.7 -> 7.7).
+struct RankScale {
+  uint32_t k0;
+  float v0, scale;
+  bool by_key;
+  __device__ __forceinline__ static float value(uint32_t key) {
+    return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
+  }
+  __device__ __forceinline__ RankScale(uint32_t kmin, uint32_t kmax) {
+    by_key = kmin >= 0x80000000u && kmax - kmin < (8u << 23);
+    // the ends as finite values (kmin may be below every value, kmax infinity)
+    const uint32_t lowest = 0x00800000u, highest = 0xFF7FFFFFu;  // keys of -/+ the largest finite value
+    k0 = kmin;
+    v0 = value(kmin < lowest ? lowest : kmin);
+    const float v1 = value(kmax > highest ? highest : kmax);
+    const float range = by_key ? static_cast<float>(kmax - kmin) + 1.0f : v1 - v0;
+    scale = range < 3e38f ? static_cast<float>(kRankBuckets) / fmaxf(range, 1e-30f) : 0.f;
+  }
+  __device__ __forceinline__ uint32_t bucket(uint32_t key) const {
+    const float d = (by_key ? static_cast<float>(key - k0) : value(key) - v0) * scale;
+    return d < static_cast<float>(kRankBuckets - 1) ? static_cast<uint32_t>(d > 0.f ? d : 0.f) : kRankBuckets - 1;
+  }
+};
 template <int PER>
-__device__ bool rank_store(const uint64_t (&v)[PER], int n, uint32_t kmin, uint32_t kmax, int k_sel, int64_t row,
+__device__ bool rank_store(const uint64_t (&v)[PER], uint32_t kmin, uint32_t kmax, int k_sel, int64_t row,
                            int k, void *out, int out_i64, int causal, int64_t limit, int64_t offset, uint64_t *tmp,
                            SelShared &sh) {
   static_assert(kRankBuckets == 2 * kTopkThreads, "two buckets per thread");
@@ -1112,15 +1190,14 @@ __device__ bool rank_store(const uint64_t (&v)[PER], int n, uint32_t kmin, uint3
   cnt[tid] = 0u;
   cnt[tid + kTopkThreads] = 0u;
   __syncthreads();
-  const float scale = static_cast<float>(kRankBuckets) / (static_cast<float>(kmax - kmin) + 1.0f);
+  const RankScale rk(kmin, kmax);
   uint32_t bk[PER], pos[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     bk[j] = 0u;
     pos[j] = 0u;
-    if (j * kTopkThreads + tid < n && (v[j] >> 32) != 0u) {  // key 0: an empty slot, not ranked
-      const uint32_t d = static_cast<uint32_t>(static_cast<float>(static_cast<uint32_t>(v[j] >> 32) - kmin) * scale);
-      bk[j] = d < kRankBuckets - 1 ? d : kRankBuckets - 1;
+    if ((v[j] >> 32) != 0u) {
+      bk[j] = rk.bucket(static_cast<uint32_t>(v[j] >> 32));
       pos[j] = atomicAdd(&cnt[bk[j]], 1u);  // the entry's place in its bucket (arrival order)
     }
   }
@@ -1133,11 +1210,11 @@ __device__ bool rank_store(const uint64_t (&v)[PER], int n, uint32_t kmin, uint3
   if (__syncthreads_or(c_hi > kRankBucketMax || c_lo > kRankBucketMax)) return false;  // uniform
 #pragma unroll
   for (int j = 0; j < PER; ++j)
-    if (j * kTopkThreads + tid < n && (v[j] >> 32) != 0u) tmp[start[bk[j]] + pos[j]] = v[j];
+    if ((v[j] >> 32) != 0u) tmp[start[bk[j]] + pos[j]] = v[j];
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    if (j * kTopkThreads + tid < n && (v[j] >> 32) != 0u) {
+    if ((v[j] >> 32) != 0u) {
       const uint32_t s0 = start[bk[j]], c = cnt[bk[j]];
       uint32_t r = s0, e = 0;
       // four members per step, read together (one LDS round trip per step, not per member)
@@ -1155,17 +1232,19 @@ __device__ bool rank_store(const uint64_t (&v)[PER], int n, uint32_t kmin, uint3
   return true;
 }
 
-// One workgroup per row: the row's list (every column of its top k, each with its exact score; at least k_sel
-// entries) sorted, and the first k_sel stored with the post-processing.  A list past its capacity (its length
-// counter still counts every entry) falls back to the exact selection over the row's keys: the score where
-// U = 0 (exact, recomputed ones included), the upper end elsewhere (below tau, so below every score of the top k).
+// One workgroup per row: the lists of the row's segments (together every column of its top k, each with its exact score;
+// at least k_sel entries) sorted, and the first k_sel stored with the post-processing.  2^tpl = 1024 / (the power of two
+// >= segs) threads read a segment's list; a list longer than those threads hold is first gathered in LDS.  More entries
+// than LDS takes (cap) fall back to the exact selection over the row's keys, spread by column into the row of the bounds
+// (which no launch reads any more).
 template <int KPT>
-__global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(const float *scores, const float *bounds,
-                                                                     int64_t ld, int64_t S, int T, int k, int causal,
+__global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *keys, int64_t ld, int64_t S, int T, int k, int causal,
                                                                      int64_t start_pos, int ratio, int64_t offset,
                                                                      void *__restrict__ out, int out_i64,
                                                                      const uint64_t *__restrict__ lists, int cap,
-                                                                     int spec, const uint32_t *__restrict__ rstate) {
+                                                                     int spec, int segs, int SW, int tpl,
+                                                                     const uint2 *__restrict__ sstate,
+                                                                     const uint2 *__restrict__ rstate) {
   extern __shared__ uint64_t cand[];  // 2 cap composites: the list, then the sort's exchange buffers
   __shared__ SelShared sh;
   const int64_t row = blockIdx.x;
@@ -1179,52 +1258,78 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(const floa
   }
   const int k_sel = k < n_valid ? k : n_valid;
   if (k_sel > 0) {
-    // the length and the list's first spec entries go out together (a list rarely runs much past k; the loads
-    // past the length are discarded), the rest of the list once the length asks for it
-    const uint4 st = *reinterpret_cast<const uint4 *>(rstate + 4 * row);  // length, tau, largest key
-    const uint32_t n = st.x;
-    const uint64_t *src = lists + row * cap;
+    // every wave reads the states of the row's segments (lane = segment; at most 64 of them), and each segment's threads
+    // the first spec rounds of its list with them (a list rarely runs much past its share of k; what lies past its
+    // length is discarded), the rest once the lengths ask for it
+    const int lane = tid & 63, nseg = (n_valid + SW - 1) / SW;
+    const uint2 ss = sstate[row * segs + (lane < nseg ? lane : 0)];
+    const uint32_t tau = rstate[row].x;
+    const int tps = 1 << tpl, seg = tid >> tpl, i0 = tid & (tps - 1);
+    const uint64_t *src = lists + (row * segs + (seg < nseg ? seg : 0)) * static_cast<int64_t>(SW);
     constexpr int kMaxPer = kTopkListCap / kTopkThreads;
     uint64_t v[kMaxPer];
 #pragma unroll
     for (int j = 0; j < kMaxPer; ++j) {
-      const int i = j * kTopkThreads + tid;
+      const int i = j * tps + i0;
       v[j] = 0;
-      if (j * kTopkThreads < spec) v[j] = src[i < cap ? i : 0];  // uniform
+      if (j < spec) v[j] = src[i < SW ? i : 0];  // uniform
     }
-#pragma unroll
-    for (int j = 0; j < kMaxPer; ++j) {
-      const int i = j * kTopkThreads + tid;
-      if (j * kTopkThreads >= spec && j * kTopkThreads < static_cast<int>(n < static_cast<uint32_t>(cap) ? n : cap))
-        v[j] = src[i < cap ? i : 0];  // uniform
-    }
+    const uint32_t c = lane < nseg ? ss.x : 0u;
+    const uint32_t incl = wave_incl_scan(c);
+    const uint32_t n = __builtin_amdgcn_readlane(incl, 63);
+    uint32_t most = c, top = lane < nseg ? ss.y : 0u;
+    wave_max2(most, top);
+    const uint32_t mine = __shfl(c, seg, 64);
+    auto gather = [&]() {  // the lists one after the other in LDS
+      for (int g = tid >> 6; g < nseg; g += kTopkWaves) {
+        const uint32_t len = __shfl(c, g, 64), at = __shfl(incl, g, 64) - len;
+        const uint64_t *gs = lists + (row * segs + g) * static_cast<int64_t>(SW);
+        for (uint32_t i = lane; i < len; i += 64) cand[at + i] = gs[i];
+      }
+      __syncthreads();
+    };
     if (n >= static_cast<uint32_t>(k_sel) && n <= static_cast<uint32_t>(cap)) {  // uniform
-      if (!rank_store<kMaxPer>(v, static_cast<int>(n), st.y, st.z, k_sel, row, k, out, out_i64, causal, limit, offset,
-                               cand, sh)) {
+      if (most <= static_cast<uint32_t>(kMaxPer * tps)) {  // uniform
+#pragma unroll
+        for (int j = 0; j < kMaxPer; ++j) {
+          const uint32_t i = static_cast<uint32_t>(j * tps + i0);
+          if (j >= spec && static_cast<uint32_t>(j * tps) < most) v[j] = src[i < static_cast<uint32_t>(SW) ? i : 0];  // uniform
+          if (i >= mine || seg >= nseg) v[j] = 0;
+        }
+      } else {
+        gather();
 #pragma unroll
         for (int j = 0; j < kMaxPer; ++j) {
           const uint32_t i = static_cast<uint32_t>(j * kTopkThreads + tid);
-          if (i < n) cand[i] = v[j];
+          v[j] = i < n ? cand[i] : 0;
         }
-        __syncthreads();
+      }
+      if (!rank_store<kMaxPer>(v, tau, top, k_sel, row, k, out, out_i64, causal, limit, offset, cand, sh)) {
+        gather();
         int P = 128;
         while (P < static_cast<int>(n)) P <<= 1;
         sort_merge_store(cand, P, static_cast<int>(n), k_sel, row, k, out, out_i64, causal, limit, offset, nullptr);
       }
     } else {
-      const float *src = scores + row * ld;
-      const float *ub = bounds + row * ld;
-      float sv[KPT], uv[KPT];
+      uint32_t *kr = keys + row * ld;
+      for (int i = tid; i < n_valid; i += kTopkThreads) kr[i] = 0u;
+      __syncthreads();
+      for (int g = tid >> 6; g < nseg; g += kTopkWaves) {
+        const uint32_t len = __shfl(c, g, 64);
+        const uint64_t *gs = lists + (row * segs + g) * static_cast<int64_t>(SW);
+        for (uint32_t i = lane; i < len; i += 64) {
+          const uint64_t e = gs[i];
+          kr[~static_cast<uint32_t>(e)] = static_cast<uint32_t>(e >> 32);
+        }
+      }
+      __threadfence_block();
+      __syncthreads();
+      uint32_t key[KPT];
 #pragma unroll
       for (int j = 0; j < KPT; ++j) {
         const int col = j * kTopkThreads + tid;
-        sv[j] = src[col < n_valid ? col : 0];
-        uv[j] = ub[col < n_valid ? col : 0];
+        key[j] = col < n_valid ? kr[col] : 0u;
       }
-      uint32_t key[KPT];
-#pragma unroll
-      for (int j = 0; j < KPT; ++j)
-        key[j] = j * kTopkThreads + tid < n_valid ? score_key(uv[j] > 0.f ? sv[j] + uv[j] : sv[j]) : 0u;
       if (tid == 0) sh.k_rem = static_cast<uint32_t>(k_sel);
       for (int i = tid; i < 2048; i += kTopkThreads) sh.hist[0][i] = 0;
       __syncthreads();
@@ -1293,32 +1398,19 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   if (rows == 0) return KS_OK;
   const int Ti = static_cast<int>(T), ki = static_cast<int>(k);
   const int c = causal ? 1 : 0, o = out_i64 ? 1 : 0;
-  // counted: the score kernel has counted each row whole (one slice); otherwise the histogram launch counts slices
-  const int np = rc.counted ? 1 : topk_slices(rows, Ti);
-  int W = kTopkThreads;  // columns per histogram slice: 1024 times a power of two
-  while (W * np < Ti) W <<= 1;
-  const int NP = (Ti + W - 1) / W;
-  const int cap = topk_list_cap(Ti);
-  // columns per recomputation thread: 8, 4 or 2, the largest that still gives ~512 workgroups (two per CU; each
-  // wave should own about one tile of candidates: the tile's chain of dependent steps, not the arithmetic, sets
-  // its time, while every workgroup stages the row's query once)
-  int kpb = 8;
-  while (kpb > 2 && rows * ((Ti + kRecThreads * kpb - 1) / (kRecThreads * kpb)) < 512) kpb >>= 1;
-  const int segs = (Ti + kRecThreads * kpb - 1) / (kRecThreads * kpb);
+  const SelPlan pl = sel_plan(rows, Ti);
+  const int segs = pl.segs, NP = pl.NP, W = pl.W, kpb = pl.kpb, cap = topk_list_cap(Ti, ki);
   KS_CHECK_ARG(rows * segs < (int64_t(1) << 31), "indexer top-k (bounded): too many rows");
-  const int64_t need = topk_bounded_slots(rows, NP, cap);
-  KS_CHECK_ARG(rc.part != nullptr && rc.part_cap >= need,
-               "indexer top-k (bounded): %lld 64-bit workspace slots required, %lld given", (long long)need,
+  const SelRegions rg = sel_regions(rc.part, rows, pl);
+  KS_CHECK_ARG(rc.part != nullptr && rc.part_cap >= rg.slots,
+               "indexer top-k (bounded): %lld 64-bit workspace slots required, %lld given", (long long)rg.slots,
                (long long)rc.part_cap);
-  uint64_t *lists = rc.part;
-  uint32_t *hists = reinterpret_cast<uint32_t *>(rc.part + rows * cap);
-  uint32_t *rstate = hists + rows * NP * 2048;
   const float *bnd = rc.bounds;
-  if (!rc.counted) {
+  if (NP > 0) {
     const dim3 hgrid(static_cast<unsigned>(rows), static_cast<unsigned>(NP));
 #define KS_HIST(KPT_)                                                                                          \
   hipLaunchKernelGGL(topk_slice_hist_kernel<KPT_>, hgrid, dim3(kTopkThreads), 0, st, scores, bnd, ld, S, Ti, c, \
-                     start_pos, ratio, W, hists, rstate)
+                     start_pos, ratio, W, rg.hists, rg.rstate)
     switch (W / kTopkThreads) {
       case 1: KS_HIST(1); break;
       case 2: KS_HIST(2); break;
@@ -1335,7 +1427,7 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   KS_CHECK_ARG(f8 == (rc.ks != nullptr), "indexer top-k (bounded): FP8 keys need codes and scales");
 #define KS_REC(KPB_, F8_)                                                                                           \
   hipLaunchKernelGGL((topk_recompute_kernel<KPB_, F8_>), rgrid, dim3(kRecThreads), 0, st, scores, ld, S, Ti, ki, c, \
-                     start_pos, ratio, rc, segs, NP, hists, lists, cap, rstate)
+                     start_pos, ratio, rc, segs, NP, rg.hists, rg.lists, rg.sstate, rg.rstate)
   if (f8) {
     if (kpb == 2) KS_REC(2, true);
     else if (kpb == 4) KS_REC(4, true);
@@ -1348,11 +1440,18 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
 #undef KS_REC
   KS_CHECK_LAUNCH("topk_recompute_kernel");
   const size_t shmem = static_cast<size_t>(2 * cap) * sizeof(uint64_t);
-  // list entries loaded with the length (a multiple of the workgroup): ~1.25 k, which the lists rarely exceed
-  const int spec = static_cast<int>(ceil_div(ki + ki / 4, kTopkThreads) * kTopkThreads);
+  // threads per segment's list: 1024 over the power of two >= segs (at most 32: T <= 32768, 1024 columns or more each)
+  int tpl = 10;
+  while ((kTopkThreads >> tpl) < segs) --tpl;
+  const int tps = 1 << tpl;
+  // rounds of a segment's list read with the lengths: its share of ~1.25 k (a list rarely holds more)
+  const int64_t share = ceil_div(static_cast<int64_t>(ki) + ki / 4, segs);
+  const int spec = static_cast<int>(share < kRecThreads * kpb ? ceil_div(share, tps) : ceil_div(kRecThreads * kpb, tps));
 #define KS_COLL(KPT_)                                                                                                \
   hipLaunchKernelGGL(topk_collected_kernel<KPT_>, dim3(static_cast<unsigned>(rows)), dim3(kTopkThreads), shmem, st, \
-                     scores, bnd, ld, S, Ti, ki, c, start_pos, ratio, offset, out, o, lists, cap, spec, rstate)
+                     reinterpret_cast<uint32_t *>(rc.bounds), ld, S, Ti, ki, c, start_pos, ratio, offset, out, o,    \
+                     rg.lists, cap, spec, segs, kRecThreads * kpb, tpl, rg.sstate,                                  \
+                     rg.rstate)
   if (Ti <= 1024) KS_COLL(1);
   else if (Ti <= 2048) KS_COLL(2);
   else if (Ti <= 4096) KS_COLL(4);
@@ -1364,34 +1463,20 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   return KS_OK;
 }
 
-uint32_t *ks::topk_bounded_state(uint64_t *part, int64_t rows, int64_t T, bool counted) {
-  const int Ti = static_cast<int>(T), np = counted ? 1 : topk_slices(rows, Ti);
-  int W = kTopkThreads;
-  while (W * np < Ti) W <<= 1;
-  return reinterpret_cast<uint32_t *>(part + rows * topk_list_cap(Ti)) + rows * ((Ti + W - 1) / W) * 2048;
-}
-
-uint32_t *ks::topk_bounded_counts(uint64_t *part, int64_t rows, int64_t T) {
-  // the lists first (rows x cap composites), then one slice of counts per row and the row states, as the
-  // launcher lays them out for NP = 1
-  return reinterpret_cast<uint32_t *>(part + rows * topk_list_cap(static_cast<int>(T)));
+uint32_t *ks::topk_bounded_state(uint64_t *part, int64_t rows, int64_t T) {
+  return reinterpret_cast<uint32_t *>(sel_regions(part, rows, sel_plan(rows, static_cast<int>(T))).rstate);
 }
 
 int64_t ks::topk_bounded_part_capacity(int64_t rows, int64_t T) {
   if (rows <= 0 || T < 1 || T > 32768) return 0;
-  const int Ti = static_cast<int>(T);
-  const int np = topk_slices(rows, Ti);
-  int W = kTopkThreads;
-  while (W * np < Ti) W <<= 1;
-  return topk_bounded_slots(rows, (Ti + W - 1) / W, topk_list_cap(Ti));
+  return sel_regions(nullptr, rows, sel_plan(rows, static_cast<int>(T))).slots;
 }
 
 // Diagnostic entry (not part of the public header) of the bounded top-k, for timing it alone: scores and
 // bounds from ks_dbg_indexer_scores_bounded over rotated q / k (with their row statistics); the scores that
 // are recomputed are rewritten in place (bound 0).  ratio 1, int32 output.  part: part_cap 64-bit slots, at
-// least ks_dbg_topk_bounded_slots(B S, T) of them, holding, where the fused entry counts the rows in the score
-// kernel (ks::scores_count_rows), the counts that ks_dbg_indexer_scores_bounded accumulated into its zeroed
-// count region; otherwise the selection counts the rows itself (its histogram launch).
+// least ks_dbg_topk_bounded_slots(B S, T) of them, as ks_dbg_indexer_scores_bounded left them (the rows' histogram
+// scales).  kmax is not read.
 extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const float *kmax, const uint16_t *q,
                                            const uint16_t *k, const float *w, const float *q_norm,
                                            const int32_t *q_span, const float *k_norm, const int32_t *k_span,
@@ -1399,11 +1484,11 @@ extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const f
                                            int64_t start_pos, void *out, void *stream, uint64_t *part,
                                            int64_t part_cap) {
   ks::last_error().clear();
-  KS_CHECK_ARG(scores && bounds && kmax && q && k && w && q_norm && q_span && k_norm && k_span && out && part,
+  KS_CHECK_ARG(scores && bounds && q && k && w && q_norm && q_span && k_norm && k_span && out && part,
                "ks_dbg_indexer_topk_bounded: null pointer");
   KS_CHECK_ARG(T <= 32768 && k_top <= 2048, "ks_dbg_indexer_topk_bounded: T <= 32768 and k <= 2048");
-  const ks::TopkRecompute rc{bounds, kmax, q, k, w, q_norm, q_span, k_norm, k_span, T, ks::kScoreBoundC, nullptr, 0,
-                             part, part_cap, ks::scores_count_rows(B, S, T) ? 1 : 0};
+  const ks::TopkRecompute rc{bounds, q, k, w, q_norm, q_span, k_norm, k_span, T, ks::kScoreBoundC, nullptr, 0, part,
+                             part_cap};
   return ks::launch_indexer_topk_bounded(scores, T, B, S, T, k_top, causal ? 1 : 0, start_pos, 1, 0, out, 0, rc,
                                          static_cast<hipStream_t>(stream));
 }

@@ -1,0 +1,73 @@
+"""The fused indexer's bounded path (64 heads of 128 dims) at the sizes where its forms change: few queries a batch
+(a workgroup per query), rows counted by the recomputation or by a histogram launch, and top-k lists that fall into one
+segment of a row; indices against the oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from kernelswift_amd import ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+_u16 = workloads.bf16_bits
+
+
+def _check(device, q, k, w, k_top, causal, start_pos, ratio=1, offset=0, rows=None):
+    tab = workloads.freqs_table(64, max(k.shape[1], start_pos + q.shape[1]) + 1)
+    got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), k_top, causal, start_pos, ratio, offset,
+                      0, 64, True).cpu().numpy().astype(np.int64)
+    for b in range(q.shape[0]):
+        want = oracle.indexer(_u16(q[b:b + 1]), _u16(k[b:b + 1]), w[b:b + 1].numpy() if w.dtype == torch.float32
+                              else _u16(w[b:b + 1]), tab.numpy(), k_top, causal, start_pos, ratio, offset, 0, 64, True)
+        np.testing.assert_array_equal(got[b:b + 1], want)
+
+
+# one to five queries (the few-queries form up to four); one key, a partial group of 64, a partial last workgroup;
+# 8192 and 8193 columns (counted by the recomputation / by the histogram launch); causal limits inside a group and before
+# the row's later groups; several groups per wave (B 9 x S 4 x T 16000)
+@pytest.mark.parametrize("B,S,T,k_top,causal,start,ratio", [
+    (1, 1, 1, 1, False, 0, 1), (2, 1, 63, 64, False, 0, 1), (3, 2, 65, 32, True, 30, 1), (1, 4, 511, 100, True, 508, 1),
+    (2, 3, 1025, 512, False, 700, 1), (1, 1, 8192, 512, False, 8191, 1), (1, 2, 8193, 2048, True, 8191, 1),
+    (1, 5, 8193, 700, True, 4000, 1), (2, 1, 5000, 300, True, 4399, 2), (1, 4, 600, 64, True, 0, 3)])
+def test_few_queries(device, B, S, T, k_top, causal, start, ratio):
+    g = torch.Generator().manual_seed(B * 7 + S * T)
+    q = torch.randn(B, S, 64, 128, generator=g).bfloat16()
+    k = torch.randn(B, T, 128, generator=g).bfloat16()
+    w = torch.randn(B, S, 64, generator=g) / 8
+    print(f"[case] few queries B={B} S={S} T={T} k={k_top} causal={causal} start={start}", flush=True)
+    _check(device, q, k, w, k_top, causal, start, ratio, offset=5)
+
+
+def test_few_queries_several_groups_per_wave(device):
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn(24, 4, 64, 128, generator=g).bfloat16()
+    k = torch.randn(24, 16000, 128, generator=g).bfloat16()
+    w = torch.randn(24, 4, 64, generator=g) / 8
+    print("[case] few queries, several groups per wave", flush=True)
+    tab = workloads.freqs_table(64, 16001)
+    got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), 256, True, 15996, 1, 0, 0, 64, True)
+    for b in (0, 23):  # the oracle on the first and last batch
+        want = oracle.indexer(_u16(q[b:b + 1]), _u16(k[b:b + 1]), w[b:b + 1].numpy(), tab.numpy(), 256, True, 15996, 1, 0,
+                              0, 64, True)
+        np.testing.assert_array_equal(got[b:b + 1].cpu().numpy().astype(np.int64), want)
+
+
+# the whole top k in one segment of the row (keys parallel to the queries there): its list outgrows the threads that read
+# it, and at T = 12000 with k = 2048 the others stay empty
+@pytest.mark.parametrize("S,T,k_top,lo", [(64, 12000, 2048, 8200), (3, 8192, 1500, 4096), (130, 4000, 1024, 2900)])
+def test_top_k_in_one_segment(device, S, T, k_top, lo):
+    g = torch.Generator().manual_seed(S + T)
+    q = torch.randn(1, S, 64, 128, generator=g)
+    q[..., 64:] = torch.randn(128 - 64, generator=g)  # the unrotated half, shared by every query and head
+    k = torch.randn(1, T, 128, generator=g) * 0.25
+    k[0, lo:lo + k_top, 64:] += q[0, 0, 0, 64:] * 2
+    q, k = q.bfloat16(), k.bfloat16()
+    w = torch.rand(1, S, 64, generator=g) / 8
+    print(f"[case] top k in one segment S={S} T={T} k={k_top}", flush=True)
+    rows = slice(0, min(S, 4))
+    tab = workloads.freqs_table(64, T + 1)
+    got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), k_top, False, 0, 1, 0, 0, 64, True)
+    want = oracle.indexer(_u16(q[:, rows]), _u16(k), w[:, rows].numpy(), tab.numpy(), k_top, False, 0, 1, 0, 0, 64, True)
+    np.testing.assert_array_equal(got[:, rows].cpu().numpy().astype(np.int64), want)
+    assert ((want >= lo) & (want < lo + k_top)).mean() > 0.9
