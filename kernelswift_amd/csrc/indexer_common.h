@@ -306,7 +306,8 @@ int launch_fp8_rows(const Fp8RowJob &job0, const Fp8RowJob &job1, int D, hipStre
 // Exact scores (bounds == nullptr), or, with bounds (H = 64, D = 128), a score and a bound U: the exact score lies in
 // [score - U, score + U], both ends also after rounding to nearest; row_state [B S][2] (word 1) then receives the scale of
 // each row's threshold histogram (bound_digit).  With ksc (bound mode), k holds e4m3 codes with those row scales (FP8
-// keys), read directly; kn / ksp are the statistics of the dequantised rows.
+// keys), read directly; kn / ksp are the statistics of the dequantised rows.  Bound mode: a batch's statistics start at
+// b * kns (0: like its rows, at b * kbs).
 constexpr int kScoreKeyBlock = 256;
 // q rows split over two buffers (the exact path when the row preparation wrote only the rotated dims): dims
 // [lo, hi) (32-aligned) from rot, the others from the q argument; rot == nullptr: all of q from the argument.
@@ -319,24 +320,27 @@ int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, i
                           const int32_t *qsp, const float *kn, const int32_t *ksp, float *scores, int64_t B,
                           int64_t S, int64_t H, int64_t D, int64_t T, int64_t kbs, int causal, int64_t start_pos,
                           int ratio, float bound_c, uint32_t *stats, hipStream_t stream, float *bounds = nullptr,
-                          uint32_t *row_state = nullptr, const float *ksc = nullptr, const QSplit *qsplit = nullptr);
+                          uint32_t *row_state = nullptr, const float *ksc = nullptr, const QSplit *qsplit = nullptr,
+                          int64_t kns = 0);
 
 // Sorted exact top-k of rows of bounded scores (the bound-emitting score kernel's output): a threshold from the
 // lower ends, exact recomputation of the scores that may reach the top k (interval test with the score kernel's
 // half-widths, exact double-precision dots for the near ties, canonical head sum),
 // then a sort of the exact scores at or above the threshold.  q / k: the rotated rows and their statistics
-// (64 heads, D = 128), w fp32 [B, S, 64]; with kc / ks set, the keys are e4m3 codes and row scales (the statistics
+// (64 heads, D = 128), w [B, S, 64]; with kc / ks set, the keys are e4m3 codes and row scales (the statistics
 // those of the dequantised rows), read directly and dequantised in registers.
 struct TopkRecompute {
   float *bounds;  // overwritten where a row's list outgrows LDS
   const uint16_t *q;
   const uint16_t *k;
-  const float *w;
+  const void *w;  // fp32, or bf16 (w_bf16)
+  int w_bf16;
   const float *qn;
   const int32_t *qsp;
   const float *kn;
   const int32_t *ksp;
-  int64_t kbs;  // key rows per batch in k, kn, ksp
+  int64_t kbs;  // key rows per batch in k (kc, ks)
+  int64_t kns;  // ... in kn, ksp
   float bound_c;
   uint32_t *stats;  // optional: [0] += exact dot recomputations, [1] += dots outside the exact range
   int stats_ext;    // with stats: [2] += recomputed scores

@@ -692,9 +692,9 @@ struct RecWave {
 // (q_h and the key row from LDS: exact_dot_bf16's arithmetic), and the fp32 fma head sum runs in the
 // canonical order over the corrected values.  F8: the key rows are e4m3 codes with row scales, dequantised in
 // registers to the contract's bf16 rows (q comes dequantised).
-template <int NW, bool F8>
+template <int NW, bool F8, bool WBF>
 __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
-                                 const RecShared &rs, RecWave &rw, int64_t kbrow0, float qpmax,
+                                 const RecShared &rs, RecWave &rw, int64_t kbrow0, int64_t knrow0, float qpmax,
                                  uint32_t &n_exact, uint32_t &n_unres) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
@@ -716,8 +716,8 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
 #pragma unroll
       for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = *reinterpret_cast<const uint4 *>(rc.k + krow * kRecD + 32 * kk + 8 * g);
     }
-    const int32_t ksv = rc.ksp[krow];
-    const float knm = rc.kn[krow];
+    const int32_t ksv = rc.ksp[knrow0 + col];
+    const float knm = rc.kn[knrow0 + col];
     if constexpr (F8) {
       if (__builtin_amdgcn_ballot_w64(!fp8_scale_pow2(kscale)) == 0ull) {
 #pragma unroll
@@ -803,7 +803,7 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
           } else {
             // wide dynamic range (rare): products above / below 2^(top - 38) accumulate separately
             const int li2 = 16 * t + kl;
-            const int64_t kr2 = kbrow0 + list[li2 < n ? li2 : n - 1];
+            const int64_t kr2 = knrow0 + list[li2 < n ? li2 : n - 1];
             const double thr = split ? ldexp(1.0, frexp_exp(rs.qn[h]) + frexp_exp(rc.kn[kr2]) - 38) : 0.0;
 #pragma unroll 1
             for (int c = 0; c < 8; ++c) {
@@ -864,15 +864,26 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
     }
+    // the canonical head sum: fma per head (fp32 weights), or the products of a pair rounded to bf16 together and added
+    // in head order, and the score rounded to bf16 (bf16 weights)
     float G = 0.f;
 #pragma unroll
     for (int m = 0; m < kRecH / 16; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t p2 = pl[2 * m + (r >> 1)];
-        G = __builtin_fmaf((r & 1) ? unpack_hi(p2) : unpack_lo(p2), rs.w[16 * m + 4 * g + r], G);
+      for (int rp = 0; rp < 2; ++rp) {
+        const uint32_t p2 = pl[2 * m + rp];
+        const float w0 = rs.w[16 * m + 4 * g + 2 * rp], w1 = rs.w[16 * m + 4 * g + 2 * rp + 1];
+        if constexpr (WBF) {
+          const uint32_t pr = cvt_pk_bf16(unpack_lo(p2) * w0, unpack_hi(p2) * w1);
+          G = G + unpack_lo(pr);
+          G = G + unpack_hi(pr);
+        } else {
+          G = __builtin_fmaf(unpack_lo(p2), w0, G);
+          G = __builtin_fmaf(unpack_hi(p2), w1, G);
+        }
       }
-    const float tot = combine_groups(G);
+    float tot = combine_groups(G);
+    if constexpr (WBF) tot = unpack_lo(cvt_pk_bf16(tot, tot));
     // the score replaces its column in the list too (read back from LDS when the batch is the last one):
     // the tile's lanes read their list slots (and lanes past n read slot n - 1, of this same tile) before
     if (g == 0 && kv) list[li] = __builtin_bit_cast(int32_t, tot);
@@ -931,7 +942,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 //  - these columns fill the segment's list, in column-slot order: the exact key of each, or 0 where the exact score
 //    fell below tau; the segment's state receives the number of slots and an upper bound of the largest key (the
 //    largest upper end), the row's state tau.
-template <int KPB, bool F8>
+template <int KPB, bool F8, bool WBF>
 __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const float *scores, int64_t ld, int64_t S, int T,
                                                                     int k, int causal, int64_t start_pos, int ratio,
                                                                     TopkRecompute rc, int segs, int NP,
@@ -982,7 +993,9 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     qv[i] = *reinterpret_cast<const uint4 *>(rc.q + (qrow0 + h) * kRecD + 8 * c);
   }
   const int hh = tid & (kRecH - 1);
-  const float wv = rc.w[qrow0 + hh], qnv = rc.qn[qrow0 + hh];
+  const float wv = WBF ? bf16_to_f32(static_cast<const uint16_t *>(rc.w)[qrow0 + hh])
+                       : static_cast<const float *>(rc.w)[qrow0 + hh];
+  const float qnv = rc.qn[qrow0 + hh];
   const int32_t qsv = rc.qsp[qrow0 + hh];
   const uint32_t mrow = rstate[row].y;
   float sv[KPB], uv[KPB];
@@ -1103,7 +1116,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   uint32_t n_exact = 0, n_unres = 0;
   if (ncand > 0) {
     const int64_t kbrow0 = b * rc.kbs;
-    recompute_scores<kRecWaves, F8>(list, static_cast<int>(ncand), rc, rs, rw[tid >> 6], kbrow0, qpmax,
+    recompute_scores<kRecWaves, F8, WBF>(list, static_cast<int>(ncand), rc, rs, rw[tid >> 6], kbrow0, b * rc.kns, qpmax,
                                 n_exact, n_unres);
   }
   {
@@ -1425,19 +1438,22 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   const dim3 rgrid(static_cast<unsigned>(rows * segs));
   const bool f8 = rc.kc != nullptr;
   KS_CHECK_ARG(f8 == (rc.ks != nullptr), "indexer top-k (bounded): FP8 keys need codes and scales");
-#define KS_REC(KPB_, F8_)                                                                                           \
-  hipLaunchKernelGGL((topk_recompute_kernel<KPB_, F8_>), rgrid, dim3(kRecThreads), 0, st, scores, ld, S, Ti, ki, c, \
-                     start_pos, ratio, rc, segs, NP, rg.hists, rg.lists, rg.sstate, rg.rstate)
-  if (f8) {
-    if (kpb == 2) KS_REC(2, true);
-    else if (kpb == 4) KS_REC(4, true);
-    else KS_REC(8, true);
-  } else {
-    if (kpb == 2) KS_REC(2, false);
-    else if (kpb == 4) KS_REC(4, false);
-    else KS_REC(8, false);
-  }
-#undef KS_REC
+  auto rec = [&](auto kern) {
+    hipLaunchKernelGGL(kern, rgrid, dim3(kRecThreads), 0, st, scores, ld, S, Ti, ki, c, start_pos, ratio, rc, segs, NP,
+                       rg.hists, rg.lists, rg.sstate, rg.rstate);
+  };
+  auto rec_k = [&](auto F8, auto WBF) {
+    constexpr bool f = decltype(F8)::value, wb = decltype(WBF)::value;
+    if (kpb == 2) rec(topk_recompute_kernel<2, f, wb>);
+    else if (kpb == 4) rec(topk_recompute_kernel<4, f, wb>);
+    else rec(topk_recompute_kernel<8, f, wb>);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (f8 && rc.w_bf16) rec_k(yes, yes);
+  else if (f8) rec_k(yes, no);
+  else if (rc.w_bf16) rec_k(no, yes);
+  else rec_k(no, no);
   KS_CHECK_LAUNCH("topk_recompute_kernel");
   const size_t shmem = static_cast<size_t>(2 * cap) * sizeof(uint64_t);
   // threads per segment's list: 1024 over the power of two >= segs (at most 32: T <= 32768, 1024 columns or more each)
@@ -1487,7 +1503,7 @@ extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const f
   KS_CHECK_ARG(scores && bounds && q && k && w && q_norm && q_span && k_norm && k_span && out && part,
                "ks_dbg_indexer_topk_bounded: null pointer");
   KS_CHECK_ARG(T <= 32768 && k_top <= 2048, "ks_dbg_indexer_topk_bounded: T <= 32768 and k <= 2048");
-  const ks::TopkRecompute rc{bounds, q, k, w, q_norm, q_span, k_norm, k_span, T, ks::kScoreBoundC, nullptr, 0, part,
+  const ks::TopkRecompute rc{bounds, q, k, w, 0, q_norm, q_span, k_norm, k_span, T, T, ks::kScoreBoundC, nullptr, 0, part,
                              part_cap};
   return ks::launch_indexer_topk_bounded(scores, T, B, S, T, k_top, causal ? 1 : 0, start_pos, 1, 0, out, 0, rc,
                                          static_cast<hipStream_t>(stream));

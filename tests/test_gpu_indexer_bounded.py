@@ -71,3 +71,34 @@ def test_top_k_in_one_segment(device, S, T, k_top, lo):
     want = oracle.indexer(_u16(q[:, rows]), _u16(k), w[:, rows].numpy(), tab.numpy(), k_top, False, 0, 1, 0, 0, 64, True)
     np.testing.assert_array_equal(got[:, rows].cpu().numpy().astype(np.int64), want)
     assert ((want >= lo) & (want < lo + k_top)).mean() > 0.9
+
+
+# bf16 head weights: products and scores rounded to bf16, so that many scores tie and the order rests on the columns
+@pytest.mark.parametrize("B,S,T,k_top,causal,start,scale", [
+    (1, 24, 3000, 512, True, 2976, 1.0), (2, 1, 9000, 512, False, 8999, 1.0), (2, 3, 700, 700, True, 100, 1.0),
+    (1, 40, 750, 512, True, 0, 1.0), (1, 9, 2048, 300, False, 0, 2.0 ** -60), (1, 9, 2048, 300, False, 0, 2.0 ** 40)])
+def test_bf16_weights(device, B, S, T, k_top, causal, start, scale):
+    g = torch.Generator().manual_seed(B + S * T)
+    q = (torch.randn(B, S, 64, 128, generator=g) * scale).bfloat16()
+    k = torch.randn(B, T, 128, generator=g).bfloat16()
+    w = (torch.randn(B, S, 64, generator=g) * 0.05)
+    w[:, :, ::9] = 0.0
+    print(f"[case] bf16 weights B={B} S={S} T={T} k={k_top} causal={causal} scale={scale}", flush=True)
+    _check(device, q, k, w.bfloat16(), k_top, causal, start)
+
+
+@pytest.mark.parametrize("wbf", [False, True])
+def test_equal_keys_and_tiny_weights(device, wbf):
+    # every key the same row (every score ties: the columns decide), and weights from subnormal to large
+    g = torch.Generator().manual_seed(6)
+    q = torch.randn(1, 6, 64, 128, generator=g).bfloat16()
+    k = torch.randn(1, 1, 128, generator=g).expand(1, 5000, 128).contiguous().bfloat16()
+    w = torch.randn(1, 6, 64, generator=g)
+    w[0, 1] = 0.0
+    w[0, 2] *= 2.0 ** -130
+    w[0, 3] *= 2.0 ** -115
+    w[0, 4] *= 2.0 ** 60
+    print(f"[case] equal keys, weights of all magnitudes, bf16={wbf}", flush=True)
+    _check(device, q, k, w.bfloat16() if wbf else w, 600, False, 0)
+    k = torch.randn(1, 1500, 128, generator=g).bfloat16()
+    _check(device, q, k, w.bfloat16() if wbf else w, 600, False, 0)
