@@ -84,9 +84,9 @@ int check_indexer_args(const char *fn, int64_t k_top, int64_t start_pos, int32_t
 }
 
 // Whether the scores take the bounded path (path: 0 = bounded when the shape allows it, 1 = exact, 2 = bounded,
-// 3 = bounded with the extended counters).  It is the faster one even where nearly every score has to be recomputed:
-// bf16 weights, 2 x 3001 queries of a prompt over 750 keys, k 512: scores and selection 689 us exact, 453 us bounded; 16
-// single queries over 16382 keys: 199 and 43 us.
+// 3 = bounded with the extended counters).  It is the faster one even where nearly every score has to be recomputed (rows
+// of at most 1024 keys then skip the approximate scores: topk_bounded_all): bf16 weights, 2 x 3001 queries of a prompt
+// over 750 keys, k 512: scores and selection 689 us exact, 232 us bounded; 16 single queries over 16382 keys: 199 and 43 us.
 bool takes_bounded(int64_t k_top, int64_t H, int64_t D, int64_t T, int path) {
   const int64_t kk = k_top < T ? k_top : T;
   return H == 64 && D == 128 && T <= 32768 && kk <= 2048 && path != 1;
@@ -115,16 +115,19 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
     // FP8 keys: the codes with their row scales (the statistics are indexed like the rows: B == 1 or kbs == T)
     const uint16_t *krows = direct ? reinterpret_cast<const uint16_t *>(f8.kc) : ws.k_rot;
     const int64_t kbs = direct ? f8.kbs : T;
-    rc = ks::launch_indexer_scores(ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm, ws.q_span, ws.k_norm, ws.k_span,
-                                   ws.scores, B, S, H, D, T, kbs, causal ? 1 : 0, start_pos, ratio, bound_c, nullptr, st, ws.bounds,
-                                   ks::topk_bounded_state(ws.part, B * S, T), f8.ks, nullptr, T);
-    if (rc != KS_OK) return rc;
+    const bool all = ks::topk_bounded_all(S, T, kk, causal ? 1 : 0, start_pos, ratio);
+    if (!all) {
+      rc = ks::launch_indexer_scores(ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm, ws.q_span, ws.k_norm, ws.k_span,
+                                     ws.scores, B, S, H, D, T, kbs, causal ? 1 : 0, start_pos, ratio, bound_c, nullptr, st,
+                                     ws.bounds, ks::topk_bounded_state(ws.part, B * S, T), f8.ks, nullptr, T);
+      if (rc != KS_OK) return rc;
+    }
     ks::TopkRecompute trc{ws.bounds, ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm,
                           ws.q_span, ws.k_norm, ws.k_span, kbs, T, bound_c, stats, path == 3 ? 1 : 0, ws.part,
                           ws.part_cap};
     trc.kc = f8.kc;
     trc.ks = f8.ks;
-    return ks::launch_indexer_topk_bounded(ws.scores, T, B, S, T, kk, causal ? 1 : 0, start_pos, ratio, offset, out,
+    return ks::launch_indexer_topk_bounded(all ? nullptr : ws.scores, T, B, S, T, kk, causal ? 1 : 0, start_pos, ratio, offset, out,
                                            out_i64 ? 1 : 0, trc, st);
   }
   // q_unrot: the caller's q rows, whose dims outside [rot_lo, rot_hi) the row preparation did not copy (ws.q_rot

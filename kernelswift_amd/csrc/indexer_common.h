@@ -353,6 +353,9 @@ struct TopkRecompute {
 };
 // Slots the bounded selection needs for `rows` rows of T <= 32768 columns (0 outside that range).
 int64_t topk_bounded_part_capacity(int64_t rows, int64_t T);
+// Whether the bounded selection of rows of T columns should compute every score exactly, without scores and bounds
+// (launch_indexer_topk_bounded then takes scores == nullptr): it recomputes what may reach the top k anyway.
+bool topk_bounded_all(int64_t S, int64_t T, int64_t k, int causal, int64_t start_pos, int ratio);
 // The row states in part ([rows][2]: tau, histogram scale); the score kernel writes the scale.
 uint32_t *topk_bounded_state(uint64_t *part, int64_t rows, int64_t T);
 // ks_indexer_topk with the caller's guarantee that every score is a bf16 value (bf16_vals = 1), which spares the

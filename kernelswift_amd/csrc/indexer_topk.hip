@@ -206,6 +206,7 @@ __device__ __forceinline__ void run_sort(V (&v)[2], int lane) {
 // log2(P / 128) merge-path rounds then double the runs through the two halves of cand[0, 2P), one
 // barrier each, and the last round stores.  ~10 dependent LDS reads per round per thread, against the
 // bitonic network's log2(P) (log2(P) + 1) / 2 stages, of which those at distances >= 64 need a barrier.
+template <int NT = kTopkThreads>
 __device__ void sort_merge_store(uint64_t *cand, int P, int n, int k_sel, int64_t row, int k, void *out,
                                  int out_i64, int causal, int64_t limit, int64_t offset, uint64_t *part) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -218,7 +219,7 @@ __device__ void sort_merge_store(uint64_t *cand, int P, int n, int k_sel, int64_
     }
   };
   const int runs = P / 128;
-  for (int rr = wave; rr < runs; rr += kTopkWaves) {
+  for (int rr = wave; rr < runs; rr += NT / 64) {
     uint64_t v[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
@@ -238,7 +239,7 @@ __device__ void sort_merge_store(uint64_t *cand, int P, int n, int k_sel, int64_
   if (runs == 1) return;
   __syncthreads();
   uint64_t *src = cand, *dst = cand + P;
-  const int E = P > kTopkThreads ? P / kTopkThreads : 1;  // outputs per thread and round
+  const int E = P > NT ? P / NT : 1;  // outputs per thread and round
   for (int L = 128; L < P; L <<= 1) {  // every thread runs every round (P is uniform)
     const int d = tid * E;
     const int pair = d / (2 * L), d0 = d % (2 * L);
@@ -631,6 +632,7 @@ constexpr int kRecWaves = kRecThreads / 64;
 
 inline SelPlan sel_plan(int64_t rows, int T) {
   SelPlan p{8, 0, 0, kTopkThreads};
+  if (T <= 2 * kRecThreads) p.kpb = 2;  // one segment: the recomputation ranks and stores the row
   while (p.kpb > 2 && rows * ceil_div(T, kRecThreads * p.kpb) < 512) p.kpb >>= 1;
   p.segs = static_cast<int>(ceil_div(T, kRecThreads * p.kpb));
   if (T > kTopkSelfCount) {
@@ -652,7 +654,8 @@ struct SelRegions {
 };
 inline SelRegions sel_regions(uint64_t *part, int64_t rows, const SelPlan &p) {
   SelRegions r{};
-  const int64_t nl = rows * p.segs * kRecThreads * p.kpb, nh = rows * p.NP * 1024, ns = rows * p.segs;
+  // one segment of two columns per thread: ranked by the recomputation, no lists
+  const int64_t nl = p.segs == 1 && p.kpb == 2 ? 0 : rows * p.segs * kRecThreads * p.kpb, nh = rows * p.NP * 1024, ns = rows * p.segs;
   r.slots = nl + nh + ns + rows;
   r.lists = part;
   r.hists = reinterpret_cast<uint32_t *>(part + nl);
@@ -669,6 +672,7 @@ struct RecShared {
   float w[kRecH];
   float qn[kRecH];
   float qd[kRecH];  // bound_c 2^-23 (qn + 2^-122): the per-head factor of the interval half-widths
+  uint16_t wneg[kRecH];  // all ones where the head's weight is negative
   int32_t qsp[kRecH];
 };
 
@@ -679,81 +683,179 @@ __device__ __forceinline__ uint4 rec_q(const RecShared &rs, int h, int c) { retu
 constexpr int kNearCap = 256;  // near-tie dots listed at a time (a tile has at most 64 x 16)
 struct RecWave {
   uint4 k[16 * kRecC];
-  int32_t ksp[16];         // the tile's key spans
+  int32_t ksp[16];         // the tile's key spans and norms
+  float kn[16];
   uint16_t ent[kNearCap];  // lane << 4 | head bit (4 m + r); overwritten by the dot's exact value
   int64_t limb[18];        // the integer accumulator of the rare dots beyond the double-precision paths
 };
 
-// Exact scores of the keys list[0 .. n) of one row, by the canonical contract, written over the keys'
+// A pair of heads' terms of the canonical sum (relu'd bf16 dots p2): fma per head (fp32 weights), or the products of the
+// pair rounded to bf16 together and added in head order (bf16 weights).
+template <bool WBF>
+__device__ __forceinline__ void head_sum(uint32_t p2, float w0, float w1, float &G) {
+  if constexpr (WBF) {
+    const uint32_t pr = cvt_pk_bf16(unpack_lo(p2) * w0, unpack_hi(p2) * w1);
+    G = G + unpack_lo(pr);
+    G = G + unpack_hi(pr);
+  } else {
+    G = __builtin_fmaf(unpack_lo(p2), w0, G);
+    G = __builtin_fmaf(unpack_hi(p2), w1, G);
+  }
+}
+
+// A tile of 16 keys' rows as loaded (lane (l16, g): chunks 4 kk + g of the key at row krow), and as MFMA B-fragments.  F8:
+// e4m3 codes with row scales, dequantised in registers to the contract's bf16 rows.
+template <bool F8>
+struct TileKeys {
+  uint4 kb[F8 ? 1 : kRecD / 32];
+  uint2 kc[F8 ? kRecD / 32 : 1];
+  float scale;
+  __device__ __forceinline__ void load(const TopkRecompute &rc, int64_t krow, int g) {
+    if constexpr (F8) {
+#pragma unroll
+      for (int kk = 0; kk < kRecD / 32; ++kk) kc[kk] = *reinterpret_cast<const uint2 *>(rc.kc + krow * kRecD + 32 * kk + 8 * g);
+      scale = rc.ks[krow];
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = *reinterpret_cast<const uint4 *>(rc.k + krow * kRecD + 32 * kk + 8 * g);
+    }
+  }
+  __device__ __forceinline__ void fragments(uint4 (&f)[kRecD / 32]) const {
+    if constexpr (!F8) {
+#pragma unroll
+      for (int kk = 0; kk < kRecD / 32; ++kk) f[kk] = kb[kk];
+    } else if (__builtin_amdgcn_ballot_w64(!fp8_scale_pow2(scale)) == 0ull) {
+#pragma unroll
+      for (int kk = 0; kk < kRecD / 32; ++kk) f[kk] = fp8_dequant8<true>(kc[kk], scale);
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < kRecD / 32; ++kk) f[kk] = fp8_dequant8<false>(kc[kk], scale);
+    }
+  }
+};
+
+// The relu'd bf16 ends of a tile's dots: word 2 m + rp holds heads 16 m + 4 g + 2 rp (low half) and the next.  Interval
+// half-widths: one fma per dot from the per-head factor qd (two roundings, within the three that the bound constant
+// allows for evaluating the width, so the width still bounds the MFMA error; it need not equal the score kernel's, since
+// any valid width certifies the same exact values).  kp: the key's padded norm.
+__device__ __forceinline__ void tile_ends(const RecShared &rs, const uint4 (&kb)[kRecD / 32], float kp, int l16, int g,
+                                          uint32_t (&pl)[8], uint32_t (&ph)[8]) {
+#pragma unroll
+  for (int m = 0; m < kRecH / 16; ++m) {
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < kRecD / 32; ++kk) acc = mfma16(rec_q(rs, 16 * m + l16, 4 * kk + g), kb[kk], acc);
+#pragma unroll
+    for (int rp = 0; rp < 2; ++rp) {
+      const int h0 = 16 * m + 4 * g + 2 * rp;
+      const float d0 = __builtin_fmaf(rs.qd[h0], kp, 0x1p-144f), d1 = __builtin_fmaf(rs.qd[h0 + 1], kp, 0x1p-144f);
+      pl[2 * m + rp] = cvt_relu_pk(acc[2 * rp] - d0, acc[2 * rp + 1] - d1);
+      ph[2 * m + rp] = cvt_relu_pk(acc[2 * rp] + d0, acc[2 * rp + 1] + d1);
+    }
+  }
+}
+
+// bf16 weights: the score itself is a bf16 value, so most near ties cannot change it.  Every operation of the canonical
+// sum rounds monotonically, so the sums over the ends that make each product smallest and largest enclose the score;
+// where both round to the same bf16 value, that is the score.  This pass writes those of the keys list[0 .. n) over their
+// slots and appends the other keys' positions to unc (count *n_unc, zero on entry); recompute_scores then takes only
+// these.  2 x 3001 queries over up to 750 keys (recomputed: nearly all of them): 275 us with every near tie computed exactly
+// in the tile, 250 us with open keys' only, 238 us with the open keys packed into tiles of their own, 232 us with the next
+// tile's keys in flight.
+template <int NW, bool F8>
+__device__ void certify_scores(int32_t *list, int n, const TopkRecompute &rc, const RecShared &rs, uint16_t *unc,
+                               uint32_t *n_unc, int64_t kbrow0, int64_t knrow0, float qpmax) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int ntile = (n + 15) / 16;
+  TileKeys<F8> next;
+  float next_kn = 0.f;
+  auto load = [&](int t) {
+    const int li = 16 * t + l16;
+    const int col = list[li < n ? li : n - 1];
+    next.load(rc, kbrow0 + col, g);
+    next_kn = rc.kn[knrow0 + col];
+  };
+  if (wave < ntile) load(wave);
+  for (int t = wave; t < ntile; t += NW) {
+    const int li = 16 * t + l16;
+    const bool kv = li < n;
+    uint4 kb[kRecD / 32];
+    next.fragments(kb);
+    const float kp = next_kn + 0x1p-122f;
+    if (t + NW < ntile) load(t + NW);  // in flight during this tile
+    uint32_t pl[8], ph[8];
+    tile_ends(rs, kb, kp, l16, g, pl, ph);
+    float lo = 0.f, hi = 0.f;
+#pragma unroll
+    for (int i = 0; i < kRecH / 8; ++i) {
+      const int h0 = 16 * (i >> 1) + 4 * g + 2 * (i & 1);
+      const uint32_t neg = *reinterpret_cast<const uint32_t *>(&rs.wneg[h0]);
+      head_sum<true>((pl[i] & ~neg) | (ph[i] & neg), rs.w[h0], rs.w[h0 + 1], lo);
+      head_sum<true>((ph[i] & ~neg) | (pl[i] & neg), rs.w[h0], rs.w[h0 + 1], hi);
+    }
+    lo = combine_groups(lo);
+    hi = combine_groups(hi);
+    const uint32_t r2 = cvt_pk_bf16(lo, hi);
+    // past the norm overflow guard the ends say nothing
+    const bool open = (r2 & 0xFFFFu) != (r2 >> 16) || !(qpmax * kp < 0x1p126f);
+    if (g == 0 && kv && !open) list[li] = static_cast<int32_t>(r2 << 16);
+    const uint64_t om = __builtin_amdgcn_ballot_w64(g == 0 && kv && open);
+    if (om != 0ull) {  // uniform
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(n_unc, static_cast<uint32_t>(__builtin_popcountll(om)));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if ((om >> lane) & 1ull) unc[base + __builtin_popcountll(om & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(li);
+    }
+  }
+}
+
+// Exact scores of n keys of one row (list[0 .. n), or list[sel[0 .. n)]), by the canonical contract, written over their
 // list slots (bit patterns of the scores).  Each wave takes tiles of 16 keys: four
 // 16-head MFMA rounds (heads 16m + 4g + r, m = 0..3) with the score kernel's interval test (same
 // half-widths: bound_c 2^-23 ||q_h|| times the key's norm) keep the relu'd lower ends of all
-// 64 heads; the tile's near-tie dots are then recomputed exactly, 16 at a time with a quad of lanes per dot
-// (q_h and the key row from LDS: exact_dot_bf16's arithmetic), and the fp32 fma head sum runs in the
+// 64 heads; the tile's near-tie dots are then recomputed exactly, with a pair of lanes per dot (8 lanes where a tile
+// has at most 8; q_h and the key row from LDS: exact_dot_bf16's arithmetic), and the head sum runs in the
 // canonical order over the corrected values.  F8: the key rows are e4m3 codes with row scales, dequantised in
 // registers to the contract's bf16 rows (q comes dequantised).
+// sel: the positions in list of the keys to take (bf16 weights: those that certify_scores left open), or null for all.
 template <int NW, bool F8, bool WBF>
-__device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
+__device__ void recompute_scores(int32_t *list, const uint16_t *sel, int n, const TopkRecompute &rc,
                                  const RecShared &rs, RecWave &rw, int64_t kbrow0, int64_t knrow0, float qpmax,
                                  uint32_t &n_exact, uint32_t &n_unres) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int ntile = (n + 15) / 16;
   for (int t = wave; t < ntile; t += NW) {
-    const int li = 16 * t + l16;
-    const bool kv = li < n;
-    const int col = list[kv ? li : n - 1];
-    const int64_t krow = kbrow0 + col;
+    const bool kv = 16 * t + l16 < n;
+    int li = kv ? 16 * t + l16 : n - 1;
+    if constexpr (WBF) li = sel[li];
+    const int col = list[li];
     // the tile's loads go out together (one round trip): key rows, key span and norm
-    uint4 kb[kRecD / 32];
-    uint2 kc8[F8 ? kRecD / 32 : 1];
-    float kscale = 0.f;
-    if constexpr (F8) {
-#pragma unroll
-      for (int kk = 0; kk < kRecD / 32; ++kk) kc8[kk] = *reinterpret_cast<const uint2 *>(rc.kc + krow * kRecD + 32 * kk + 8 * g);
-      kscale = rc.ks[krow];
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = *reinterpret_cast<const uint4 *>(rc.k + krow * kRecD + 32 * kk + 8 * g);
-    }
+    TileKeys<F8> raw;
+    raw.load(rc, kbrow0 + col, g);
     const int32_t ksv = rc.ksp[knrow0 + col];
     const float knm = rc.kn[knrow0 + col];
-    if constexpr (F8) {
-      if (__builtin_amdgcn_ballot_w64(!fp8_scale_pow2(kscale)) == 0ull) {
-#pragma unroll
-        for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = fp8_dequant8<true>(kc8[kk], kscale);
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < kRecD / 32; ++kk) kb[kk] = fp8_dequant8<false>(kc8[kk], kscale);
-      }
-    }
+    uint4 kb[kRecD / 32];
+    raw.fragments(kb);
 #pragma unroll
     for (int kk = 0; kk < kRecD / 32; ++kk) rw.k[l16 * kRecC + ((4 * kk + g) ^ l16)] = kb[kk];
     rw.ksp[l16] = ksv;  // the four lanes of a key write the same span; read by the near-tie dots below
-    uint32_t pl[8];     // relu'd lower ends, heads 16m + 4g + (0, 1) | (2, 3): pl[2m], pl[2m + 1]
-    uint32_t ntm = 0;   // bit 4m + r: head 16m + 4g + r is a near tie
-    // Interval half-widths: one fma per dot from the per-head factor qd (two roundings, within the three that
-    // the bound constant allows for evaluating the width, so the width still bounds the MFMA error; it need not
-    // equal the score kernel's, since any valid width certifies the same exact values).  When the query's
-    // largest padded norm times a key's reaches 2^126 (uniform over the wave, and rare), the MFMA may
+    rw.kn[l16] = knm;
+    // When the query's largest padded norm times a key's reaches 2^126 (uniform over the wave, and rare), the MFMA may
     // overflow: every dot of the tile is then taken as a near tie and computed exactly.
     const float kp = knm + 0x1p-122f;
     const bool overflow = __builtin_amdgcn_ballot_w64(!(qpmax * kp < 0x1p126f)) != 0ull;
+    uint32_t pl[8];    // relu'd lower ends, heads 16m + 4g + (0, 1) | (2, 3): pl[2m], pl[2m + 1]
+    uint32_t ntm = 0;  // bit 4m + r: head 16m + 4g + r is a near tie
+    {
+      uint32_t ph[8];
+      tile_ends(rs, kb, kp, l16, g, pl, ph);
 #pragma unroll
-    for (int m = 0; m < kRecH / 16; ++m) {
-      f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < kRecD / 32; ++kk) acc = mfma16(rec_q(rs, 16 * m + l16, 4 * kk + g), kb[kk], acc);
-#pragma unroll
-      for (int rp = 0; rp < 2; ++rp) {
-        const int h0 = 16 * m + 4 * g + 2 * rp;
-        const float d0 = __builtin_fmaf(rs.qd[h0], kp, 0x1p-144f), d1 = __builtin_fmaf(rs.qd[h0 + 1], kp, 0x1p-144f);
-        const uint32_t lo = cvt_relu_pk(acc[2 * rp] - d0, acc[2 * rp + 1] - d1);
-        const uint32_t hi = cvt_relu_pk(acc[2 * rp] + d0, acc[2 * rp + 1] + d1);
-        pl[2 * m + rp] = lo;
-        const uint32_t x = lo ^ hi;
-        ntm |= ((x & 0xFFFFu) != 0u && kv ? 1u : 0u) << (4 * m + 2 * rp);
-        ntm |= ((x >> 16) != 0u && kv ? 1u : 0u) << (4 * m + 2 * rp + 1);
+      for (int i = 0; i < kRecH / 8; ++i) {
+        const uint32_t x = pl[i] ^ ph[i];
+        ntm |= ((x & 0xFFFFu) != 0u && kv ? 1u : 0u) << (2 * i);
+        ntm |= ((x >> 16) != 0u && kv ? 1u : 0u) << (2 * i + 1);
       }
     }
     if (overflow) ntm = kv ? 0xFFFFu : 0u;
@@ -762,7 +864,6 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
       const uint32_t incl = wave_incl_scan(cnt);
       const int nd = static_cast<int>(__builtin_amdgcn_readlane(incl, 63));
       const int pos0 = static_cast<int>(incl - cnt);
-      const int dq = lane >> 1, sub = lane & 1;  // a pair of lanes per dot, 8 of the 16 chunks each
       for (int s0 = 0; s0 < nd; s0 += kNearCap) {  // list segments of kNearCap dots
         const int ns = nd - s0 < kNearCap ? nd - s0 : kNearCap;
         {
@@ -777,72 +878,83 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int b0 = 0; b0 < ns; b0 += 32) {
-          const int e = rw.ent[min(b0 + dq, ns - 1)];
-          const int sl = e >> 4, bit = e & 15;
-          const int h = 16 * (bit >> 2) + 4 * (sl >> 4) + (bit & 3), kl = sl & 15;
-          const int span = rs.qsp[h] + rw.ksp[kl];
-          const bool split = span > 52;
-          double hi = 0.0, lo = 0.0;
-          if (__builtin_amdgcn_ballot_w64(split) == 0ull) {
-            // four independent fma chains (every partial sum is exact when the span fits 52 bits)
-            double a[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-              const uint4 qv = rec_q(rs, h, 8 * sub + c);
-              const uint4 kv4 = rw.k[kl * kRecC + ((8 * sub + c) ^ kl)];
-              const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
-              const uint32_t kw[4] = {kv4.x, kv4.y, kv4.z, kv4.w};
-#pragma unroll
-              for (int p = 0; p < 4; ++p) {
-                a[p] = __builtin_fma(static_cast<double>(unpack_lo(qw[p])), static_cast<double>(unpack_lo(kw[p])), a[p]);
-                a[p] = __builtin_fma(static_cast<double>(unpack_hi(qw[p])), static_cast<double>(unpack_hi(kw[p])), a[p]);
+        // SUB lanes per dot, 16 / SUB of the 16 chunks each
+        auto exact_dots = [&](auto SUB) {
+          constexpr int kSub = decltype(SUB)::value, kCh = kRecC / kSub;
+          const int dq = lane / kSub, sub = lane % kSub;
+          for (int b0 = 0; b0 < ns; b0 += 64 / kSub) {
+            const int e = rw.ent[min(b0 + dq, ns - 1)];
+            const int sl = e >> 4, bit = e & 15;
+            const int h = 16 * (bit >> 2) + 4 * (sl >> 4) + (bit & 3), kl = sl & 15;
+            const int span = rs.qsp[h] + rw.ksp[kl];
+            const bool split = span > 52;
+            double hi = 0.0, lo = 0.0;
+            if (__builtin_amdgcn_ballot_w64(split) == 0ull) {
+              // four independent fma chains (every partial sum is exact when the span fits 52 bits)
+              double a[4] = {0.0, 0.0, 0.0, 0.0};
+  #pragma unroll
+              for (int c = 0; c < kCh; ++c) {
+                const uint4 qv = rec_q(rs, h, kCh * sub + c);
+                const uint4 kv4 = rw.k[kl * kRecC + ((kCh * sub + c) ^ kl)];
+                const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
+                const uint32_t kw[4] = {kv4.x, kv4.y, kv4.z, kv4.w};
+  #pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                  a[p] = __builtin_fma(static_cast<double>(unpack_lo(qw[p])), static_cast<double>(unpack_lo(kw[p])), a[p]);
+                  a[p] = __builtin_fma(static_cast<double>(unpack_hi(qw[p])), static_cast<double>(unpack_hi(kw[p])), a[p]);
+                }
+              }
+              hi = (a[0] + a[1]) + (a[2] + a[3]);
+            } else {
+              // wide dynamic range (rare): products above / below 2^(top - 38) accumulate separately
+              const double thr = split ? ldexp(1.0, frexp_exp(rs.qn[h]) + frexp_exp(rw.kn[kl]) - 38) : 0.0;
+  #pragma unroll 1
+              for (int c = 0; c < kCh; ++c) {
+                const uint4 qv = rec_q(rs, h, kCh * sub + c);
+                const uint4 kv4 = rw.k[kl * kRecC + ((kCh * sub + c) ^ kl)];
+                const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
+                const uint32_t kw[4] = {kv4.x, kv4.y, kv4.z, kv4.w};
+  #pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                  const double p0 = static_cast<double>(unpack_lo(qw[p])) * static_cast<double>(unpack_lo(kw[p]));
+                  const double p1 = static_cast<double>(unpack_hi(qw[p])) * static_cast<double>(unpack_hi(kw[p]));
+                  if (!split || fabs(p0) >= thr) hi += p0; else lo += p0;
+                  if (!split || fabs(p1) >= thr) hi += p1; else lo += p1;
+                }
               }
             }
-            hi = (a[0] + a[1]) + (a[2] + a[3]);
-          } else {
-            // wide dynamic range (rare): products above / below 2^(top - 38) accumulate separately
-            const int li2 = 16 * t + kl;
-            const int64_t kr2 = knrow0 + list[li2 < n ? li2 : n - 1];
-            const double thr = split ? ldexp(1.0, frexp_exp(rs.qn[h]) + frexp_exp(rc.kn[kr2]) - 38) : 0.0;
-#pragma unroll 1
-            for (int c = 0; c < 8; ++c) {
-              const uint4 qv = rec_q(rs, h, 8 * sub + c);
-              const uint4 kv4 = rw.k[kl * kRecC + ((8 * sub + c) ^ kl)];
-              const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
-              const uint32_t kw[4] = {kv4.x, kv4.y, kv4.z, kv4.w};
-#pragma unroll
-              for (int p = 0; p < 4; ++p) {
-                const double p0 = static_cast<double>(unpack_lo(qw[p])) * static_cast<double>(unpack_lo(kw[p]));
-                const double p1 = static_cast<double>(unpack_hi(qw[p])) * static_cast<double>(unpack_hi(kw[p]));
-                if (!split || fabs(p0) >= thr) hi += p0; else lo += p0;
-                if (!split || fabs(p1) >= thr) hi += p1; else lo += p1;
-              }
+            hi += dpp_f64<0xB1>(hi);  // the dot's parts: lanes l ^ 1 (quad_perm [1, 0, 3, 2]) ...
+            lo += dpp_f64<0xB1>(lo);
+            if constexpr (kSub == 8) {  // ... l ^ 2 (quad_perm [2, 3, 0, 1]), and 7 - l of the eight (row_half_mirror)
+              hi += dpp_f64<0x4E>(hi);
+              lo += dpp_f64<0x4E>(lo);
+              hi += dpp_f64<0x141>(hi);
+              lo += dpp_f64<0x141>(lo);
             }
+            uint16_t v;
+            if (!split && (hi == 0.0 || (fabs(hi) >= 0x1p-126 && fabs(hi) < 0x1p127))) v = round_to_bf16_fast(hi);
+            else v = round2_to_bf16(hi, lo);
+            // wider still (rare): the integer accumulator, any range, one dot at a time by the whole wave (its limbs
+            // in LDS, so the recomputation's register budget does not carry them)
+            uint64_t wide = __builtin_amdgcn_ballot_w64(span > 84 && sub == 0 && b0 + dq < ns);
+            while (wide) {  // uniform
+              const int wl = __builtin_ctzll(wide);
+              wide &= wide - 1;
+              const int wh = __builtin_amdgcn_readlane(h, wl), wk = __builtin_amdgcn_readlane(kl, wl);
+              const uint16_t r = wave_exact_dot_wide_bf16(
+                  [&](int j) { return reinterpret_cast<const uint32_t *>(&rs.q[wh * kRecC + ((j >> 2) ^ (wh & 15))])[j & 3]; },
+                  [&](int j) { return reinterpret_cast<const uint32_t *>(&rw.k[wk * kRecC + ((j >> 2) ^ wk)])[j & 3]; },
+                  rw.limb);
+              if (dq == wl / kSub) v = r;  // the lanes that own the dot
+              if (lane == wl) ++n_unres;   // counted: dots that needed the integer accumulator
+            }
+            const uint16_t rv = (v & 0x8000u) ? 0 : v;  // ReLU (also maps -0 to +0)
+            // a dot's lanes read only its own entry before this write (the value replaces the entry)
+            if (sub == 0 && b0 + dq < ns) rw.ent[b0 + dq] = rv;
           }
-          hi += dpp_f64<0xB1>(hi);  // the pair's two halves (quad_perm [1, 0, 3, 2])
-          lo += dpp_f64<0xB1>(lo);
-          uint16_t v;
-          if (!split && (hi == 0.0 || (fabs(hi) >= 0x1p-126 && fabs(hi) < 0x1p127))) v = round_to_bf16_fast(hi);
-          else v = round2_to_bf16(hi, lo);
-          // wider still (rare): the integer accumulator, any range, one dot at a time by the whole wave (its limbs
-          // in LDS, so the recomputation's register budget does not carry them)
-          uint64_t wide = __builtin_amdgcn_ballot_w64(span > 84 && sub == 0 && b0 + dq < ns);
-          while (wide) {  // uniform
-            const int wl = __builtin_ctzll(wide);
-            wide &= wide - 1;
-            const int wh = __builtin_amdgcn_readlane(h, wl), wk = __builtin_amdgcn_readlane(kl, wl);
-            const uint16_t r = wave_exact_dot_wide_bf16(
-                [&](int j) { return reinterpret_cast<const uint32_t *>(&rs.q[wh * kRecC + ((j >> 2) ^ (wh & 15))])[j & 3]; },
-                [&](int j) { return reinterpret_cast<const uint32_t *>(&rw.k[wk * kRecC + ((j >> 2) ^ wk)])[j & 3]; },
-                rw.limb);
-            if (dq == (wl >> 1)) v = r;  // the pair that owns the dot
-            if (lane == wl) ++n_unres;   // counted: dots that needed the integer accumulator
-          }
-          const uint16_t rv = (v & 0x8000u) ? 0 : v;  // ReLU (also maps -0 to +0)
-          // each pair reads only its own entry before this write (the value replaces the entry)
-          if (sub == 0 && b0 + dq < ns) rw.ent[b0 + dq] = rv;
-        }
+        };
+        if (ns <= 8) exact_dots(std::integral_constant<int, 8>{});
+        else exact_dots(std::integral_constant<int, 2>{});
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         uint32_t mm = ntm;
@@ -864,30 +976,114 @@ __device__ void recompute_scores(int32_t *list, int n, const TopkRecompute &rc,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
     }
-    // the canonical head sum: fma per head (fp32 weights), or the products of a pair rounded to bf16 together and added
-    // in head order, and the score rounded to bf16 (bf16 weights)
     float G = 0.f;
 #pragma unroll
-    for (int m = 0; m < kRecH / 16; ++m)
-#pragma unroll
-      for (int rp = 0; rp < 2; ++rp) {
-        const uint32_t p2 = pl[2 * m + rp];
-        const float w0 = rs.w[16 * m + 4 * g + 2 * rp], w1 = rs.w[16 * m + 4 * g + 2 * rp + 1];
-        if constexpr (WBF) {
-          const uint32_t pr = cvt_pk_bf16(unpack_lo(p2) * w0, unpack_hi(p2) * w1);
-          G = G + unpack_lo(pr);
-          G = G + unpack_hi(pr);
-        } else {
-          G = __builtin_fmaf(unpack_lo(p2), w0, G);
-          G = __builtin_fmaf(unpack_hi(p2), w1, G);
-        }
-      }
+    for (int i = 0; i < kRecH / 8; ++i) {
+      const int h0 = 16 * (i >> 1) + 4 * g + 2 * (i & 1);
+      head_sum<WBF>(pl[i], rs.w[h0], rs.w[h0 + 1], G);
+    }
     float tot = combine_groups(G);
     if constexpr (WBF) tot = unpack_lo(cvt_pk_bf16(tot, tot));
-    // the score replaces its column in the list too (read back from LDS when the batch is the last one):
-    // the tile's lanes read their list slots (and lanes past n read slot n - 1, of this same tile) before
+    // the score replaces its column: the tile's lanes read their list slots (and lanes past n the last one's, of this
+    // same tile) before
     if (g == 0 && kv) list[li] = __builtin_bit_cast(int32_t, tot);
   }
+}
+
+// Sorted store of the k_sel largest of the unique composites held in v (key 0: none; at most cap in all), whose keys
+// lie in [kmin, kmax], by ranks from a counting sort: 2048 buckets over [kmin, kmax] (RankScale: the bucket is a monotone
+// function of the key, so a higher bucket holds only larger composites); bucket starts from a block
+// scan from the top bucket; every entry is scattered into its bucket's range of tmp, and its rank is its bucket's
+// start plus the number of its bucket's entries above it.  Three barriers and O(n) work, against the log2(n)
+// dependent merge rounds of a sort.  Returns false, having stored nothing, when a bucket holds more than
+// kRankBucketMax entries (keys tied or clustered far beyond a smooth distribution); the caller then sorts.  Uses
+// cnt and start (kRankBuckets each), wsum and tmp[0, cap).
+constexpr int kRankBuckets = 2048;
+constexpr int kRankBucketMax = 256;
+// Uniform in the key (logarithmic in the score) over a positive range of at most eight octaves; otherwise uniform in the
+// score: a range that reaches down to zero or below it holds so many octaves of tiny magnitudes that uniform keys left
+// all large scores in a few buckets (12000 columns, k = 2048, where a third of the rows' k-th scores lie there:
+// the 128-row launch took 32.6 us, with this 7.7; 64 rows of 32768: 15.7 -> 7.7).
+struct RankScale {
+  uint32_t k0;
+  float v0, scale;
+  bool by_key;
+  __device__ __forceinline__ static float value(uint32_t key) {
+    return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
+  }
+  __device__ __forceinline__ RankScale(uint32_t kmin, uint32_t kmax) {
+    by_key = kmin >= 0x80000000u && kmax - kmin < (8u << 23);
+    // the ends as finite values (kmin may be below every value, kmax infinity)
+    const uint32_t lowest = 0x00800000u, highest = 0xFF7FFFFFu;  // keys of -/+ the largest finite value
+    k0 = kmin;
+    v0 = value(kmin < lowest ? lowest : kmin);
+    const float v1 = value(kmax > highest ? highest : kmax);
+    const float range = by_key ? static_cast<float>(kmax - kmin) + 1.0f : v1 - v0;
+    scale = range < 3e38f ? static_cast<float>(kRankBuckets) / fmaxf(range, 1e-30f) : 0.f;
+  }
+  __device__ __forceinline__ uint32_t bucket(uint32_t key) const {
+    const float d = (by_key ? static_cast<float>(key - k0) : value(key) - v0) * scale;
+    return d < static_cast<float>(kRankBuckets - 1) ? static_cast<uint32_t>(d > 0.f ? d : 0.f) : kRankBuckets - 1;
+  }
+};
+template <int PER, int NT = kTopkThreads>
+__device__ bool rank_store(const uint64_t (&v)[PER], uint32_t kmin, uint32_t kmax, int k_sel, int64_t row,
+                           int k, void *out, int out_i64, int causal, int64_t limit, int64_t offset, uint64_t *tmp,
+                           uint32_t *cnt, uint32_t *start, uint32_t *wsum) {
+  constexpr int kPer = kRankBuckets / NT;  // buckets per thread
+  const int tid = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) cnt[tid + i * NT] = 0u;
+  __syncthreads();
+  const RankScale rk(kmin, kmax);
+  uint32_t bk[PER], pos[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    bk[j] = 0u;
+    pos[j] = 0u;
+    if ((v[j] >> 32) != 0u) {
+      bk[j] = rk.bucket(static_cast<uint32_t>(v[j] >> 32));
+      pos[j] = atomicAdd(&cnt[bk[j]], 1u);  // the entry's place in its bucket (arrival order)
+    }
+  }
+  __syncthreads();
+  const int hi = kRankBuckets - 1 - kPer * tid;  // buckets hi, hi - 1, .., scanned from the top
+  uint32_t c[kPer], sum = 0, most = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    c[i] = cnt[hi - i];
+    sum += c[i];
+    most = c[i] > most ? c[i] : most;
+  }
+  uint32_t at = block_inclusive_scan<false, NT / 64>(sum, wsum) - sum;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    start[hi - i] = at;
+    at += c[i];
+  }
+  if (__syncthreads_or(most > kRankBucketMax)) return false;  // uniform
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if ((v[j] >> 32) != 0u) tmp[start[bk[j]] + pos[j]] = v[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if ((v[j] >> 32) != 0u) {
+      const uint32_t s0 = start[bk[j]], c = cnt[bk[j]];
+      uint32_t r = s0, e = 0;
+      // four members per step, read together (one LDS round trip per step, not per member)
+      for (; e + 4 <= c; e += 4) {
+        const uint64_t a0 = tmp[s0 + e], a1 = tmp[s0 + e + 1], a2 = tmp[s0 + e + 2], a3 = tmp[s0 + e + 3];
+        r += (a0 > v[j] ? 1u : 0u) + (a1 > v[j] ? 1u : 0u) + (a2 > v[j] ? 1u : 0u) + (a3 > v[j] ? 1u : 0u);
+      }
+      for (; e < c; ++e) r += tmp[s0 + e] > v[j] ? 1u : 0u;
+      if (r < static_cast<uint32_t>(k_sel)) {
+        const int64_t col = static_cast<int64_t>(~static_cast<uint32_t>(v[j] & 0xFFFFFFFFull));
+        store_index(out, out_i64, row * k + r, col, causal, limit, offset);
+      }
+    }
+  }
+  return true;
 }
 
 // Workgroup (row, slice): counts of the buckets (bound_digit, 2048) of the lower ends score - U of slice p's valid
@@ -942,10 +1138,21 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 //  - these columns fill the segment's list, in column-slot order: the exact key of each, or 0 where the exact score
 //    fell below tau; the segment's state receives the number of slots and an upper bound of the largest key (the
 //    largest upper end), the row's state tau.
-template <int KPB, bool F8, bool WBF>
+// MODE kRecOneSeg: rows of one segment (two columns per thread); the workgroup ranks its keys and stores the row's
+// indices itself, without lists (2 x 3001 rows of at most 750 columns, k 512: the rank launch of 1024 lanes a row took
+// 95 us; here the other workgroup's tiles fill the chain of barriers, and the two launches' 346 us became 238).
+// MODE kRecAll: the same without scores and bounds: every valid column is recomputed (topk_bounded_all; saves the 76 us of
+// the score launch at that shape).
+constexpr int kRecLists = 0, kRecOneSeg = 1, kRecAll = 2;
+struct RecOut {  // the output of the one-segment modes
+  void *out;
+  int64_t offset;
+  int out_i64;
+};
+template <int KPB, bool F8, bool WBF, int MODE>
 __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const float *scores, int64_t ld, int64_t S, int T,
                                                                     int k, int causal, int64_t start_pos, int ratio,
-                                                                    TopkRecompute rc, int segs, int NP,
+                                                                    TopkRecompute rc, RecOut ro, int segs, int NP,
                                                                     const uint32_t *__restrict__ hists,
                                                                     uint64_t *__restrict__ lists,
                                                                     uint2 *__restrict__ sstate,
@@ -955,7 +1162,8 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   __shared__ RecWave rw[kRecWaves];
   __shared__ int32_t list[SW];
   __shared__ uint32_t wsum[kRecWaves];
-  __shared__ uint32_t s_tau, s_max[kRecWaves];
+  __shared__ uint32_t s_tau, s_unc, s_max[kRecWaves];
+  __shared__ uint16_t unc[WBF ? SW : 2];  // list positions that certify_scores left open
   // the row's counts (NP = 0) share the LDS of the recomputation's scratch, which they precede
   static_assert(sizeof(RecWave) * kRecWaves >= 2048 * sizeof(uint32_t), "bucket counts fit");
   uint32_t *hist = reinterpret_cast<uint32_t *>(rw);
@@ -975,6 +1183,12 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   const int k_row = k < n_valid ? k : n_valid;
   const int c0 = seg * SW;
   const int nv = n_valid - c0 <= 0 ? 0 : (n_valid - c0 < SW ? n_valid - c0 : SW);
+  if constexpr (MODE != kRecLists) {
+    // masked tail: fewer valid columns than k (the -inf ties, in ascending column order)
+    const int64_t lim = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
+    for (int j = k_row + tid; j < k; j += kRecThreads)
+      store_index(ro.out, ro.out_i64, row * k + j, static_cast<int64_t>(n_valid) + (j - k_row), causal, lim, ro.offset);
+  }
   if (k_row == 0 || nv == 0) return;  // uniform, before any barrier: no valid column here
   const float *srow = scores + row * ld;
   const float *urow = rc.bounds + row * ld;
@@ -997,10 +1211,10 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
                        : static_cast<const float *>(rc.w)[qrow0 + hh];
   const float qnv = rc.qn[qrow0 + hh];
   const int32_t qsv = rc.qsp[qrow0 + hh];
-  const uint32_t mrow = rstate[row].y;
+  const uint32_t mrow = MODE == kRecAll ? 0u : rstate[row].y;
   float sv[KPB], uv[KPB];
 #pragma unroll
-  for (int j = 0; j < KPB; ++j) {
+  for (int j = 0; j < KPB && MODE != kRecAll; ++j) {
     const int col = j * kRecThreads + tid;
     sv[j] = srow[c0 + (col < nv ? col : 0)];
     uv[j] = urow[c0 + (col < nv ? col : 0)];
@@ -1022,104 +1236,117 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   rs.qn[hh] = qnv;
   rs.qd[hh] = rc.bound_c * 0x1p-23f * (qnv + 0x1p-122f);
   rs.qsp[hh] = qsv;
+  rs.wneg[hh] = __builtin_bit_cast(uint32_t, wv) >> 31 ? 0xFFFFu : 0u;
   // the query's largest padded head norm (lane h of every wave holds head h): decides per tile whether the
   // one-fma half-widths apply
   float qpmax = qnv + 0x1p-122f;
   qpmax = wave_max_f32(qpmax);
   qpmax = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int32_t, qpmax)));
 
-  // ---- tau: bucket e of the thread's kBPT is 2048 - kBPT (tid + 1) + e (the top one is e = kBPT - 1)
-  if (NP == 0) {  // uniform
-    reinterpret_cast<uint4 *>(hist)[tid] = make_uint4(0, 0, 0, 0);
-    __syncthreads();
-    // eight columns per thread at a time, their loads in flight together
-    for (int j0 = 0; j0 * kRecThreads < n_valid; j0 += 8) {
-      float sa[8], ua[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int col = (j0 + j) * kRecThreads + tid;
-        sa[j] = srow[col < n_valid ? col : 0];
-        ua[j] = urow[col < n_valid ? col : 0];
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if ((j0 + j) * kRecThreads + tid < n_valid) atomicAdd(&hist[bound_digit(sa[j] - ua[j], mrow)], 1u);
-    }
-    __syncthreads();
-    hv0 = *reinterpret_cast<const uint4 *>(hist + 2048 - kBPT * (tid + 1));
-  } else {
-    auto add = [&](uint4 h, bool in) {
-      hv0.x += in ? h.x : 0u;
-      hv0.y += in ? h.y : 0u;
-      hv0.z += in ? h.z : 0u;
-      hv0.w += in ? h.w : 0u;
-    };
-    add(hv1, NP > 1);
-    add(hv2, NP > 2);
-    add(hv3, NP > 3);
-  }
-  const uint32_t hc[kBPT] = {hv0.x, hv0.y, hv0.z, hv0.w};
-  uint32_t mine = 0;
-#pragma unroll
-  for (int e = 0; e < kBPT; ++e) mine += hc[e];
-  const uint32_t kr = static_cast<uint32_t>(k_row);
-  {
-    const uint32_t incl = block_inclusive_scan<true, kRecWaves>(mine, wsum);
-    const uint32_t excl = incl - mine;
-    if (excl < kr && incl >= kr) {  // exactly one thread: the row holds n_valid >= k_row nonzero lower ends
-      uint32_t acc = excl, bucket = 0;
-      bool found = false;
-#pragma unroll
-      for (int e = kBPT - 1; e >= 0; --e) {
-        acc += hc[e];
-        if (!found && acc >= kr) {
-          bucket = static_cast<uint32_t>(2048 - kBPT * (tid + 1) + e);
-          found = true;
-        }
-      }
-      s_tau = bound_digit_edge(bucket, mrow);
-    }
-  }
-  __syncthreads();
-  const uint32_t tau = s_tau;
-  if (seg == 0 && tid == 0) rstate[row].x = tau;
-
-  // ---- the segment's candidates: every column whose upper end reaches tau, with U > 0 (a score with U = 0 is exact
-  // already and takes its slot as it is); one block scan counts candidates (low 16 bits) and slots (high 16)
-  // (few registers stay live across the recomputation: the masks share one word, the bases another, and the
-  // largest upper end is taken from hik afterwards)
+  if (tid == 0) s_unc = 0u;
   uint32_t hik[KPB], masks = 0;  // bit j: column j is a candidate; bit 8 + j: it has a slot
-  static_assert(KPB <= 8, "masks of up to 8 columns per thread");
+  uint32_t tau = 1u, ncand = 0, nres = 0, bexcl = 0;
+  if constexpr (MODE == kRecAll) {
+    ncand = static_cast<uint32_t>(nv);
+    for (int i = tid; i < nv; i += kRecThreads) list[i] = i;
+  } else {
+    // ---- tau: bucket e of the thread's kBPT is 2048 - kBPT (tid + 1) + e (the top one is e = kBPT - 1)
+    if (NP == 0) {  // uniform
+      reinterpret_cast<uint4 *>(hist)[tid] = make_uint4(0, 0, 0, 0);
+      __syncthreads();
+      // eight columns per thread at a time, their loads in flight together
+      for (int j0 = 0; j0 * kRecThreads < n_valid; j0 += 8) {
+        float sa[8], ua[8];
 #pragma unroll
-  for (int j = 0; j < KPB; ++j) {
-    const bool v = j * kRecThreads + tid < nv;
-    const uint32_t lo = score_key(uv[j] > 0.f ? sv[j] - uv[j] : sv[j]);
-    hik[j] = v ? score_key(uv[j] > 0.f ? sv[j] + uv[j] : sv[j]) : 0u;
-    if (v && hik[j] >= tau) masks |= (lo != hik[j] ? 0x101u : 0x100u) << j;
-  }
-  static_assert(SW < 65536, "candidate and slot counts share a 32-bit scan");
-  const uint32_t both = __builtin_popcount(masks & 0xFFu) | (__builtin_popcount(masks >> 8) << 16);
-  const uint32_t bexcl = block_inclusive_scan<true, kRecWaves>(both, wsum) - both;  // slots << 16 | candidates
-  uint32_t ncand = 0, nres = 0;
+        for (int j = 0; j < 8; ++j) {
+          const int col = (j0 + j) * kRecThreads + tid;
+          sa[j] = srow[col < n_valid ? col : 0];
+          ua[j] = urow[col < n_valid ? col : 0];
+        }
 #pragma unroll
-  for (int w = 0; w < kRecWaves; ++w) {
-    ncand += wsum[w] & 0xFFFFu;
-    nres += wsum[w] >> 16;
-  }
-  {
-    uint32_t p = bexcl & 0xFFFFu;
+        for (int j = 0; j < 8; ++j)
+          if ((j0 + j) * kRecThreads + tid < n_valid) atomicAdd(&hist[bound_digit(sa[j] - ua[j], mrow)], 1u);
+      }
+      __syncthreads();
+      hv0 = *reinterpret_cast<const uint4 *>(hist + 2048 - kBPT * (tid + 1));
+    } else {
+      auto add = [&](uint4 h, bool in) {
+        hv0.x += in ? h.x : 0u;
+        hv0.y += in ? h.y : 0u;
+        hv0.z += in ? h.z : 0u;
+        hv0.w += in ? h.w : 0u;
+      };
+      add(hv1, NP > 1);
+      add(hv2, NP > 2);
+      add(hv3, NP > 3);
+    }
+    const uint32_t hc[kBPT] = {hv0.x, hv0.y, hv0.z, hv0.w};
+    uint32_t mine = 0;
 #pragma unroll
-    for (int j = 0; j < KPB; ++j)
-      if ((masks >> j) & 1u) list[p++] = c0 + j * kRecThreads + tid;
+    for (int e = 0; e < kBPT; ++e) mine += hc[e];
+    const uint32_t kr = static_cast<uint32_t>(k_row);
+    {
+      const uint32_t incl = block_inclusive_scan<true, kRecWaves>(mine, wsum);
+      const uint32_t excl = incl - mine;
+      if (excl < kr && incl >= kr) {  // exactly one thread: the row holds n_valid >= k_row nonzero lower ends
+        uint32_t acc = excl, bucket = 0;
+        bool found = false;
+#pragma unroll
+        for (int e = kBPT - 1; e >= 0; --e) {
+          acc += hc[e];
+          if (!found && acc >= kr) {
+            bucket = static_cast<uint32_t>(2048 - kBPT * (tid + 1) + e);
+            found = true;
+          }
+        }
+        s_tau = bound_digit_edge(bucket, mrow);
+      }
+    }
+    __syncthreads();
+    tau = s_tau;
+    if (MODE == kRecLists && seg == 0 && tid == 0) rstate[row].x = tau;
+
+    // ---- the segment's candidates: every column whose upper end reaches tau, with U > 0 (a score with U = 0 is exact
+    // already and takes its slot as it is); one block scan counts candidates (low 16 bits) and slots (high 16)
+    // (few registers stay live across the recomputation: the masks share one word, the bases another, and the
+    // largest upper end is taken from hik afterwards)
+    static_assert(KPB <= 8, "masks of up to 8 columns per thread");
+#pragma unroll
+    for (int j = 0; j < KPB; ++j) {
+      const bool v = j * kRecThreads + tid < nv;
+      const uint32_t lo = score_key(uv[j] > 0.f ? sv[j] - uv[j] : sv[j]);
+      hik[j] = v ? score_key(uv[j] > 0.f ? sv[j] + uv[j] : sv[j]) : 0u;
+      if (v && hik[j] >= tau) masks |= (lo != hik[j] ? 0x101u : 0x100u) << j;
+    }
+    static_assert(SW < 65536, "candidate and slot counts share a 32-bit scan");
+    const uint32_t both = __builtin_popcount(masks & 0xFFu) | (__builtin_popcount(masks >> 8) << 16);
+    bexcl = block_inclusive_scan<true, kRecWaves>(both, wsum) - both;  // slots << 16 | candidates
+#pragma unroll
+    for (int w = 0; w < kRecWaves; ++w) {
+      ncand += wsum[w] & 0xFFFFu;
+      nres += wsum[w] >> 16;
+    }
+    {
+      uint32_t p = bexcl & 0xFFFFu;
+#pragma unroll
+      for (int j = 0; j < KPB; ++j)
+        if ((masks >> j) & 1u) list[p++] = c0 + j * kRecThreads + tid;
+    }
   }
   __syncthreads();
   uint32_t n_exact = 0, n_unres = 0;
   if (ncand > 0) {
     const int64_t kbrow0 = b * rc.kbs;
-    recompute_scores<kRecWaves, F8, WBF>(list, static_cast<int>(ncand), rc, rs, rw[tid >> 6], kbrow0, b * rc.kns, qpmax,
-                                n_exact, n_unres);
+    int nrec = static_cast<int>(ncand);
+    if constexpr (WBF) {
+      certify_scores<kRecWaves, F8>(list, nrec, rc, rs, unc, &s_unc, kbrow0, b * rc.kns, qpmax);
+      __syncthreads();
+      nrec = static_cast<int>(s_unc);
+    }
+    recompute_scores<kRecWaves, F8, WBF>(list, unc, nrec, rc, rs, rw[tid >> 6], kbrow0, b * rc.kns, qpmax, n_exact,
+                                         n_unres);
   }
-  {
+  if constexpr (MODE == kRecLists) {
     uint32_t umax = 0, unused = 0;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) umax = ((masks >> (8 + j)) & 1u) && hik[j] > umax ? hik[j] : umax;
@@ -1128,7 +1355,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   }
   __syncthreads();  // every recomputed score is in its list slot
   const int64_t sg = row * segs + seg;
-  if (tid == 0) {
+  if (MODE == kRecLists && tid == 0) {
     uint32_t m = s_max[0];
 #pragma unroll
     for (int w = 1; w < kRecWaves; ++w) m = s_max[w] > m ? s_max[w] : m;
@@ -1140,109 +1367,68 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     if (rc.stats_ext && tid == 0 && ncand) atomicAdd(&rc.stats[2], ncand);
   }
 
-  // ---- the segment's slots: the exact key, or 0 where a recomputed score fell below tau
   const float *listf = reinterpret_cast<const float *>(list);
-  uint64_t *dst = lists + sg * SW;
-  uint32_t pos = bexcl >> 16, p = bexcl & 0xFFFFu;
+  if constexpr (MODE != kRecLists) {
+    // ---- ranks of the exact keys (at most two per thread) and the store
+    uint64_t v[KPB];
+    uint32_t p = bexcl & 0xFFFFu, kmax = 0, kmin = 0;  // kmin: complement of the smallest key
 #pragma unroll
-  for (int j = 0; j < KPB; ++j) {
-    if ((masks >> (8 + j)) & 1u) {
-      const bool cj = (masks >> j) & 1u;
-      uint32_t key = cj ? score_key(listf[p]) : hik[j];
-      p += cj ? 1u : 0u;
-      if (key < tau) key = 0u;
-      const uint32_t col = static_cast<uint32_t>(c0 + j * kRecThreads + tid);
-      dst[pos++] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
-    }
-  }
-}
-
-// Sorted store of the k_sel largest of the unique composites held in v (key 0: none; at most cap in all), whose keys
-// lie in [kmin, kmax], by ranks from a counting sort: 2048 buckets over [kmin, kmax] (RankScale: the bucket is a monotone
-// function of the key, so a higher bucket holds only larger composites); bucket starts from a block
-// scan from the top bucket; every entry is scattered into its bucket's range of tmp, and its rank is its bucket's
-// start plus the number of its bucket's entries above it.  Three barriers and O(n) work, against the log2(n)
-// dependent merge rounds of a sort.  Returns false, having stored nothing, when a bucket holds more than
-// kRankBucketMax entries (keys tied or clustered far beyond a smooth distribution); the caller then sorts.  Uses
-// sh.hist (counts, then starts), sh.wsum and tmp[0, cap).
-constexpr int kRankBuckets = 2048;
-constexpr int kRankBucketMax = 256;
-// Uniform in the key (logarithmic in the score) over a positive range of at most eight octaves; otherwise uniform in the
-// score: a range that reaches down to zero or below it holds so many octaves of tiny magnitudes that uniform keys left
-// all large scores in a few buckets (12000 columns, k = 2048, where a third of the rows' k-th scores lie there:
-// the 128-row launch took 32.6 us, with this 7.7; 64 rows of 32768: 15.7 -> 7.7).
-struct RankScale {
-  uint32_t k0;
-  float v0, scale;
-  bool by_key;
-  __device__ __forceinline__ static float value(uint32_t key) {
-    return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
-  }
-  __device__ __forceinline__ RankScale(uint32_t kmin, uint32_t kmax) {
-    by_key = kmin >= 0x80000000u && kmax - kmin < (8u << 23);
-    // the ends as finite values (kmin may be below every value, kmax infinity)
-    const uint32_t lowest = 0x00800000u, highest = 0xFF7FFFFFu;  // keys of -/+ the largest finite value
-    k0 = kmin;
-    v0 = value(kmin < lowest ? lowest : kmin);
-    const float v1 = value(kmax > highest ? highest : kmax);
-    const float range = by_key ? static_cast<float>(kmax - kmin) + 1.0f : v1 - v0;
-    scale = range < 3e38f ? static_cast<float>(kRankBuckets) / fmaxf(range, 1e-30f) : 0.f;
-  }
-  __device__ __forceinline__ uint32_t bucket(uint32_t key) const {
-    const float d = (by_key ? static_cast<float>(key - k0) : value(key) - v0) * scale;
-    return d < static_cast<float>(kRankBuckets - 1) ? static_cast<uint32_t>(d > 0.f ? d : 0.f) : kRankBuckets - 1;
-  }
-};
-template <int PER>
-__device__ bool rank_store(const uint64_t (&v)[PER], uint32_t kmin, uint32_t kmax, int k_sel, int64_t row,
-                           int k, void *out, int out_i64, int causal, int64_t limit, int64_t offset, uint64_t *tmp,
-                           SelShared &sh) {
-  static_assert(kRankBuckets == 2 * kTopkThreads, "two buckets per thread");
-  const int tid = threadIdx.x;
-  uint32_t *cnt = sh.hist[0], *start = sh.hist[1];
-  cnt[tid] = 0u;
-  cnt[tid + kTopkThreads] = 0u;
-  __syncthreads();
-  const RankScale rk(kmin, kmax);
-  uint32_t bk[PER], pos[PER];
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    bk[j] = 0u;
-    pos[j] = 0u;
-    if ((v[j] >> 32) != 0u) {
-      bk[j] = rk.bucket(static_cast<uint32_t>(v[j] >> 32));
-      pos[j] = atomicAdd(&cnt[bk[j]], 1u);  // the entry's place in its bucket (arrival order)
-    }
-  }
-  __syncthreads();
-  const int hi = kRankBuckets - 1 - 2 * tid;  // buckets hi and hi - 1, scanned from the top
-  const uint32_t c_hi = cnt[hi], c_lo = cnt[hi - 1];
-  const uint32_t excl = block_inclusive_scan<false>(c_hi + c_lo, sh.wsum) - (c_hi + c_lo);
-  start[hi] = excl;
-  start[hi - 1] = excl + c_hi;
-  if (__syncthreads_or(c_hi > kRankBucketMax || c_lo > kRankBucketMax)) return false;  // uniform
-#pragma unroll
-  for (int j = 0; j < PER; ++j)
-    if ((v[j] >> 32) != 0u) tmp[start[bk[j]] + pos[j]] = v[j];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    if ((v[j] >> 32) != 0u) {
-      const uint32_t s0 = start[bk[j]], c = cnt[bk[j]];
-      uint32_t r = s0, e = 0;
-      // four members per step, read together (one LDS round trip per step, not per member)
-      for (; e + 4 <= c; e += 4) {
-        const uint64_t a0 = tmp[s0 + e], a1 = tmp[s0 + e + 1], a2 = tmp[s0 + e + 2], a3 = tmp[s0 + e + 3];
-        r += (a0 > v[j] ? 1u : 0u) + (a1 > v[j] ? 1u : 0u) + (a2 > v[j] ? 1u : 0u) + (a3 > v[j] ? 1u : 0u);
+    for (int j = 0; j < KPB; ++j) {
+      const int col = j * kRecThreads + tid;
+      uint32_t key = 0u;
+      if constexpr (MODE == kRecAll) {
+        if (col < nv) key = score_key(listf[col]);
+      } else if ((masks >> (8 + j)) & 1u) {
+        const bool cj = (masks >> j) & 1u;
+        key = cj ? score_key(listf[p]) : hik[j];
+        p += cj ? 1u : 0u;
+        if (key < tau) key = 0u;
       }
-      for (; e < c; ++e) r += tmp[s0 + e] > v[j] ? 1u : 0u;
-      if (r < static_cast<uint32_t>(k_sel)) {
-        const int64_t col = static_cast<int64_t>(~static_cast<uint32_t>(v[j] & 0xFFFFFFFFull));
-        store_index(out, out_i64, row * k + r, col, causal, limit, offset);
+      v[j] = key == 0u ? 0ull : (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~static_cast<uint32_t>(col));
+      kmax = key > kmax ? key : kmax;
+      if (key != 0u) kmin = ~key > kmin ? ~key : kmin;
+    }
+    wave_max2(kmin, kmax);
+    if ((tid & 63) == 0) {
+      s_max[tid >> 6] = kmax;
+      wsum[tid >> 6] = kmin;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kRecWaves; ++w) {
+      kmax = s_max[w] > kmax ? s_max[w] : kmax;
+      kmin = wsum[w] > kmin ? wsum[w] : kmin;
+    }
+    // the waves' scratch of the recomputation is free: buckets, starts and the composites (twice, for the sort)
+    constexpr int kCap = KPB * kRecThreads;
+    static_assert(sizeof(RecWave) * kRecWaves >= 2 * kRankBuckets * sizeof(uint32_t) + 2 * kCap * sizeof(uint64_t), "rank scratch");
+    uint32_t *cnt = reinterpret_cast<uint32_t *>(rw), *start = cnt + kRankBuckets;
+    uint64_t *cand = reinterpret_cast<uint64_t *>(start + kRankBuckets);
+    const int64_t lim = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
+    if (!rank_store<KPB, kRecThreads>(v, ~kmin, kmax, k_row, row, k, ro.out, ro.out_i64, causal, lim, ro.offset, cand, cnt,
+                                      start, wsum)) {
+      // clustered keys: a merge sort over the columns' slots (absent: 0)
+#pragma unroll
+      for (int j = 0; j < KPB; ++j) cand[j * kRecThreads + tid] = v[j];
+      __syncthreads();
+      sort_merge_store<kRecThreads>(cand, kCap, kCap, k_row, row, k, ro.out, ro.out_i64, causal, lim, ro.offset, nullptr);
+    }
+  } else {
+    // ---- the segment's slots: the exact key, or 0 where a recomputed score fell below tau
+    uint64_t *dst = lists + sg * SW;
+    uint32_t pos = bexcl >> 16, p = bexcl & 0xFFFFu;
+#pragma unroll
+    for (int j = 0; j < KPB; ++j) {
+      if ((masks >> (8 + j)) & 1u) {
+        const bool cj = (masks >> j) & 1u;
+        uint32_t key = cj ? score_key(listf[p]) : hik[j];
+        p += cj ? 1u : 0u;
+        if (key < tau) key = 0u;
+        const uint32_t col = static_cast<uint32_t>(c0 + j * kRecThreads + tid);
+        dst[pos++] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
       }
     }
   }
-  return true;
 }
 
 // One workgroup per row: the lists of the row's segments (together every column of its top k, each with its exact score;
@@ -1317,7 +1503,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
           v[j] = i < n ? cand[i] : 0;
         }
       }
-      if (!rank_store<kMaxPer>(v, tau, top, k_sel, row, k, out, out_i64, causal, limit, offset, cand, sh)) {
+      if (!rank_store<kMaxPer>(v, tau, top, k_sel, row, k, out, out_i64, causal, limit, offset, cand,
+                               sh.hist[0], sh.hist[1], sh.wsum)) {
         gather();
         int P = 128;
         while (P < static_cast<int>(n)) P <<= 1;
@@ -1437,16 +1624,21 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   }
   const dim3 rgrid(static_cast<unsigned>(rows * segs));
   const bool f8 = rc.kc != nullptr;
+  const bool one = kpb == 2 && segs == 1, all = scores == nullptr;
+  KS_CHECK_ARG(!all || one, "indexer top-k (bounded): scores are needed past %d columns", 2 * kRecThreads);
   KS_CHECK_ARG(f8 == (rc.ks != nullptr), "indexer top-k (bounded): FP8 keys need codes and scales");
+  const RecOut ro{out, offset, o};
   auto rec = [&](auto kern) {
-    hipLaunchKernelGGL(kern, rgrid, dim3(kRecThreads), 0, st, scores, ld, S, Ti, ki, c, start_pos, ratio, rc, segs, NP,
+    hipLaunchKernelGGL(kern, rgrid, dim3(kRecThreads), 0, st, scores, ld, S, Ti, ki, c, start_pos, ratio, rc, ro, segs, NP,
                        rg.hists, rg.lists, rg.sstate, rg.rstate);
   };
   auto rec_k = [&](auto F8, auto WBF) {
     constexpr bool f = decltype(F8)::value, wb = decltype(WBF)::value;
-    if (kpb == 2) rec(topk_recompute_kernel<2, f, wb>);
-    else if (kpb == 4) rec(topk_recompute_kernel<4, f, wb>);
-    else rec(topk_recompute_kernel<8, f, wb>);
+    if (all) rec(topk_recompute_kernel<2, f, wb, kRecAll>);
+    else if (one) rec(topk_recompute_kernel<2, f, wb, kRecOneSeg>);
+    else if (kpb == 2) rec(topk_recompute_kernel<2, f, wb, kRecLists>);
+    else if (kpb == 4) rec(topk_recompute_kernel<4, f, wb, kRecLists>);
+    else rec(topk_recompute_kernel<8, f, wb, kRecLists>);
   };
   const std::true_type yes;
   const std::false_type no;
@@ -1455,6 +1647,7 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   else if (rc.w_bf16) rec_k(no, yes);
   else rec_k(no, no);
   KS_CHECK_LAUNCH("topk_recompute_kernel");
+  if (one) return KS_OK;
   const size_t shmem = static_cast<size_t>(2 * cap) * sizeof(uint64_t);
   // threads per segment's list: 1024 over the power of two >= segs (at most 32: T <= 32768, 1024 columns or more each)
   int tpl = 10;
@@ -1477,6 +1670,23 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
 #undef KS_COLL
   KS_CHECK_LAUNCH("topk_collected_kernel");
   return KS_OK;
+}
+
+bool ks::topk_bounded_all(int64_t S, int64_t T, int64_t k, int causal, int64_t start_pos, int ratio) {
+  if (T > 2 * kRecThreads) return false;
+  // live columns and selected ones, over at most 64 queries spread over the batch
+  // A recomputed score costs about ten approximate ones, and the bounds let a tenth to a quarter of the columns past the
+  // k-th through: from three quarters selected, the approximate pass costs more than it spares.
+  int64_t live = 0, sel = 0;
+  const int64_t n = S < 64 ? S : 64;
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t s = i * S / n;
+    const int64_t lim = causal ? (start_pos + s + 1) / ratio : T;
+    const int64_t v = lim < T ? lim : T;
+    live += v;
+    sel += v < k ? v : k;
+  }
+  return 4 * sel >= 3 * live;
 }
 
 uint32_t *ks::topk_bounded_state(uint64_t *part, int64_t rows, int64_t T) {

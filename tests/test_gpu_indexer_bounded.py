@@ -102,3 +102,39 @@ def test_equal_keys_and_tiny_weights(device, wbf):
     _check(device, q, k, w.bfloat16() if wbf else w, 600, False, 0)
     k = torch.randn(1, 1500, 128, generator=g).bfloat16()
     _check(device, q, k, w.bfloat16() if wbf else w, 600, False, 0)
+
+
+# rows of one segment (at most 1024 keys), ranked by the recomputation: with every column recomputed (k near the row's
+# length, causal prompts) and with a threshold; edges of the two columns per thread, tiles of 16, rows without a live key
+@pytest.mark.parametrize("wbf", [False, True])
+@pytest.mark.parametrize("B,S,T,k_top,causal,start,ratio", [
+    (1, 6, 1, 1, False, 0, 1), (1, 7, 17, 16, False, 0, 1), (2, 40, 33, 12, True, 0, 1), (1, 9, 512, 512, False, 0, 1),
+    (1, 9, 513, 40, False, 0, 1), (1, 6, 1023, 1000, False, 0, 1), (1, 6, 1024, 100, False, 0, 1),
+    (1, 6, 1025, 1000, False, 0, 1), (1, 70, 600, 512, True, 531, 1), (1, 300, 75, 64, True, 0, 4)])
+def test_one_segment_rows(device, wbf, B, S, T, k_top, causal, start, ratio):
+    g = torch.Generator().manual_seed(B + S * T + k_top)
+    q = torch.randn(B, S, 64, 128, generator=g).bfloat16()
+    k = torch.randn(B, T, 128, generator=g).bfloat16()
+    w = torch.randn(B, S, 64, generator=g) / 8
+    w[:, ::3, ::5] = 0.0
+    print(f"[case] one segment B={B} S={S} T={T} k={k_top} causal={causal} start={start} bf16={wbf}", flush=True)
+    _check(device, q, k, w.bfloat16() if wbf else w, k_top, causal, start, ratio, offset=3)
+
+
+@pytest.mark.parametrize("wbf", [False, True])
+@pytest.mark.parametrize("k_top", [90, 600])
+def test_one_segment_rows_ties_and_range(device, wbf, k_top):
+    g = torch.Generator().manual_seed(k_top)
+    w = torch.randn(1, 5, 64, generator=g) * 0.05
+    w[0, 1] = 0.0                                          # every score zero: the columns decide (and the merge sort)
+    q = torch.randn(1, 5, 64, 128, generator=g)
+    k = torch.randn(1, 700, 128, generator=g)
+    k[0, 300:] = k[0, :1]                                  # 400 equal keys
+    print(f"[case] one segment, ties, k={k_top} bf16={wbf}", flush=True)
+    _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, k_top, False, 0)
+    # integers: dots on bf16 midpoints; norms past the overflow guard: no end certifies a score
+    q, k = torch.randint(-4, 5, q.shape, generator=g).float(), torch.randint(-4, 5, k.shape, generator=g).float()
+    print(f"[case] one segment, midpoints, k={k_top} bf16={wbf}", flush=True)
+    _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, k_top, False, 0)
+    print(f"[case] one segment, overflow guard, k={k_top} bf16={wbf}", flush=True)
+    _check(device, (q * 2.0 ** 59).bfloat16(), (k * 2.0 ** 59).bfloat16(), w.bfloat16() if wbf else w, k_top, False, 0)
