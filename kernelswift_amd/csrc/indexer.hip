@@ -92,18 +92,20 @@ bool takes_bounded(int64_t k_top, int64_t H, int64_t D, int64_t T, int path) {
   return H == 64 && D == 128 && T <= 32768 && kk <= 2048 && path != 1;
 }
 
-// FP8 keys read directly by the bounded kernels (codes and row scales at batch stride kbs), or none.
-struct Fp8Direct {
+// Keys that the bounded kernels read directly from the caller's rows at batch stride kbs: FP8 codes with their row scales,
+// or bf16 rows that take no rotation; or none (the prepared rows).
+struct DirectKeys {
   const uint8_t *kc = nullptr;
   const float *ks = nullptr;
+  const uint16_t *k = nullptr;
   int64_t kbs = 0;
 };
 
-// Scores of the prepared rows (ws.q_rot / ws.k_rot with their statistics, or the FP8 rows of f8) -> exact top-k.
+// Scores of the prepared rows (ws.q_rot / ws.k_rot with their statistics, or the keys of dk) -> exact top-k.
 int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w_bf16, int64_t k_top, int32_t causal,
                    int64_t start_pos, int32_t ratio, int64_t offset, void *out, int32_t out_i64, int64_t B, int64_t S,
                    int64_t H, int64_t D, int64_t T, hipStream_t st, float bound_c, uint32_t *stats, int path,
-                   const Fp8Direct &f8 = Fp8Direct{}, const uint16_t *q_unrot = nullptr, int rot_lo = 0,
+                   const DirectKeys &dk = DirectKeys{}, const uint16_t *q_unrot = nullptr, int rot_lo = 0,
                    int rot_hi = 0) {
   const int64_t kk = k_top < T ? k_top : T;
   const bool can_bound = takes_bounded(k_top, H, D, T, 0);
@@ -111,22 +113,21 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
                "%s: the bounded path needs H = 64, D = 128, T <= 32768 and k <= 2048", fn);
   int rc;
   if (can_bound && path != 1) {
-    const bool direct = f8.kc != nullptr;
-    // FP8 keys: the codes with their row scales (the statistics are indexed like the rows: B == 1 or kbs == T)
-    const uint16_t *krows = direct ? reinterpret_cast<const uint16_t *>(f8.kc) : ws.k_rot;
-    const int64_t kbs = direct ? f8.kbs : T;
+    const bool direct = dk.kc != nullptr || dk.k != nullptr;
+    const uint16_t *krows = dk.kc != nullptr ? reinterpret_cast<const uint16_t *>(dk.kc) : direct ? dk.k : ws.k_rot;
+    const int64_t kbs = direct ? dk.kbs : T;
     const bool all = ks::topk_bounded_all(S, T, kk, causal ? 1 : 0, start_pos, ratio);
     if (!all) {
       rc = ks::launch_indexer_scores(ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm, ws.q_span, ws.k_norm, ws.k_span,
                                      ws.scores, B, S, H, D, T, kbs, causal ? 1 : 0, start_pos, ratio, bound_c, nullptr, st,
-                                     ws.bounds, ks::topk_bounded_state(ws.part, B * S, T), f8.ks, nullptr, T);
+                                     ws.bounds, ks::topk_bounded_state(ws.part, B * S, T), dk.ks, nullptr, T);
       if (rc != KS_OK) return rc;
     }
     ks::TopkRecompute trc{ws.bounds, ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm,
                           ws.q_span, ws.k_norm, ws.k_span, kbs, T, bound_c, stats, path == 3 ? 1 : 0, ws.part,
                           ws.part_cap};
-    trc.kc = f8.kc;
-    trc.ks = f8.ks;
+    trc.kc = dk.kc;
+    trc.ks = dk.ks;
     return ks::launch_indexer_topk_bounded(all ? nullptr : ws.scores, T, B, S, T, kk, causal ? 1 : 0, start_pos, ratio, offset, out,
                                            out_i64 ? 1 : 0, trc, st);
   }
@@ -175,7 +176,14 @@ int indexer_impl(const uint16_t *q, const uint16_t *k, const void *w, int32_t w_
   const bool split = !bounded && rope_start % 32 == 0 && rd % 32 == 0;
   ks::RowJob qjob{q, ws.q_rot, ws.q_norm, ws.q_span, B * S * H, B * S * H, B * S * H, H, S, start_pos, rd};
   qjob.rotated_only = split ? 1 : 0;
-  const ks::RowJob kjob{k, ws.k_rot, ws.k_norm, ws.k_span, B * T, T, k_batch_stride, 1, T, 0, rope_k ? rd : 0};
+  // keys that take no rotation are read where they are by the bounded kernels; this pass then forms their statistics only
+  // (a layer generating one token for each of 16 caches of 16382 keys: the call 92.2 -> 75.2 us)
+  DirectKeys dk;
+  if (bounded && !(rope_k && rd > 0)) {
+    dk.k = k;
+    dk.kbs = k_batch_stride;
+  }
+  const ks::RowJob kjob{k, dk.k != nullptr ? nullptr : ws.k_rot, ws.k_norm, ws.k_span, B * T, T, k_batch_stride, 1, T, 0, rope_k ? rd : 0};
   // w_scale != 1: the row preparation also writes the scaled weights (one per q row), which the later launches read
   const bool scaled = w_scale != 1.0f;
   const ks::WeightScale wsc{w, ws.w_scaled, w_scale, w_bf16 ? 1 : 0};
@@ -183,7 +191,7 @@ int indexer_impl(const uint16_t *q, const uint16_t *k, const void *w, int32_t w_
                             scaled ? &wsc : nullptr);
   if (rc != KS_OK) return rc;
   return indexer_select("ks_indexer", ws, scaled ? ws.w_scaled : w, w_bf16, k_top, causal, start_pos, ratio, offset,
-                        out, out_i64, B, S, H, D, T, st, bound_c, stats, path, Fp8Direct{}, split ? q : nullptr,
+                        out, out_i64, B, S, H, D, T, st, bound_c, stats, path, dk, split ? q : nullptr,
                         static_cast<int>(rope_start), static_cast<int>(rope_start) + rd);
 }
 
@@ -214,14 +222,14 @@ int indexer_fp8_impl(const uint8_t *q, const float *q_scale, const uint8_t *k, c
   const ks::Fp8RowJob kjob{k, k_scale, direct ? nullptr : ws.k_rot, ws.k_norm, ws.k_span, B * T, T, k_batch_stride};
   rc = ks::launch_fp8_rows(qjob, kjob, static_cast<int>(D), st);
   if (rc != KS_OK) return rc;
-  Fp8Direct f8;
+  DirectKeys dk;
   if (direct) {
-    f8.kc = k;
-    f8.ks = k_scale;
-    f8.kbs = k_batch_stride;
+    dk.kc = k;
+    dk.ks = k_scale;
+    dk.kbs = k_batch_stride;
   }
   return indexer_select("ks_indexer_fp8", ws, w, w_bf16, k_top, causal, start_pos, ratio, offset, out, out_i64, B, S,
-                        H, D, T, st, bound_c, stats, path, f8);
+                        H, D, T, st, bound_c, stats, path, dk);
 }
 }  // namespace
 
