@@ -481,7 +481,7 @@ __global__ __launch_bounds__((SaShape<DQK, DV, GW>::THREADS)) void sparse_attn_k
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// MLA-shaped heads (Dqk = 576, Dv = 512, H = 32 NW): one work item per workgroup of NW waves, 32 heads per
+// MLA-shaped heads (Dqk = 576, Dv = 512, H = 32 NW, NW = 3 or 4; 32 and 64 heads: sparse_attn_mla_kernel_cols): one work item per workgroup of NW waves, 32 heads per
 // wave (two 16-head tiles), one wave per SIMD.  Each K fragment and each V fragment read from LDS feeds two
 // MFMAs (one per head tile), which halves the LDS read traffic per flop of a 16-head wave, and a wave
 // alone on its SIMD has 512 registers: the 16 x 512 fp32 O accumulators of both tiles (256) and the q
@@ -677,22 +677,18 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
   const uint32_t kb_lds = __builtin_amdgcn_readfirstlane(lds_addr(&kb[0][0]));
   auto issue = [&](int c) {
     const int buf = c % NBUF;
-    // one-wave workgroups (36 gathers) redo the slot arithmetic per chunk (opaque lane): kept live across
-    // the loop, their per-gather offsets would take 72 registers
-    int ln = lane;
-    if constexpr (NW == 1) asm volatile("" : "+v"(ln));
-    // index reads in batches of a divisor of NJ (36, 18, 12, 9): one LDS latency per batch
+    // index reads together: one LDS latency
     constexpr int BATCH = NJ <= 12 ? NJ : 9;
     static_assert(NJ % BATCH == 0, "every batch lies inside the wave's NJ gathers");
 #pragma unroll
     for (int i0 = 0; i0 < NJ; i0 += BATCH) {
       int32_t r[BATCH];
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) r[i] = sidx[c * kKC + (64 * (wave + NW * (i0 + i)) + ln) / UPR];
+      for (int i = 0; i < BATCH; ++i) r[i] = sidx[c * kKC + (64 * (wave + NW * (i0 + i)) + lane) / UPR];
 #pragma unroll
       for (int i = 0; i < BATCH; ++i) {
         const int jj = wave + NW * (i0 + i);
-        const int sl = 64 * jj + ln;
+        const int sl = 64 * jj + lane;
         const int key = sl / UPR;
         const uint32_t voff =
             static_cast<uint32_t>(r[i] < 0 ? 0 : r[i]) * (Sh::DQK * 2) + ((sl % UPR) ^ (key & 7)) * 16;
@@ -715,7 +711,8 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
     for (int p = 0; p < 4; ++p) pv_off[t][p] = Sh::slot(kv_key, 0, 2 * p + ((l16 & 3) >> 1)) * 8 + 4 * (l16 & 1);
   }
 
-  float m_ref[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};  // per head (lane l16), replicated over g
+  // per head (lane l16): the reference max, replicated over g, and the lane's own keys' part of the sum
+  float m_ref[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
   f32x4_t o[2][CT];
 #pragma unroll
   for (int ht = 0; ht < 2; ++ht)
@@ -751,18 +748,29 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
       }
     }
     mfma_vgpr_leave(st);
-    // ---- online softmax per head tile (lane: head l16, keys 16t + 4g + r)
-    const uint32_t vbits = vm >> (4 * g);
-    float cmax[2];
+    // ---- online softmax per head tile (lane: head l16, keys 16t + 4g + r).  A wave alone on its SIMD cannot hide its VALU
+    // work: whole chunks skip the key masks, and the lanes' sums meet once, after the loop (512 queries, K 2048, N 8192:
+    // 314 -> 304 us; 256 queries' worth of K 512: 107 -> 103).
 #pragma unroll
-    for (int ht = 0; ht < 2; ++ht) {
-      float mx = -INFINITY;
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ht = 0; ht < 2; ++ht) st[t][ht] *= scale_log2;
+    if (vm != 0xFFFFFFFFu) {  // uniform: most chunks are whole
+      const uint32_t vbits = vm >> (4 * g);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if ((vbits >> (16 * t + r)) & 1u) mx = fmaxf(mx, st[t][ht][r] * scale_log2);
-      cmax[ht] = rows_max(mx);
+        for (int r = 0; r < 4; ++r) {
+          const bool ok = (vbits >> (16 * t + r)) & 1u;
+          st[t][0][r] = ok ? st[t][0][r] : -INFINITY;
+          st[t][1][r] = ok ? st[t][1][r] : -INFINITY;
+        }
+    }
+    float cmax[2];
+#pragma unroll
+    for (int ht = 0; ht < 2; ++ht) {
+      const f32x4_t a = st[0][ht], b = st[1][ht];
+      cmax[ht] = rows_max(fmaxf(fmaxf(fmaxf(fmaxf(a[0], a[1]), a[2]), a[3]), fmaxf(fmaxf(fmaxf(b[0], b[1]), b[2]), b[3])));
     }
     const bool need0 = cmax[0] > m_ref[0] + kRescaleTau, need1 = cmax[1] > m_ref[1] + kRescaleTau;
     if (__builtin_amdgcn_ballot_w64(need0 || need1) != 0ull) {
@@ -789,15 +797,11 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
     uint4 pa[2];
 #pragma unroll
     for (int ht = 0; ht < 2; ++ht) {
-      float p[8], csum = 0.f;
+      float p[8];
+      const float mu = m_ref[ht] == -INFINITY ? 0.f : m_ref[ht];  // masked keys: exp2(-inf - 0) while no key was valid
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const bool ok = (vbits >> (16 * (i >> 2) + (i & 3))) & 1u;
-        p[i] = ok ? fast_exp2(st[i >> 2][ht][i & 3] * scale_log2 - m_ref[ht]) : 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) csum += p[i];
-      l_run[ht] += rows_sum(csum);
+      for (int i = 0; i < 8; ++i) p[i] = fast_exp2(st[i >> 2][ht][i & 3] - mu);
+      l_run[ht] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       pa[ht] = make_uint4(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
                           pack_bf16x2(p[6], p[7]));
     }
@@ -815,6 +819,8 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
     mfma_agpr_settle(o);
   }
   mfma_agpr_leave(o);
+#pragma unroll
+  for (int ht = 0; ht < 2; ++ht) l_run[ht] = rows_sum(l_run[ht]);
 
   // ---- finalise (one range per query: sink added, bf16 output) or write the partial range
   const int64_t obase = NS == 1 ? qm : item;
@@ -865,6 +871,250 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
       float *pml = part_ml + (item * H + 32 * wave + 16 * ht + l16) * 2;
       pml[0] = m_ref[ht];
       pml[1] = l_run[ht];
+    }
+  }
+}
+
+// 32 or 64 heads (NHT = 2 or 4 head tiles of 16): with 32 heads per wave, as above, one or two of a CU's four SIMDs would
+// work.  Here an item's 2 NHT waves split both products: for the scores a wave takes one head tile and one of the chunk's
+// two key tiles (q of one tile: 72 registers, none in LDS), for P V it takes 32 / (2 NHT) column tiles of all heads (64
+// accumulator registers), so that V is read from LDS once per chunk and not once per 32 heads.  The probabilities cross in
+// LDS, already in the layout of the PV A-fragment: lane (l16, g) of key tile t writes its four to half t of the lane's 16
+// bytes.  All waves share each head's lazily moved reference max; a wave whose chunk maximum passes it by the threshold
+// raises a flag, and after the barrier that publishes P every wave takes the (rare) path that moves the references,
+// rescales and forms P again.  Two barriers per chunk; gather ring, staged indices, partials and their combine as above.
+// 512 queries of 32 heads, K 2048, N 8192: 577 -> 168 us; 256 queries of 64 heads: 162 -> 106 us.  (96 heads' column tiles
+// do not divide by its waves; 128 heads would need 16 waves of 128 registers.)
+template <int NHT>
+__global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
+    const uint16_t *__restrict__ q, const uint16_t *__restrict__ kv, const float *__restrict__ sink,
+    const int32_t *__restrict__ idx, uint16_t *__restrict__ out, uint16_t *__restrict__ part_o,
+    float *__restrict__ part_ml, int64_t M, int64_t N, int64_t K, int NS, int KR, float scale_log2) {
+  constexpr int NW = 2 * NHT, NBUF = 3, THREADS = 64 * NW, H = 16 * NHT;
+  using Sh = MlaShape<4, NBUF>;  // the chunk's geometry
+  constexpr int QJ = Sh::QJ, UPR = Sh::UPR, TI = Sh::TI;
+  constexpr int CTW = Sh::CT / NW;            // column tiles per wave
+  constexpr int NJ = (TI + NW - 1) / NW;      // DMA instructions per wave and chunk, at most
+  static_assert(CTW % 4 == 0, "a wave's first column tile has the four swizzle patterns in order");
+  __shared__ __attribute__((aligned(16))) uint16_t kb[NBUF][Sh::BUF];
+  __shared__ __attribute__((aligned(16))) uint2 pb[NHT][64][2];
+  __shared__ int32_t sidx[Sh::KR_MAX];
+  __shared__ float sx[2][H];      // per key tile and head: chunk maxima (moving references), at the end the sums
+  __shared__ uint32_t moved[2];   // chunk parity: some reference has to move
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int ht = wave >> 1, kt = wave & 1;  // the wave's score tile
+  const int64_t nblk = gridDim.x;
+  const int64_t item = (nblk % 8 == 0) ? (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int64_t qm = item / NS;
+  const int split = static_cast<int>(item % NS);
+  const int64_t b = qm / M;
+  const int k_begin = split * KR;
+  const int k_end = k_begin + KR < K ? k_begin + KR : static_cast<int>(K);
+  const int nch = (k_end - k_begin + kKC - 1) / kKC;  // >= 1: every range of the plan is non-empty
+  const global_ptr<const uint16_t> kvb = uniform_ptr(kv + b * N * Sh::DQK);
+
+  // the item's indices and the wave's q rows are loaded together (one round trip), as above
+  constexpr int kIPT = Sh::KR_MAX / THREADS;
+  const int ntot = nch * kKC;  // <= KR_MAX (host-checked range length, rounded up to whole chunks)
+  int32_t iraw[kIPT];
+  {
+    const int32_t *irow = idx + qm * K;
+#pragma unroll
+    for (int i = 0; i < kIPT; ++i) {
+      const int pos = k_begin + tid + i * THREADS;
+      iraw[i] = -1;
+      if (i * THREADS < ntot) iraw[i] = irow[pos < k_end ? pos : k_end - 1];
+    }
+  }
+  uint4 qf[QJ];
+  {
+    const uint16_t *qrow = q + (qm * H + 16 * ht + l16) * Sh::DQK + 8 * g;
+#pragma unroll
+    for (int j = 0; j < QJ; ++j) qf[j] = *reinterpret_cast<const uint4 *>(qrow + 32 * j);
+  }
+#pragma unroll
+  for (int i = 0; i < kIPT; ++i) {
+    const int t = tid + i * THREADS;
+    if (t < ntot) sidx[t] = (k_begin + t < k_end && iraw[i] >= 0 && iraw[i] < N) ? iraw[i] : -1;
+  }
+  if (tid < 2) moved[tid] = 0u;
+#pragma unroll
+  for (int j = 0; j < QJ; ++j)  // the q loads complete here, not inside the loop
+    asm volatile("" : "+v"(qf[j].x), "+v"(qf[j].y), "+v"(qf[j].z), "+v"(qf[j].w));
+  __syncthreads();  // indices staged
+
+  const uint32_t kb_lds = __builtin_amdgcn_readfirstlane(lds_addr(&kb[0][0]));
+  const int njw = (TI - wave + NW - 1) / NW;  // this wave's DMA instructions per chunk
+  auto issue = [&](int c) {
+    const int buf = c % NBUF;
+    int32_t r[NJ];
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int jj = wave + NW * i < TI ? wave + NW * i : TI - 1;
+      r[i] = sidx[c * kKC + (64 * jj + lane) / UPR];
+    }
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int jj = wave + NW * i;
+      if (jj < TI) {  // uniform
+        const int sl = 64 * jj + lane;
+        const int key = sl / UPR;
+        const uint32_t voff =
+            static_cast<uint32_t>(r[i] < 0 ? 0 : r[i]) * (Sh::DQK * 2) + ((sl % UPR) ^ (key & 7)) * 16;
+        dma16((const void *)kvb, voff, kb_lds + (buf * Sh::BUF + 64 * jj * 8) * 2);
+      }
+    }
+  };
+  const int npre = nch < NBUF - 1 ? nch : NBUF - 1;
+  for (int c = 0; c < npre; ++c) issue(c);
+
+  // per-lane LDS element offsets, as above: QK key 16 kt + l16, PV keys 4g + (l16 >> 2) (+ 16)
+  int qk_off[2], pv_off[2][4];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) qk_off[p] = Sh::slot(16 * kt + l16, 0, 4 * p + g) * 8;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      pv_off[t][p] = Sh::slot(4 * g + (l16 >> 2) + 16 * t, 0, 2 * p + ((l16 & 3) >> 1)) * 8 + 4 * (l16 & 1) +
+                     2 * CTW * wave * 8;
+
+  float m_own = -INFINITY, l_run = 0.f;  // head 16 ht + l16: reference max; the lane's own keys' part of the sum
+  float m_ref[NHT];                      // references of heads 16 h + l16, the same in every wave
+  f32x4_t o[NHT][CTW];
+#pragma unroll
+  for (int h = 0; h < NHT; ++h) {
+    m_ref[h] = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < CTW; ++c) o[h][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  for (int c = 0; c < nch; ++c) {
+    // this wave's part of chunk c has landed once at most (chunks issued after it) x njw gathers remain
+    const int later = (nch - 1 - c) < (NBUF - 2) ? (nch - 1 - c) : (NBUF - 2);
+    wait_vm_le<(NBUF - 2) * NJ>(later * njw);
+    __syncthreads();  // everyone's part of chunk c is in place; chunk c - 1's buffer and probabilities are free
+    if (c + NBUF - 1 < nch) issue(c + NBUF - 1);
+    if (tid == 0) moved[(c + 1) & 1] = 0u;  // last read before this barrier, next written after the next chunk's
+    const uint32_t vm = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(sidx[c * kKC + (lane & 31)] >= 0));
+    const uint16_t *kbp = kb[c % NBUF];
+
+    // ---- S^T = K Q^T of the wave's tile: key 16 kt + 4 g + r, head 16 ht + l16 (two chains of the k-steps)
+    f32x4_t st, s2;
+    st = s2 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_nop 2" : "+v"(st), "+v"(s2));  // fences of the in-place MFMAs, as mfma_vgpr_enter / leave
+#pragma unroll
+    for (int j = 0; j < QJ; j += 2) {
+      mfma16_vgpr(st, *reinterpret_cast<const uint4 *>(kbp + qk_off[0] + ((4 * j) & ~7) * 8), qf[j]);
+      mfma16_vgpr(s2, *reinterpret_cast<const uint4 *>(kbp + qk_off[1] + ((4 * j + 4) & ~7) * 8), qf[j + 1]);
+    }
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(st), "+v"(s2));
+    st = (st + s2) * scale_log2;
+    if (vm != 0xFFFFFFFFu) {  // uniform
+      const uint32_t vbits = vm >> (16 * kt + 4 * g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] = ((vbits >> r) & 1u) ? st[r] : -INFINITY;
+    }
+    const float cmax = rows_max(fmaxf(fmaxf(st[0], st[1]), fmaxf(st[2], st[3])));
+    if (__builtin_amdgcn_ballot_w64(cmax > m_own + kRescaleTau) != 0ull && lane == 0) moved[c & 1] = 1u;
+    float p[4];
+    auto probabilities = [&]() {
+      const float mu = m_own == -INFINITY ? 0.f : m_own;  // masked keys: exp2(-inf - 0) while no key was valid
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p[r] = fast_exp2(st[r] - mu);
+      pb[ht][lane][kt] = make_uint2(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]));
+    };
+    probabilities();
+    __syncthreads();  // P and the flag are published
+    if (moved[c & 1] != 0u) {  // uniform over the workgroup
+      if (g == 0) sx[kt][16 * ht + l16] = cmax;
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < NHT; ++h) {
+        const float mx = fmaxf(sx[0][16 * h + l16], sx[1][16 * h + l16]);
+        const float m_old = m_ref[h];
+        const bool need = mx > m_old + kRescaleTau;
+        const float alpha = need ? (m_old == -INFINITY ? 0.f : fast_exp2(m_old - mx)) : 1.f;
+        m_ref[h] = need ? mx : m_old;
+        if (h == ht) {  // uniform
+          l_run *= alpha;
+          m_own = m_ref[h];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float ar = __shfl(alpha, 4 * g + r, 64);
+#pragma unroll
+          for (int cc = 0; cc < CTW; ++cc) o[h][cc][r] *= ar;
+        }
+      }
+      probabilities();
+      __syncthreads();
+    }
+    l_run += (p[0] + p[1]) + (p[2] + p[3]);
+
+    // ---- O += P V on the wave's columns; each V fragment feeds every head tile
+    uint4 pa[NHT];
+#pragma unroll
+    for (int h = 0; h < NHT; ++h) pa[h] = *reinterpret_cast<const uint4 *>(&pb[h][lane][0]);
+#pragma unroll
+    for (int cc = 0; cc < CTW; ++cc) {
+      const int hi = ((2 * cc) & ~7) * 8;
+      const uint2 b0 = lds_read_tr16(kbp + pv_off[0][cc & 3] + hi);
+      const uint2 b1 = lds_read_tr16(kbp + pv_off[1][cc & 3] + hi);
+      const uint4 vb = make_uint4(b0.x, b0.y, b1.x, b1.y);
+#pragma unroll
+      for (int h = 0; h < NHT; ++h) o[h][cc] = mfma16(pa[h], vb, o[h][cc]);
+    }
+  }
+
+  // ---- finalise (one range per query: sink added, bf16 output) or write the partial range
+  l_run = rows_sum(l_run);
+  __syncthreads();  // sx is free
+  if (g == 0) sx[kt][16 * ht + l16] = l_run;
+  __syncthreads();
+  if (NS > 1) {
+#pragma unroll
+    for (int h = 0; h < NHT; ++h) {
+      uint4 *pf = reinterpret_cast<uint4 *>(part_o) + mla_frag_offset(item, H / 32, h >> 1, h & 1, wave * (CTW / 2), lane);
+#pragma unroll
+      for (int cc = 0; cc < CTW; cc += 2)
+        pf[(cc / 2) * 64] = make_uint4(pack_bf16x2(o[h][cc][0], o[h][cc][1]), pack_bf16x2(o[h][cc][2], o[h][cc][3]),
+                                       pack_bf16x2(o[h][cc + 1][0], o[h][cc + 1][1]),
+                                       pack_bf16x2(o[h][cc + 1][2], o[h][cc + 1][3]));
+    }
+    if (kt == 0 && g == 0) {
+      const int head = 16 * ht + l16;
+      float *pml = part_ml + (item * H + head) * 2;
+      pml[0] = m_own;
+      pml[1] = sx[0][head] + sx[1][head];
+    }
+    return;
+  }
+#pragma unroll
+  for (int h = 0; h < NHT; ++h) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int hr = 16 * h + 4 * g + r;
+      const float mx = __shfl(m_ref[h], 4 * g + r, 64);
+      const float sm = sx[0][hr] + sx[1][hr];
+      const float sk = sink[hr] * kLog2e;
+      const float zmax = fmaxf(mx, sk);
+      float scale_o = 0.f;
+      if (zmax != -INFINITY) {
+        const float e = (mx == -INFINITY) ? 0.f : exp2f(mx - zmax);
+        const float den = sm * e + exp2f(sk - zmax);
+        scale_o = den > 0.f ? e / den : 0.f;
+      }
+      uint16_t *orow = out + (qm * H + hr) * Sh::DV + 16 * CTW * wave;
+#pragma unroll
+      for (int cc = 0; cc < CTW; cc += 2) {
+        const uint32_t pk = pack_bf16x2(o[h][cc][r] * scale_o, o[h][cc + 1][r] * scale_o);
+        orow[16 * cc + l16] = static_cast<uint16_t>(pk & 0xFFFFu);
+        orow[16 * (cc + 1) + l16] = static_cast<uint16_t>(pk >> 16);
+      }
     }
   }
 }
@@ -1171,7 +1421,6 @@ inline SaSplit mla_plan(int64_t B, int64_t M, int64_t K) {
 template <int NW>
 int launch_mla_nw(const uint16_t *q, const uint16_t *kv, const float *sink, const int32_t *idx, uint16_t *out,
                   int64_t B, int64_t M, int64_t H, int64_t N, int64_t K, float scale, void *ws, hipStream_t stream) {
-  using Sh = MlaShape<NW, kMlaBuffers>;
   const SaSplit sp = mla_plan(B, M, K);
   const int64_t n_items = B * M * sp.ns;
   uint16_t *part_o = nullptr;
@@ -1180,9 +1429,15 @@ int launch_mla_nw(const uint16_t *q, const uint16_t *kv, const float *sink, cons
     part_ml = static_cast<float *>(ws);
     part_o = reinterpret_cast<uint16_t *>(part_ml + n_items * H * 2);
   }
-  hipLaunchKernelGGL((sparse_attn_mla_kernel<NW, kMlaBuffers>), dim3(static_cast<unsigned>(n_items)),
-                     dim3(Sh::THREADS), 0, stream, q, kv, sink, idx, out, part_o, part_ml, M, static_cast<int>(H), N,
-                     K, sp.ns, sp.kr, scale * kLog2e);
+  if constexpr (NW <= 2) {
+    hipLaunchKernelGGL((sparse_attn_mla_kernel_cols<2 * NW>), dim3(static_cast<unsigned>(n_items)), dim3(256 * NW), 0,
+                       stream, q, kv, sink, idx, out, part_o, part_ml, M, N, K, sp.ns, sp.kr, scale * kLog2e);
+  } else {
+    using Sh = MlaShape<NW, kMlaBuffers>;
+    hipLaunchKernelGGL((sparse_attn_mla_kernel<NW, kMlaBuffers>), dim3(static_cast<unsigned>(n_items)),
+                       dim3(Sh::THREADS), 0, stream, q, kv, sink, idx, out, part_o, part_ml, M, static_cast<int>(H), N,
+                       K, sp.ns, sp.kr, scale * kLog2e);
+  }
   KS_CHECK_LAUNCH("sparse_attn_mla_kernel");
   if (sp.ns > 1) {
     // waves of (query, wave of the attention kernel, head tile, column tiles of kMlaCombineUnits units)

@@ -184,6 +184,35 @@ def test_sparse_attn_mla_leading_invalid(device):
     np.testing.assert_allclose(got, want, **TOL)
 
 
+# 32 and 64 heads split both products over the item's waves (scores by head and key tile, P V by columns): one chunk, the
+# ring's first three and a ragged last one, ranges capped at 2048 keys, one range per query and several, whole chunks of
+# invalid keys, and references that move in several chunks (also in the last one)
+@pytest.mark.parametrize("H", [32, 64])
+@pytest.mark.parametrize("B,M,K,bad", [(1, 1, 1, 0), (1, 2, 33, 0), (2, 1, 96, 40), (1, 257, 100, 0), (1, 1, 2049, 3),
+                                       (1, 2, 4000, 1500), (1, 300, 64, 64)])
+def test_sparse_attn_mla_split_by_columns(device, H, B, M, K, bad):
+    g = torch.Generator().manual_seed(H + K)
+    N = 2500
+    q = torch.randn(B, M, H, 576, generator=g).bfloat16()
+    kv = torch.randn(B, N, 576, generator=g).bfloat16()
+    idx = torch.randint(-3, N, (B, M, K), generator=g, dtype=torch.int32)
+    idx[:, :, :bad] = -1
+    sink = torch.randn(H, generator=g)
+    got = _run(q.to(device), kv.to(device), sink.to(device), idx.to(device), 576 ** -0.5, 512, f"mla cols H={H} K={K}")
+    want = oracle.sparse_attn(bits(q), bits(kv), sink.numpy(), idx.numpy(), 576 ** -0.5, 512)
+    np.testing.assert_allclose(got, want, **TOL)
+
+
+@pytest.mark.parametrize("H", [32, 64])
+def test_sparse_attn_mla_split_by_columns_rescale(device, H):
+    g = torch.Generator().manual_seed(23 + H)
+    q, kv, idx, scale = _rising_case(g, H, 512, [31, 32, 200, 330, 511])
+    sink = torch.zeros(H)
+    got = _run(q.to(device), kv.to(device), sink.to(device), idx.to(device), scale, 512, f"mla cols rescale H={H}")
+    want = oracle.sparse_attn(bits(q), bits(kv), sink.numpy(), idx.numpy(), scale, 512)
+    np.testing.assert_allclose(got, want, **TOL)
+
+
 # The count-mask kernel (ks_dbg_sparse_attn_count: the dense formulation over key splits, timed beside the gather
 # kernel by bench.py; ks_sparse_attn does not dispatch to it): one split finalised in place or several merged by the
 # combine kernel; N not a multiple of the 32-key chunk; the last 128-row block of a batch partly past the batch;
