@@ -101,12 +101,20 @@ struct DirectKeys {
   int64_t kbs = 0;
 };
 
+// Query rows that the recomputation prepares itself (TopkRecompute::rope), or none.
+struct RawQueries {
+  const uint16_t *q = nullptr;
+  const float *freqs = nullptr;
+  int rope_start = 0, rope_dim = 0;
+  float w_scale = 1.f;
+};
+
 // Scores of the prepared rows (ws.q_rot / ws.k_rot with their statistics, or the keys of dk) -> exact top-k.
 int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w_bf16, int64_t k_top, int32_t causal,
                    int64_t start_pos, int32_t ratio, int64_t offset, void *out, int32_t out_i64, int64_t B, int64_t S,
                    int64_t H, int64_t D, int64_t T, hipStream_t st, float bound_c, uint32_t *stats, int path,
                    const DirectKeys &dk = DirectKeys{}, const uint16_t *q_unrot = nullptr, int rot_lo = 0,
-                   int rot_hi = 0) {
+                   int rot_hi = 0, const RawQueries &rq = RawQueries{}) {
   const int64_t kk = k_top < T ? k_top : T;
   const bool can_bound = takes_bounded(k_top, H, D, T, 0);
   KS_CHECK_ARG(path < 2 || can_bound,
@@ -126,6 +134,14 @@ int indexer_select(const char *fn, const IndexerWs &ws, const void *w, int32_t w
     ks::TopkRecompute trc{ws.bounds, ws.q_rot, krows, w, w_bf16 ? 1 : 0, ws.q_norm,
                           ws.q_span, ws.k_norm, ws.k_span, kbs, T, bound_c, stats, path == 3 ? 1 : 0, ws.part,
                           ws.part_cap};
+    if (rq.q != nullptr) {
+      trc.q = rq.q;
+      trc.rope = 1;
+      trc.rope_start = rq.rope_start;
+      trc.rope_dim = rq.rope_dim;
+      trc.freqs = rq.freqs;
+      trc.w_scale = rq.w_scale;
+    }
     trc.kc = dk.kc;
     trc.ks = dk.ks;
     return ks::launch_indexer_topk_bounded(all ? nullptr : ws.scores, T, B, S, T, kk, causal ? 1 : 0, start_pos, ratio, offset, out,
@@ -187,6 +203,16 @@ int indexer_impl(const uint16_t *q, const uint16_t *k, const void *w, int32_t w_
   // w_scale != 1: the row preparation also writes the scaled weights (one per q row), which the later launches read
   const bool scaled = w_scale != 1.0f;
   const ks::WeightScale wsc{w, ws.w_scaled, w_scale, w_bf16 ? 1 : 0};
+  // every score recomputed: a query row meets one workgroup, which prepares it itself; this pass then takes the keys alone
+  const int64_t kk = k_top < T ? k_top : T;
+  if (bounded && ks::topk_bounded_all(S, T, kk, causal ? 1 : 0, start_pos, ratio)) {
+    const ks::RowJob none{nullptr, nullptr, nullptr, nullptr, 0, 1, 0, 1, 1, 0, 0};
+    rc = ks::launch_rope_rows(kjob, none, freqs, static_cast<int>(D), static_cast<int>(rope_start), st);
+    if (rc != KS_OK) return rc;
+    return indexer_select("ks_indexer", ws, w, w_bf16, k_top, causal, start_pos, ratio, offset, out, out_i64, B, S, H, D, T,
+                          st, bound_c, stats, path, dk, nullptr, 0, 0,
+                          RawQueries{q, freqs, static_cast<int>(rope_start), rd, w_scale});
+  }
   rc = ks::launch_rope_rows(qjob, kjob, freqs, static_cast<int>(D), static_cast<int>(rope_start), st,
                             scaled ? &wsc : nullptr);
   if (rc != KS_OK) return rc;

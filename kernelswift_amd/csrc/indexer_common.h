@@ -350,6 +350,11 @@ struct TopkRecompute {
   // FP8 keys (both set, or neither): codes [rows][128] and row scales, kbs rows per batch
   const uint8_t *kc = nullptr;
   const float *ks = nullptr;
+  // rope: q and w are the caller's rows and weights (qn, qsp unused): the recomputation rotates dims [rope_start,
+  // rope_start + rope_dim) of q at position start_pos + s and scales w (as launch_rope_rows does); only without scores
+  int rope = 0, rope_start = 0, rope_dim = 0;
+  const float *freqs = nullptr;
+  float w_scale = 1.f;
 };
 // Slots the bounded selection needs for `rows` rows of T <= 32768 columns (0 outside that range).
 int64_t topk_bounded_part_capacity(int64_t rows, int64_t T);

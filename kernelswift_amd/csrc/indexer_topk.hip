@@ -1143,7 +1143,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 // 95 us; here the other workgroup's tiles fill the chain of barriers, and the two launches' 346 us became 238).
 // MODE kRecAll: the same without scores and bounds: every valid column is recomputed (topk_bounded_all; saves the 76 us of
 // the score launch at that shape).
-constexpr int kRecLists = 0, kRecOneSeg = 1, kRecAll = 2;
+// MODE kRecAllRope: every query row meets one workgroup then, which also rotates it, scales its head weights and forms its
+// statistics on the way into LDS (the pass of its own, 98 MB in and out at that shape: 36 us; the call 349 -> 333 us).
+constexpr int kRecLists = 0, kRecOneSeg = 1, kRecAll = 2, kRecAllRope = 3;
 struct RecOut {  // the output of the one-segment modes
   void *out;
   int64_t offset;
@@ -1158,6 +1160,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
                                                                     uint2 *__restrict__ sstate,
                                                                     uint2 *__restrict__ rstate) {
   constexpr int SW = kRecThreads * KPB;
+  constexpr bool kAll = MODE >= kRecAll, kRope = MODE == kRecAllRope;
   __shared__ RecShared rs;
   __shared__ RecWave rw[kRecWaves];
   __shared__ int32_t list[SW];
@@ -1207,14 +1210,14 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     qv[i] = *reinterpret_cast<const uint4 *>(rc.q + (qrow0 + h) * kRecD + 8 * c);
   }
   const int hh = tid & (kRecH - 1);
-  const float wv = WBF ? bf16_to_f32(static_cast<const uint16_t *>(rc.w)[qrow0 + hh])
-                       : static_cast<const float *>(rc.w)[qrow0 + hh];
-  const float qnv = rc.qn[qrow0 + hh];
-  const int32_t qsv = rc.qsp[qrow0 + hh];
-  const uint32_t mrow = MODE == kRecAll ? 0u : rstate[row].y;
+  float wv = WBF ? bf16_to_f32(static_cast<const uint16_t *>(rc.w)[qrow0 + hh])
+                 : static_cast<const float *>(rc.w)[qrow0 + hh];
+  const float qnv = kRope ? 0.f : rc.qn[qrow0 + hh];
+  const int32_t qsv = kRope ? 0 : rc.qsp[qrow0 + hh];
+  const uint32_t mrow = kAll ? 0u : rstate[row].y;
   float sv[KPB], uv[KPB];
 #pragma unroll
-  for (int j = 0; j < KPB && MODE != kRecAll; ++j) {
+  for (int j = 0; j < KPB && !kAll; ++j) {
     const int col = j * kRecThreads + tid;
     sv[j] = srow[c0 + (col < nv ? col : 0)];
     uv[j] = urow[c0 + (col < nv ? col : 0)];
@@ -1230,23 +1233,46 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
 #pragma unroll
   for (int i = 0; i < kQPT; ++i) {
     const int idx = tid + i * kRecThreads, h = idx / kRecC, c = idx % kRecC;
+    if constexpr (kRope) {  // the head's 16 chunks are an aligned 16-lane group
+      const int e0 = 8 * c - rc.rope_start;
+      if (e0 >= 0 && e0 < rc.rope_dim)
+        qv[i] = rope_chunk(qv[i], reinterpret_cast<const float2 *>(rc.freqs) + (start_pos + s) * (rc.rope_dim / 2) + e0 / 2);
+      float ss = 0.f, norm;
+      uint32_t mmin = 0xFFFFFFFFu;
+      int32_t span;
+      chunk_stats_packed(qv[i], ss, mmin);
+      int lsb = lsb_of_min(mmin);
+      row_reduce<16>(ss, lsb);
+      row_norm_span(ss, lsb, norm, span);
+      if (c == 0) {
+        rs.qn[h] = norm;
+        rs.qd[h] = rc.bound_c * 0x1p-23f * (norm + 0x1p-122f);
+        rs.qsp[h] = span;
+      }
+    }
     rs.q[h * kRecC + (c ^ (h & 15))] = qv[i];
   }
-  rs.w[hh] = wv;  // four threads write each head entry, the same values
-  rs.qn[hh] = qnv;
-  rs.qd[hh] = rc.bound_c * 0x1p-23f * (qnv + 0x1p-122f);
-  rs.qsp[hh] = qsv;
+  if constexpr (kRope) wv = WBF ? bf16_to_f32(f32_to_bf16_rne(wv * rc.w_scale)) : wv * rc.w_scale;
+  rs.w[hh] = wv;  // eight threads write each head entry, the same values
+  if constexpr (!kRope) {
+    rs.qn[hh] = qnv;
+    rs.qd[hh] = rc.bound_c * 0x1p-23f * (qnv + 0x1p-122f);
+    rs.qsp[hh] = qsv;
+  }
   rs.wneg[hh] = __builtin_bit_cast(uint32_t, wv) >> 31 ? 0xFFFFu : 0u;
   // the query's largest padded head norm (lane h of every wave holds head h): decides per tile whether the
   // one-fma half-widths apply
-  float qpmax = qnv + 0x1p-122f;
-  qpmax = wave_max_f32(qpmax);
-  qpmax = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int32_t, qpmax)));
+  float qpmax = 0.f;
+  auto query_max = [&](float qn) {
+    qpmax = wave_max_f32(qn + 0x1p-122f);
+    qpmax = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int32_t, qpmax)));
+  };
+  if constexpr (!kRope) query_max(qnv);
 
   if (tid == 0) s_unc = 0u;
   uint32_t hik[KPB], masks = 0;  // bit j: column j is a candidate; bit 8 + j: it has a slot
   uint32_t tau = 1u, ncand = 0, nres = 0, bexcl = 0;
-  if constexpr (MODE == kRecAll) {
+  if constexpr (kAll) {
     ncand = static_cast<uint32_t>(nv);
     for (int i = tid; i < nv; i += kRecThreads) list[i] = i;
   } else {
@@ -1335,6 +1361,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   }
   __syncthreads();
   uint32_t n_exact = 0, n_unres = 0;
+  if constexpr (kRope) query_max(rs.qn[tid & (kRecH - 1)]);
   if (ncand > 0) {
     const int64_t kbrow0 = b * rc.kbs;
     int nrec = static_cast<int>(ncand);
@@ -1376,7 +1403,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     for (int j = 0; j < KPB; ++j) {
       const int col = j * kRecThreads + tid;
       uint32_t key = 0u;
-      if constexpr (MODE == kRecAll) {
+      if constexpr (kAll) {
         if (col < nv) key = score_key(listf[col]);
       } else if ((masks >> (8 + j)) & 1u) {
         const bool cj = (masks >> j) & 1u;
@@ -1625,6 +1652,7 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   const dim3 rgrid(static_cast<unsigned>(rows * segs));
   const bool f8 = rc.kc != nullptr;
   const bool one = kpb == 2 && segs == 1, all = scores == nullptr;
+  KS_CHECK_ARG(!rc.rope || (all && !f8), "indexer top-k (bounded): unrotated queries need every score recomputed");
   KS_CHECK_ARG(!all || one, "indexer top-k (bounded): scores are needed past %d columns", 2 * kRecThreads);
   KS_CHECK_ARG(f8 == (rc.ks != nullptr), "indexer top-k (bounded): FP8 keys need codes and scales");
   const RecOut ro{out, offset, o};
@@ -1634,6 +1662,9 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   };
   auto rec_k = [&](auto F8, auto WBF) {
     constexpr bool f = decltype(F8)::value, wb = decltype(WBF)::value;
+    if constexpr (!f) {
+      if (all && rc.rope) return rec(topk_recompute_kernel<2, false, wb, kRecAllRope>);
+    }
     if (all) rec(topk_recompute_kernel<2, f, wb, kRecAll>);
     else if (one) rec(topk_recompute_kernel<2, f, wb, kRecOneSeg>);
     else if (kpb == 2) rec(topk_recompute_kernel<2, f, wb, kRecLists>);

@@ -138,3 +138,26 @@ def test_one_segment_rows_ties_and_range(device, wbf, k_top):
     _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, k_top, False, 0)
     print(f"[case] one segment, overflow guard, k={k_top} bf16={wbf}", flush=True)
     _check(device, (q * 2.0 ** 59).bfloat16(), (k * 2.0 ** 59).bfloat16(), w.bfloat16() if wbf else w, k_top, False, 0)
+
+
+# rows whose every score is recomputed: the recomputation rotates the queries and scales the weights itself; rotated ranges
+# at either end, inside, of all dims and none, rotated and plain keys, a scale that is not a power of two
+@pytest.mark.parametrize("rs,rd,rope_k,wbf,scale", [
+    (0, 64, True, True, 0.0127), (64, 64, False, True, -0.0127), (64, 64, False, False, 0.0127), (24, 96, True, False, 1.0),
+    (0, 128, False, True, 1.0), (0, 0, False, False, 0.3)])
+def test_one_segment_prepares_queries(device, rs, rd, rope_k, wbf, scale):
+    g = torch.Generator().manual_seed(rs + rd)
+    B, S, T, start = 2, 37, 90, 300
+    q = torch.randn(B, S, 64, 128, generator=g).bfloat16()
+    cache = torch.randn(B, T + 7, 128, generator=g).bfloat16()
+    w = torch.randn(B, S, 64, generator=g)
+    w = w.bfloat16() if wbf else w
+    tab = workloads.freqs_table(max(rd, 2), start + S + 1)
+    print(f"[case] recomputation prepares queries rope {rs}+{rd} keys={rope_k} bf16={wbf}", flush=True)
+    got = ops.indexer(q.to(device), cache.to(device), w.to(device), tab.to(device), 80, True, start, 4, 11, rs, rd, rope_k,
+                      T=T, w_scale=scale).cpu().numpy().astype(np.int64)
+    ws = w * scale
+    for b in range(B):
+        want = oracle.indexer(_u16(q[b:b + 1]), _u16(cache[b:b + 1, :T].contiguous()), _u16(ws[b:b + 1]) if wbf else
+                              ws[b:b + 1].numpy(), tab.numpy(), 80, True, start, 4, 11, rs, rd, rope_k)
+        np.testing.assert_array_equal(got[b:b + 1], want)
