@@ -270,7 +270,8 @@ __global__ __launch_bounds__((SaShape<DQK, DV, GW>::THREADS)) void sparse_attn_k
       pv_off[t][p] = Sh::slot(kv_key, 0, 2 * p + ((l16 & 3) >> 1)) * 8 + 4 * (l16 & 1);
   }
 
-  float m_ref = -INFINITY, l_run = 0.f;  // per head (lane l16), replicated over g
+  // per head (lane l16): the reference max, replicated over g, and the lane's own keys' part of the sum
+  float m_ref = -INFINITY, l_run = 0.f;
   f32x4_t o[CT];
 #pragma unroll
   for (int c = 0; c < CT; ++c) o[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -301,19 +302,16 @@ __global__ __launch_bounds__((SaShape<DQK, DV, GW>::THREADS)) void sparse_attn_k
       }
     }
     // ---- online softmax (lane: head l16, keys 16t + 4g + r)
-    const uint32_t vbits = vm_cur >> (4 * g);  // bit 16t + r: key 16t + 4g + r
     float sc[8];
-    float cmax = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int i = 0; i < 8; ++i) sc[i] = st[i >> 2][i & 3] * scale_log2;
+    if (vm_cur != 0xFFFFFFFFu) {  // uniform per wave: whole chunks need no masks
+      const uint32_t vbits = vm_cur >> (4 * g);  // bit 16t + r: key 16t + 4g + r
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool ok = (vbits >> (16 * t + r)) & 1u;
-        const float sv = ok ? st[t][r] * scale_log2 : -INFINITY;
-        sc[4 * t + r] = sv;
-        cmax = fmaxf(cmax, sv);
-      }
-    cmax = rows_max(cmax);
+      for (int i = 0; i < 8; ++i) sc[i] = ((vbits >> (16 * (i >> 2) + (i & 3))) & 1u) ? sc[i] : -INFINITY;
+    }
+    const float cmax = rows_max(fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])),
+                                      fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7]))));
     const bool need = cmax > m_ref + kRescaleTau;  // false for cmax = -inf; true for a first valid chunk
     if (__builtin_amdgcn_ballot_w64(need) != 0ull) {
       const float m_new = need ? cmax : m_ref;
@@ -328,13 +326,11 @@ __global__ __launch_bounds__((SaShape<DQK, DV, GW>::THREADS)) void sparse_attn_k
         for (int cc = 0; cc < CT; ++cc) o[cc][r] *= ar;
       }
     }
-    float p[8], csum = 0.f;
+    float p[8];
+    const float mu = m_ref == -INFINITY ? 0.f : m_ref;  // masked keys: exp2(-inf - 0) while no key was valid
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      p[i] = sc[i] == -INFINITY ? 0.f : fast_exp2(sc[i] - m_ref);
-      csum += p[i];
-    }
-    l_run += rows_sum(csum);
+    for (int i = 0; i < 8; ++i) p[i] = fast_exp2(sc[i] - mu);
+    l_run += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     // ---- O += P V: V fragment of keys 16h + 4g + (l16 >> 2), dv columns 16cc + 4(l16 & 3) .. +3
     const uint4 pa = make_uint4(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
                                 pack_bf16x2(p[6], p[7]));
@@ -353,6 +349,8 @@ __global__ __launch_bounds__((SaShape<DQK, DV, GW>::THREADS)) void sparse_attn_k
     if constexpr (GW > 1) __syncthreads();
     vm_cur = vm_next;
   }
+
+  l_run = rows_sum(l_run);
 
   // Merge of the GROUPS ranges of one query held by this workgroup (one-wave groups): each wave leaves its
   // (max, sum) per head and its O in LDS (the chunk buffers are free now); the workgroup then combines
