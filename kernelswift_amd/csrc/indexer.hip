@@ -7,7 +7,8 @@
 // sequence rope_inplace -> fused_qk_reduce -> topk_mask (optimized/indexer_project/indexer.py:197-222).
 // All intermediates live in the caller's workspace; inputs are never modified.  RoPE stays a pass of its
 // own: done inside the score kernel it would be repeated by every workgroup that reads a row (S/8 times
-// per key row), which measured twice as slow as the separate pass.
+// per key row), which measured twice as slow as the separate pass.  (Where every score of a row is computed
+// exactly by one workgroup, without approximate scores, that workgroup rotates its query itself.)
 //
 // With 64 heads and D = 128 the scores are computed with bounds instead of exactly: the
 // score kernel keeps an approximate score and a bound on its error, and the top-k kernel recomputes exactly only the

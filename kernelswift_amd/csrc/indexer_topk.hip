@@ -624,6 +624,8 @@ __device__ __forceinline__ void wave_max2(uint32_t &a, uint32_t &b) {
 //  3. topk_collected_kernel, one workgroup per row: the lists hold every column of the top k, each with its exact
 //     score, so sorting their nonempty slots gives the top k.  More slots than LDS takes
 //     fall back to the exact selection over the row, on keys spread from the lists (0 for the columns in none).
+// Rows of one segment (at most 2 kRecThreads columns) take the second launch alone, which ranks and stores them itself;
+// where most of their columns are selected (topk_bounded_all), it takes no scores and recomputes every valid column.
 constexpr int kRecD = 128;        // head dim of the recomputation
 constexpr int kRecH = 64;         // heads
 constexpr int kRecC = kRecD / 8;  // 16-byte chunks per row
