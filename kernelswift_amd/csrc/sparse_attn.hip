@@ -881,8 +881,11 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
 // bytes.  All waves share each head's lazily moved reference max; a wave whose chunk maximum passes it by the threshold
 // raises a flag, and after the barrier that publishes P every wave takes the (rare) path that moves the references,
 // rescales and forms P again.  Two barriers per chunk; gather ring, staged indices, partials and their combine as above.
-// 512 queries of 32 heads, K 2048, N 8192: 577 -> 168 us; 256 queries of 64 heads: 162 -> 106 us.  (96 heads' column tiles
-// do not divide by its waves; 128 heads would need 16 waves of 128 registers.)
+// Every dot is one chain over its k-steps and every chunk's sum runs in key order (tile 0's four probabilities of a lane,
+// then tile 1's), so the results are those of a wave that holds both key tiles, bit for bit (two chains a dot and a sum per
+// tile would save 1% and move P's roundings).
+// 512 queries, K 2048, N 8192, against 32 heads a wave: 32 heads 582 -> 171 us, 64 heads 321 -> 202.  (96 heads'
+// column tiles do not divide by its waves; eight waves of 128 heads, a head tile and both key tiles each, are not built.)
 template <int NHT>
 __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ kv, const float *__restrict__ sink,
@@ -897,13 +900,16 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
   __shared__ __attribute__((aligned(16))) uint16_t kb[NBUF][Sh::BUF];
   __shared__ __attribute__((aligned(16))) uint2 pb[NHT][64][2];
   __shared__ int32_t sidx[Sh::KR_MAX];
-  __shared__ float sx[2][H];      // per key tile and head: chunk maxima (moving references), at the end the sums
+  __shared__ float ps[NHT][64];   // per lane of key tile 0: the sum of its four probabilities
+  __shared__ float sx[2][H];      // per key tile and head: chunk maxima (moving references); at the end the sums in sx[1]
   __shared__ uint32_t moved[2];   // chunk parity: some reference has to move
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
-  const int ht = wave >> 1, kt = wave & 1;  // the wave's score tile
+  // the wave's score tile: with eight waves each SIMD holds one wave of either key tile (tile 1's also keep the sums; with
+  // pairs of waves by head tile 512 queries took 209 us, this way 202; with four waves, one a SIMD, pairs: 173 -> 170)
+  const int ht = NHT == 4 ? wave % NHT : wave >> 1, kt = NHT == 4 ? wave / NHT : wave & 1;
   const int64_t nblk = gridDim.x;
   const int64_t item = (nblk % 8 == 0) ? (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
   const int64_t qm = item / NS;
@@ -980,7 +986,7 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
       pv_off[t][p] = Sh::slot(4 * g + (l16 >> 2) + 16 * t, 0, 2 * p + ((l16 & 3) >> 1)) * 8 + 4 * (l16 & 1) +
                      2 * CTW * wave * 8;
 
-  float m_own = -INFINITY, l_run = 0.f;  // head 16 ht + l16: reference max; the lane's own keys' part of the sum
+  float m_own = -INFINITY, l_run = 0.f;  // head 16 ht + l16: reference max; running sum (waves of key tile 1)
   float m_ref[NHT];                      // references of heads 16 h + l16, the same in every wave
   f32x4_t o[NHT][CTW];
 #pragma unroll
@@ -1000,17 +1006,15 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
     const uint32_t vm = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(sidx[c * kKC + (lane & 31)] >= 0));
     const uint16_t *kbp = kb[c % NBUF];
 
-    // ---- S^T = K Q^T of the wave's tile: key 16 kt + 4 g + r, head 16 ht + l16 (two chains of the k-steps)
-    f32x4_t st, s2;
-    st = s2 = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_nop 2" : "+v"(st), "+v"(s2));  // fences of the in-place MFMAs, as mfma_vgpr_enter / leave
+    // ---- S^T = K Q^T of the wave's tile: key 16 kt + 4 g + r, head 16 ht + l16 (one chain over the k-steps: a dot's
+    // value does not depend on how many heads share the call)
+    f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_nop 2" : "+v"(st));  // fences of the in-place MFMAs, as mfma_vgpr_enter / leave
 #pragma unroll
-    for (int j = 0; j < QJ; j += 2) {
-      mfma16_vgpr(st, *reinterpret_cast<const uint4 *>(kbp + qk_off[0] + ((4 * j) & ~7) * 8), qf[j]);
-      mfma16_vgpr(s2, *reinterpret_cast<const uint4 *>(kbp + qk_off[1] + ((4 * j + 4) & ~7) * 8), qf[j + 1]);
-    }
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(st), "+v"(s2));
-    st = (st + s2) * scale_log2;
+    for (int j = 0; j < QJ; ++j)
+      mfma16_vgpr(st, *reinterpret_cast<const uint4 *>(kbp + qk_off[j & 1] + ((4 * j) & ~7) * 8), qf[j]);
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(st));
+    st *= scale_log2;
     if (vm != 0xFFFFFFFFu) {  // uniform
       const uint32_t vbits = vm >> (16 * kt + 4 * g);
 #pragma unroll
@@ -1024,6 +1028,7 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
 #pragma unroll
       for (int r = 0; r < 4; ++r) p[r] = fast_exp2(st[r] - mu);
       pb[ht][lane][kt] = make_uint2(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]));
+      if (kt == 0) ps[ht][lane] = ((p[0] + p[1]) + p[2]) + p[3];  // uniform
     };
     probabilities();
     __syncthreads();  // P and the flag are published
@@ -1051,7 +1056,8 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
       probabilities();
       __syncthreads();
     }
-    l_run += (p[0] + p[1]) + (p[2] + p[3]);
+    // the chunk's sum in key order: tile 0's four, then tile 1's, then over the lane groups
+    if (kt == 1) l_run += rows_sum((((ps[ht][lane] + p[0]) + p[1]) + p[2]) + p[3]);
 
     // ---- O += P V on the wave's columns; each V fragment feeds every head tile
     uint4 pa[NHT];
@@ -1069,9 +1075,8 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
   }
 
   // ---- finalise (one range per query: sink added, bf16 output) or write the partial range
-  l_run = rows_sum(l_run);
   __syncthreads();  // sx is free
-  if (g == 0) sx[kt][16 * ht + l16] = l_run;
+  if (kt == 1 && g == 0) sx[1][16 * ht + l16] = l_run;
   __syncthreads();
   if (NS > 1) {
 #pragma unroll
@@ -1087,7 +1092,7 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
       const int head = 16 * ht + l16;
       float *pml = part_ml + (item * H + head) * 2;
       pml[0] = m_own;
-      pml[1] = sx[0][head] + sx[1][head];
+      pml[1] = sx[1][head];
     }
     return;
   }
@@ -1097,7 +1102,7 @@ __global__ __launch_bounds__(128 * NHT, 1) void sparse_attn_mla_kernel_cols(
     for (int r = 0; r < 4; ++r) {
       const int hr = 16 * h + 4 * g + r;
       const float mx = __shfl(m_ref[h], 4 * g + r, 64);
-      const float sm = sx[0][hr] + sx[1][hr];
+      const float sm = sx[1][hr];
       const float sk = sink[hr] * kLog2e;
       const float zmax = fmaxf(mx, sk);
       float scale_o = 0.f;

@@ -213,6 +213,23 @@ def test_sparse_attn_mla_split_by_columns_rescale(device, H):
     np.testing.assert_allclose(got, want, **TOL)
 
 
+# A head's output does not depend on how many heads share the call: every MLA form takes a dot's k-steps in one chain.  Two
+# valid keys a query, so that their sum has one order in every form.
+@pytest.mark.parametrize("H", [32, 64, 96])
+def test_sparse_attn_mla_heads_alone_or_shared(device, H):
+    g = torch.Generator().manual_seed(H)
+    M, N = 96, 300
+    q = torch.randn(1, M, 128, 576, generator=g).bfloat16().to(device)
+    kv = torch.randn(1, N, 576, generator=g).bfloat16().to(device)
+    idx = torch.full((1, M, 40), -1, dtype=torch.int32)
+    idx[:, :, 5], idx[:, :, 30] = torch.randint(0, N, (1, M), generator=g), torch.randint(0, N, (1, M), generator=g)
+    idx, sink = idx.to(device), torch.randn(128, generator=g).to(device)
+    print(f"[case] mla heads alone or shared H={H}", flush=True)
+    many = ops.sparse_attn(q, kv, sink, idx, 576 ** -0.5, dv=512)[:, :, :H]
+    few = ops.sparse_attn(q[:, :, :H].contiguous(), kv, sink[:H].contiguous(), idx, 576 ** -0.5, dv=512)
+    assert torch.equal(few.view(torch.int16), many.contiguous().view(torch.int16))
+
+
 # The count-mask kernel (ks_dbg_sparse_attn_count: the dense formulation over key splits, timed beside the gather
 # kernel by bench.py; ks_sparse_attn does not dispatch to it): one split finalised in place or several merged by the
 # combine kernel; N not a multiple of the 32-key chunk; the last 128-row block of a batch partly past the batch;
