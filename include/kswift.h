@@ -121,9 +121,11 @@ int ks_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w,
 
 /* ------------------------------------------------------------------------
  * Per-row statistics of bf16 rows of length D (64 or 128) for ks_indexer_scores:
- *   norm[r] >= ||x_r||_2 (an upper bound within 2^-11 relative),
+ *   norm[r] >= ||x_r||_2 (an upper bound within 2^-11 relative, or 2^-71 for
+ *              tiny rows; infinite where the sum of squares leaves fp32),
  *   span[r]  = ceil(log2 norm[r]) - (exponent of the least significant bit of
- *              the smallest nonzero element), 0 for an all-zero row.
+ *              the smallest nonzero element), 0 for an all-zero row, 1024
+ *              where norm[r] is infinite.
  * No reference counterpart: the reference kernel had no exactness contract.
  * ---------------------------------------------------------------------- */
 int ks_indexer_row_stats(const uint16_t *x, int64_t rows, int64_t D, float *norm,

@@ -234,12 +234,15 @@ __device__ __forceinline__ void row_reduce(float &ss, int &lsb) {
 }
 
 // Norm upper bound and span from a row's sum of squares and smallest LSB exponent: an fp32 sum of at most
-// 128 exact squares has relative error < 2^-16 and sqrt adds < 1 ulp; the 2^-12 pad covers both.
+// 128 exact squares has relative error < 2^-16 and sqrt adds < 1 ulp; the 2^-12 pad covers both.  Squares below the fp32
+// range lose up to 2^-150 each, the 2^-142 added to a nonzero row's sum (nothing beside an ordinary one).  Squares above it:
+// the norm is infinite, which makes every dot of the row a near tie, and the span sends them to the integer accumulator.
 __device__ __forceinline__ void row_norm_span(float ss, int lsb, float &norm, int32_t &span) {
-  norm = ss > 0.f ? sqrtf(ss) * (1.0f + 0x1p-12f) : 0.f;
+  const bool any = lsb < (1 << 20);
+  norm = any ? sqrtf(ss + 0x1p-142f) * (1.0f + 0x1p-12f) : 0.f;
   int top = 0;
   if (norm > 0.f) frexpf(norm, &top);  // norm < 2^top
-  span = norm > 0.f ? top - lsb : 0;
+  span = !any ? 0 : norm < __builtin_inff() ? top - lsb : 1024;
 }
 
 // Division by a runtime divisor 1 <= d < 2^32 with a multiply-high, an add and a shift (the round-up

@@ -74,6 +74,48 @@ def test_row_stats(device):
     np.testing.assert_array_equal(s[n > 0], (top - lsb)[n > 0])
 
 
+def test_row_stats_past_the_range_of_squares(device):
+    # rows whose squares leave the fp32 range: the norm stays an upper bound, and an infinite one claims no span
+    g = torch.Generator().manual_seed(3)
+    for D in (64, 128):
+        x = torch.randn(40, D, generator=g)
+        e = torch.tensor([2.0 ** i for i in range(-132, 124, 7)][:37])
+        x[:37] *= e[:, None]
+        x[37] = 2.0 ** -133
+        x[38] = 2.0 ** 64
+        x[39] = 0.0
+        x = x.bfloat16()
+        print(f"[case] row stats past the range of squares D={D}", flush=True)
+        n, s = ops.indexer_row_stats(x.to(device))
+        n, s = n.cpu().double(), s.cpu()
+        true = x.double().pow(2).sum(1).sqrt()
+        big = true > 2.0 ** -60
+        assert (n >= true).all() and ((n[big] <= true[big] * (1 + 2 ** -10)) | torch.isinf(n[big])).all()
+        assert n[39] == 0 and s[39] == 0
+        assert (s[n == float("inf")] == 1024).all() and (n == float("inf")).any()
+
+
+# dots on bf16 midpoints that a third, far smaller product decides, in rows whose squares leave the fp32 range: past it
+# (infinite norms, span unknown) and below it (norms that would come out as zero)
+@pytest.mark.parametrize("qe,ke", [(65, 0), (0, 65), (-80, 70), (70, -80), (-80, -30), (66, 40)])
+@pytest.mark.parametrize("B,S,T,H,D", [(1, 2, 300, 64, 128), (1, 9, 300, 64, 128), (1, 9, 1500, 64, 128), (1, 9, 300, 32, 128),
+                                       (1, 9, 300, 16, 64)])
+def test_indexer_midpoints_of_extreme_rows(device, qe, ke, B, S, T, H, D):
+    q = torch.zeros(B, S, H, D)
+    k = torch.zeros(B, T, D)
+    o = D - 8  # unrotated dims
+    q[..., 0, o], q[..., 0, o + 1], q[..., 0, o + 2] = 2.0 ** qe, 2.0 ** (qe - 8), 2.0 ** (qe - 30)
+    sign = torch.randint(-1, 2, (B, T), generator=torch.Generator().manual_seed(T)).float()
+    k[..., o], k[..., o + 1], k[..., o + 2] = 2.0 ** ke, 2.0 ** ke, 2.0 ** (ke - 15) * sign
+    w = torch.ones(B, S, H)
+    q, k, k_top = q.bfloat16(), k.bfloat16(), 120
+    tab = workloads.freqs_table(32, T + S)
+    print(f"[case] midpoints of extreme rows 2^{qe} 2^{ke} {B, S, T, H, D}", flush=True)
+    got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), k_top, False, 0, 1, 0, 0, 32, True)
+    want = oracle.indexer(_u16(q), _u16(k), w.numpy(), tab.numpy(), k_top, False, 0, 1, 0, 0, 32, True)
+    np.testing.assert_array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
 def oracle_lsb(b):
     e = (int(b) >> 7) & 0xFF
     return -133 if e == 0 else e - 134
