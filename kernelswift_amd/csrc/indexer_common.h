@@ -32,6 +32,35 @@ __device__ __forceinline__ uint32_t bound_digit_edge(uint32_t d, uint32_t M) {
   return d == 0u ? 1u : ~(0x80000000u | (M >= (d << 17) ? M - (d << 17) : 0u));
 }
 
+// Buckets of the rank store's counting sort over the keys [kmin, kmax]: kRankBuckets, monotone in the key for every key,
+// infinities among them.  Uniform in the key (logarithmic in the score) over a positive range of at most eight octaves;
+// otherwise uniform in the score: a range that reaches down to zero or below it holds so many octaves of tiny magnitudes that uniform keys left
+// all large scores in a few buckets (12000 columns, k = 2048, where a third of the rows' k-th scores lie there:
+// the 128-row launch took 32.6 us, with this 7.7; 64 rows of 32768: 15.7 -> 7.7).  Scores as halves and infinities as the
+// largest finite values, so that no difference overflows.
+constexpr int kRankBuckets = 2048;
+constexpr uint32_t kKeyLowest = 0x00800000u, kKeyHighest = 0xFF7FFFFFu;  // keys of -/+ the largest finite value
+struct RankScale {
+  uint32_t k0;
+  float h0, scale;
+  bool by_key;
+  __host__ __device__ __forceinline__ static float half_value(uint32_t key) {
+    key = key < kKeyLowest ? kKeyLowest : key > kKeyHighest ? kKeyHighest : key;
+    return 0.5f * __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
+  }
+  __host__ __device__ __forceinline__ RankScale(uint32_t kmin, uint32_t kmax) {
+    by_key = kmin >= 0x80000000u && kmax - kmin < (8u << 23);
+    k0 = kmin;
+    h0 = half_value(kmin);
+    const float range = by_key ? static_cast<float>(kmax - kmin) + 1.0f : half_value(kmax) - h0;
+    scale = static_cast<float>(kRankBuckets) / (range > 1e-30f ? range : 1e-30f);
+  }
+  __host__ __device__ __forceinline__ uint32_t bucket(uint32_t key) const {
+    const float d = (by_key ? static_cast<float>(key - k0) : half_value(key) - h0) * scale;
+    return d < static_cast<float>(kRankBuckets - 1) ? static_cast<uint32_t>(d > 0.f ? d : 0.f) : kRankBuckets - 1;
+  }
+};
+
 // Exponent of the least significant bit of a nonzero bf16 value: value = m * 2^lsb, m integer.
 __host__ __device__ inline int bf16_lsb_exponent(uint16_t b) {
   const int e = (b >> 7) & 0xFF;

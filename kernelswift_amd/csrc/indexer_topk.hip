@@ -1000,34 +1000,7 @@ __device__ void recompute_scores(int32_t *list, const uint16_t *sel, int n, cons
 // dependent merge rounds of a sort.  Returns false, having stored nothing, when a bucket holds more than
 // kRankBucketMax entries (keys tied or clustered far beyond a smooth distribution); the caller then sorts.  Uses
 // cnt and start (kRankBuckets each), wsum and tmp[0, cap).
-constexpr int kRankBuckets = 2048;
 constexpr int kRankBucketMax = 256;
-// Uniform in the key (logarithmic in the score) over a positive range of at most eight octaves; otherwise uniform in the
-// score: a range that reaches down to zero or below it holds so many octaves of tiny magnitudes that uniform keys left
-// all large scores in a few buckets (12000 columns, k = 2048, where a third of the rows' k-th scores lie there:
-// the 128-row launch took 32.6 us, with this 7.7; 64 rows of 32768: 15.7 -> 7.7).
-struct RankScale {
-  uint32_t k0;
-  float v0, scale;
-  bool by_key;
-  __device__ __forceinline__ static float value(uint32_t key) {
-    return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
-  }
-  __device__ __forceinline__ RankScale(uint32_t kmin, uint32_t kmax) {
-    by_key = kmin >= 0x80000000u && kmax - kmin < (8u << 23);
-    // the ends as finite values (kmin may be below every value, kmax infinity)
-    const uint32_t lowest = 0x00800000u, highest = 0xFF7FFFFFu;  // keys of -/+ the largest finite value
-    k0 = kmin;
-    v0 = value(kmin < lowest ? lowest : kmin);
-    const float v1 = value(kmax > highest ? highest : kmax);
-    const float range = by_key ? static_cast<float>(kmax - kmin) + 1.0f : v1 - v0;
-    scale = range < 3e38f ? static_cast<float>(kRankBuckets) / fmaxf(range, 1e-30f) : 0.f;
-  }
-  __device__ __forceinline__ uint32_t bucket(uint32_t key) const {
-    const float d = (by_key ? static_cast<float>(key - k0) : value(key) - v0) * scale;
-    return d < static_cast<float>(kRankBuckets - 1) ? static_cast<uint32_t>(d > 0.f ? d : 0.f) : kRankBuckets - 1;
-  }
-};
 template <int PER, int NT = kTopkThreads>
 __device__ bool rank_store(const uint64_t (&v)[PER], uint32_t kmin, uint32_t kmax, int k_sel, int64_t row,
                            int k, void *out, int out_i64, int causal, int64_t limit, int64_t offset, uint64_t *tmp,
@@ -1532,7 +1505,32 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
           v[j] = i < n ? cand[i] : 0;
         }
       }
-      if (!rank_store<kMaxPer>(v, tau, top, k_sel, row, k, out, out_i64, causal, limit, offset, cand,
+      // the range to rank: from the threshold to the largest upper end, or, where one of them lies past the finite values
+      // (bounds that say nothing, infinite scores), from the smallest to the largest listed key
+      uint32_t kmin = tau, kmax = top;
+      if (tau < kKeyLowest || top > kKeyHighest) {  // uniform
+        uint32_t nmin = 0u;
+        kmax = 0u;
+#pragma unroll
+        for (int j = 0; j < kMaxPer; ++j) {
+          const uint32_t key = static_cast<uint32_t>(v[j] >> 32);
+          kmax = key > kmax ? key : kmax;
+          if (key != 0u) nmin = ~key > nmin ? ~key : nmin;
+        }
+        wave_max2(nmin, kmax);
+        uint32_t *ends = sh.hist[1];  // free until the ranks' bucket starts
+        if (lane == 0) {
+          ends[tid >> 6] = nmin;
+          ends[kTopkWaves + (tid >> 6)] = kmax;
+        }
+        __syncthreads();
+        for (int w = 0; w < kTopkWaves; ++w) {
+          nmin = ends[w] > nmin ? ends[w] : nmin;
+          kmax = ends[kTopkWaves + w] > kmax ? ends[kTopkWaves + w] : kmax;
+        }
+        kmin = ~nmin;
+      }
+      if (!rank_store<kMaxPer>(v, kmin, kmax, k_sel, row, k, out, out_i64, causal, limit, offset, cand,
                                sh.hist[0], sh.hist[1], sh.wsum)) {
         gather();
         int P = 128;
@@ -1753,3 +1751,9 @@ extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const f
 }
 
 extern "C" int64_t ks_dbg_topk_bounded_slots(int64_t rows, int64_t T) { return ks::topk_bounded_part_capacity(rows, T); }
+
+// The rank buckets of n keys over [kmin, kmax], on the host (the device's own functions).
+extern "C" void ks_dbg_rank_buckets(const uint32_t *keys, int64_t n, uint32_t kmin, uint32_t kmax, uint32_t *out) {
+  const ks::RankScale rk(kmin, kmax);
+  for (int64_t i = 0; i < n; ++i) out[i] = rk.bucket(keys[i]);
+}

@@ -161,3 +161,26 @@ def test_one_segment_prepares_queries(device, rs, rd, rope_k, wbf, scale):
         want = oracle.indexer(_u16(q[b:b + 1]), _u16(cache[b:b + 1, :T].contiguous()), _u16(ws[b:b + 1]) if wbf else
                               ws[b:b + 1].numpy(), tab.numpy(), 80, True, start, 4, 11, rs, rd, rope_k)
         np.testing.assert_array_equal(got[b:b + 1], want)
+
+
+# infinite scores of finite inputs: they rank first (+inf) and last (-inf), among themselves by column.  One segment with
+# every column recomputed and with a threshold, lists over short causal prefixes and long rows; "dots": one head's dot
+# rounds to +inf; "weights": the weighted dot overflows
+@pytest.mark.parametrize("wbf", [False, True])
+@pytest.mark.parametrize("how", ["dots", "weights"])
+@pytest.mark.parametrize("S,T,k_top,causal,start,share", [
+    (9, 100, 100, False, 0, 0.1), (6, 250, 100, False, 0, 0.7), (7, 1024, 700, False, 0, 0.2), (8, 3000, 512, True, 120, 0.3),
+    (6, 3000, 300, False, 0, 0.95), (3, 9000, 600, False, 0, 0.04)])
+def test_infinite_scores(device, wbf, how, S, T, k_top, causal, start, share):
+    g = torch.Generator().manual_seed(T + k_top)
+    q = torch.randn(1, S, 64, 128, generator=g)
+    k = torch.randn(1, T, 128, generator=g)
+    w = torch.randn(1, S, 64, generator=g) / 8
+    w[0, :, 0] = torch.where(torch.arange(S) % 3 == 0, 1.0, -1.0)
+    rows = torch.rand(T, generator=g) < share
+    k[0, rows, 64:] = 2.0 ** (62 if how == "dots" else 10)  # the unrotated half
+    q[0, :, 0, 64:] = 2.0 ** (62 if how == "dots" else 10)  # head 0: dot 2^130 (bf16 infinity) or 2^26
+    if how == "weights":
+        w[0, :, 0] *= 2.0 ** 105
+    print(f"[case] infinite scores {how} S={S} T={T} k={k_top} causal={causal} bf16={wbf}", flush=True)
+    _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, k_top, causal, start)
