@@ -429,10 +429,11 @@ __device__ __forceinline__ uint32_t row_scale(float upqn, float kns) {  // the s
 
 // The bound-emitting form (64 heads): per (query, key) a score S and a bound U with |exact score - S| <= U, for a
 // selection that computes exactly only the scores that can reach its top k.  No dot is certified here: with A the MFMA
-// sum of a dot, p = max(bf16(A), 0) is within one bf16 rounding of each side of the exact relu'd value r,
-//   |p - r| <= delta + 2^-8 |A| + 2^-8 (|A| + delta) <= 2^-7 (1 + 2^-7) p + (1 + 2^-7) delta      (delta: dot_halfwidth;
-// for A <= 0, p = 0 and r <= (1 + 2^-8) delta), so that
-//   S = sum_h w_h p_h,   U = c1 sum_h w_up p_h + sum_h w_up delta_h + c2 |S|,
+// sum of a dot, p = max(bf16(A), 0) is within one bf16 rounding of each side of the exact relu'd value r (at most 2^-8 of
+// the value, or, below 2^-126, half a step of 2^-133),
+//   |p - r| <= delta + 2^-8 |A| + 2^-8 (|A| + delta) + 2 2^-134 <= 2^-7 (1 + 2^-7) p + (1 + 2^-7) delta + 2^-132
+// (delta: dot_halfwidth; for A <= 0, p = 0 and r <= (1 + 2^-8) delta + 2^-134), so that
+//   S = sum_h w_h p_h,   U = c1 sum_h w_up p_h + sum_h w_up (delta_h + 2^-132) + c2 |S|,
 // w_up a bf16 value >= |w_h| (and >= 2^-110 where w_h != 0, so that the low part of a tiny weight, lost below the bf16
 // range, stays under 2^-24 w_up).  The head sums run on the MFMA too: p packs into the B operand as it is (lane (key, g)
 // holds the heads of k-slots 8 g .. + 7), and the A operand's rows hold w's high and low bf16 parts and w_up.  Products
@@ -519,7 +520,8 @@ __device__ __forceinline__ void bounded_scores(ScoresLdsBound<128, false> &L, co
   L.wf[wave][3][lane] = 0;
   const float dl = dot_halfwidth(qn_v, knm, bound_c);
   const bool forced = __builtin_amdgcn_ballot_w64(dl == __builtin_inff()) != 0ull;
-  const float dsum = wave_sum_f32(wp.up * dl) * 1.03125f;  // sum_h w_up delta_h, (1 + 2^-7) and the fp32 sums covered
+  // sum_h w_up (delta_h + 2^-132), (1 + 2^-7) and the fp32 sums covered
+  const float dsum = wave_sum_f32(wp.up * (dl + 0x1p-132f)) * 1.03125f;
   const uint32_t mrow = row_scale(wp.up * qn_v, kns);
 
   if constexpr (F8) {
@@ -663,9 +665,10 @@ __device__ __forceinline__ void bounded_scores_few(ScoresLdsBound<128, true> &L,
   L.wf[0][1][lane] = wp.lo;
   L.wf[0][2][lane] = wp.up16;
   L.wf[0][3][lane] = 0;
-  // sum_h w_up delta_h = bound_c 2^-23 (knm + pad) sum(w_up (qn + pad)) + 2^-144 sum(w_up), per group's knm
+  // sum_h w_up (delta_h + 2^-132) = bound_c 2^-23 (knm + pad) sum(w_up (qn + pad)) + (2^-144 + 2^-132) sum(w_up), per
+  // group's knm
   const float a1 = wave_sum_f32(wp.up * (qn_v + 0x1p-122f)) * bound_c * 0x1p-23f * 1.03125f;
-  const float a2 = wave_sum_f32(wp.up) * 0x1p-143f;
+  const float a2 = wave_sum_f32(wp.up) * 0x1.08p-132f;
   const float qpmax = wave_max_f32(qn_v) + 0x1p-122f;
   const uint32_t mrow = row_scale(wp.up * qn_v, kns);
   if (blockIdx.x == 0 && tid == 0) row_state[2 * row + 1] = mrow;

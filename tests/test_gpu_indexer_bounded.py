@@ -184,3 +184,20 @@ def test_infinite_scores(device, wbf, how, S, T, k_top, causal, start, share):
         w[0, :, 0] *= 2.0 ** 105
     print(f"[case] infinite scores {how} S={S} T={T} k={k_top} causal={causal} bf16={wbf}", flush=True)
     _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, k_top, causal, start)
+
+
+# dots in bf16's subnormal range under large weights, where a rounding moves a dot by a whole step however small it is: the
+# first columns' dots lie 2^-155 above a tie (5 steps, 4 by the MFMA sum), which beats the 4.5 steps of the next columns
+@pytest.mark.parametrize("wbf", [False, True])
+@pytest.mark.parametrize("S,T", [(3, 600), (20, 600), (2, 9000), (12, 2500)])
+def test_subnormal_dots_large_weights(device, wbf, S, T):
+    n = 100
+    q = torch.zeros(1, S, 64, 128)
+    k = torch.zeros(1, T, 128)
+    w = torch.full((1, S, 64), 2.0 ** -10)
+    q[0, :, 0, 64], q[0, :, 0, 65], q[0, :, 1, 66] = 2.0 ** -66, 2.0 ** -78, 2.0 ** -66
+    w[0, :, 0], w[0, :, 1] = 2.0 ** 40, 2.0 ** 39
+    k[0, 50:50 + n, 64], k[0, 50:50 + n, 65] = 4.5 * 2.0 ** -67, 2.0 ** -77
+    k[0, 300:300 + 2 * n, 64], k[0, 300:300 + 2 * n, 66] = 4.0 * 2.0 ** -67, 2.0 ** -67
+    print(f"[case] subnormal dots, large weights S={S} T={T} bf16={wbf}", flush=True)
+    _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, n, False, 0)
