@@ -346,7 +346,7 @@ inline ProjPlan proj_plan(int64_t N, int64_t C) {
 }  // namespace ks
 
 extern "C" size_t ks_mhc_input_workspace_size(int64_t N, int64_t C) {
-  if (N <= 0 || C <= 0) return 0;
+  if (N <= 0 || C < 8 || C % 8 != 0) return 0;  // sizes that ks_mhc_input refuses (or, N = 0, does nothing for)
   return static_cast<size_t>(ks::proj_plan(N, C).splits) * N * ks::kPartCols * sizeof(float);
 }
 

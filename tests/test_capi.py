@@ -48,6 +48,10 @@ def test_workspace_queries():
     # many queries -> one range per query -> no workspace
     assert lib.ks_sparse_attn_workspace_size(8, 2600, 64, 128, 128, 16) == 0
     assert lib.ks_sparse_attn_workspace_size(32, 1, 128, 576, 512, 2048) > 0
+    # sizes that ks_mhc_input refuses ask for nothing
+    for n, c in [(0, 64), (-1, 64), (4, 0), (4, 1), (4, 7), (4, 12), (4, -8)]:
+        assert lib.ks_mhc_input_workspace_size(n, c) == 0
+    assert lib.ks_mhc_input_workspace_size(1, 8) == 32 * 4 and lib.ks_mhc_input_workspace_size(1000, 4096) > 0
 
 
 def test_ops_refuse_cpu_tensors():
