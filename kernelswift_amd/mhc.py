@@ -47,7 +47,12 @@ class HyperConnection(nn.Module):
 
     def _fused(self, x: torch.Tensor) -> bool:
         """Whether `pre` may form the logits inside the kernel: plain contiguous tensors of the kernel's types on one
-        GPU, with no gradient (reverse or forward mode), autocast, vmap or trace that has to see the torch operations."""
+        GPU, with no gradient (reverse or forward mode), autocast, vmap or trace that has to see the torch operations,
+        and no `logits` of a subclass's or the instance's own."""
+        if type(self).logits is not HyperConnection.logits or "logits" in self.__dict__:
+            return False
+        if not isinstance(self.norm_eps, (int, float)):
+            return False
         ts = (x, self.phi, self.alpha, self.base)
         if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.maybe_current_level() is not None:
             return False

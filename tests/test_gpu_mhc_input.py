@@ -90,6 +90,28 @@ def test_block_with_and_without_gradients(device):
             assert not hc._fused(x)
 
 
+def test_own_logits_are_used(device):
+    class Shifted(HyperConnection):
+        def logits(self, x):
+            pre, post, res = super().logits(x)
+            return pre + 1.0, post + 2.0, res + 3.0
+
+    x = torch.randn(20, 4, 128, generator=torch.Generator().manual_seed(1)).bfloat16().to(device)
+    plain = _block(device, 128, 6)
+    own = Shifted(128).to(device).requires_grad_(False)
+    own.load_state_dict(plain.state_dict())
+    patched = _block(device, 128, 6)
+    patched.logits = lambda x: Shifted.logits(own, x)
+    with torch.no_grad():
+        _, post, res = plain.pre(x)
+        want = _lib.torch_ops().mhc_pre(x, own.logits(x)[0])
+        for hc in (own, patched):
+            h, p, r = hc.pre(x)
+            assert torch.equal(h, want)
+            torch.testing.assert_close(p, post + 2.0, rtol=1e-5, atol=1e-5)
+            torch.testing.assert_close(r, res + 3.0, rtol=1e-5, atol=1e-5)
+
+
 def test_mhc_input_errors(device):
     hc = _block(device, 64, 4)
     x = torch.zeros(2, 4, 64, dtype=torch.bfloat16, device=device)
