@@ -284,10 +284,28 @@ __global__ __launch_bounds__(64 * kProjWaves, TT == 4 ? 2 : 3) void mhc_proj_ker
   }
 }
 
+// x phi of one token with x normalised first, for the tokens whose products of plain values leave the fp32 range (values
+// past 2^60 or so against large weights): one wave, lane c < 24 receives column c.  Rare, so written for few registers.
+__device__ float normalised_product(const uint16_t *__restrict__ x, const float *__restrict__ phi, float rn, int64_t K,
+                                    int lane) {
+  float z = 0.f;
+#pragma unroll 1
+  for (int c = 0; c < kLogits; ++c) {
+    float acc = 0.f;
+#pragma unroll 1
+    for (int64_t k = lane; k < K; k += 64) acc = __builtin_fmaf(bf16_to_f32(x[k]) * rn, phi[k * kLogits + c], acc);
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) acc += __shfl_xor(acc, m, 64);
+    z = lane == c ? acc : z;
+  }
+  return z;
+}
+
 // The logits from the partials, then h as mhc_pre_kernel: one wave per token.  post and res logits are stored for
 // the residual update.
 __global__ __launch_bounds__(64 * kMhcWaves) void mhc_input_kernel(const uint16_t *__restrict__ x,
                                                                   const float *__restrict__ part,
+                                                                  const float *__restrict__ phi,
                                                                   const float *__restrict__ alpha,
                                                                   const float *__restrict__ base,
                                                                   uint16_t *__restrict__ h, float *__restrict__ post,
@@ -306,7 +324,11 @@ __global__ __launch_bounds__(64 * kMhcWaves) void mhc_input_kernel(const uint16_
   z += __builtin_bit_cast(float, lane_xor<32>(__builtin_bit_cast(uint32_t, z)));
   const float ss = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, z), kLogits));
   const float rn = 1.0f / sqrtf(ss / static_cast<float>(C8 * 32) + norm_eps);
-  const float lg = al * (z * rn) + bs;
+  float zn = z * rn;
+  // a product or the sum of squares past the fp32 range (uniform; not finite on any of the 25 lanes)
+  if (__builtin_amdgcn_ballot_w64(lane <= kLogits && !(fabsf(z) < __builtin_inff())) != 0ull)
+    zn = normalised_product(x + t * kMhcN * C8 * 8, phi, rn, C8 * 32, lane);
+  const float lg = al * zn + bs;
   if (lane >= 4 && lane < 8) post[t * 4 + lane - 4] = lg;
   if (lane >= 8 && lane < kLogits) res[t * 16 + lane - 8] = lg;
   const float gate = sigmoid(lg);
@@ -379,7 +401,7 @@ extern "C" int ks_mhc_input(const uint16_t *x, const float *phi, const float *al
     hipLaunchKernelGGL(ks::mhc_proj_kernel<4>, grid, block, 0, st, x, phi, part, N, 4 * C, p.splits, p.steps);
   KS_CHECK_LAUNCH("mhc_proj_kernel");
   hipLaunchKernelGGL(ks::mhc_input_kernel, dim3(static_cast<unsigned>(ks::ceil_div(N, ks::kMhcWaves))),
-                     dim3(64 * ks::kMhcWaves), 0, st, x, part, alpha, base, h, post_logits, res_logits, N, C / 8,
+                     dim3(64 * ks::kMhcWaves), 0, st, x, part, phi, alpha, base, h, post_logits, res_logits, N, C / 8,
                      p.splits, norm_eps);
   KS_CHECK_LAUNCH("mhc_input_kernel");
   return KS_OK;

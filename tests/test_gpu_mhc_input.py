@@ -70,6 +70,30 @@ def test_mhc_input_special_values(device):
     torch.testing.assert_close(res, res_t, rtol=1e-5, atol=1e-4)
 
 
+# products of the plain streams past the fp32 range where those of the normalised streams are not: streams past the square
+# root of the range (their RMS is infinite, so they normalise to zero), large weights, some tokens only
+def test_mhc_input_large_values(device):
+    C = 264
+    hc = _block(device, C, 5)
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(40, 4, C, generator=g)
+    x[3] *= 2.0 ** 125
+    x[17] = 2.0 ** 127
+    x[30] *= 2.0 ** 50
+    x[33] *= 2.0 ** 66
+    x = x.bfloat16().to(device)
+    for scale in (1.0, 64.0, 2.0 ** 90):
+        hc.phi.copy_((torch.randn(4 * C, 24, generator=g) * ((4 * C) ** -0.5 * scale)).to(device))
+        hc.alpha.fill_(1.0 / scale)
+        print(f"[case] mhc_input large values scale={scale}", flush=True)
+        h, post, res = _lib.torch_ops().mhc_input(x, hc.phi, hc.alpha, hc.base, hc.norm_eps)
+        pre_t, post_t, res_t = hc.logits(x)
+        assert torch.isfinite(post_t).all() and torch.isfinite(res_t).all()
+        torch.testing.assert_close(post, post_t, rtol=1e-5, atol=1e-4)
+        torch.testing.assert_close(res, res_t, rtol=1e-5, atol=1e-4)
+        assert torch.equal(post[17], hc.base[4:8])
+
+
 def test_block_with_and_without_gradients(device):
     # with gradients the logits stay torch operations, and phi receives its gradient
     hc = _block(device, 512, 3)
