@@ -378,7 +378,7 @@ extern "C" int ks_mhc_input(const uint16_t *x, const float *phi, const float *al
   ks::last_error().clear();
   int rc = ks::check_mhc(x, N, C, "ks_mhc_input");
   if (rc != KS_OK) return rc;
-  KS_CHECK_ARG(C < (int64_t(1) << 28), "ks_mhc_input: C=%lld out of range", (long long)C);
+  KS_CHECK_ARG(C < (int64_t(1) << 32), "ks_mhc_input: C=%lld out of range", (long long)C);  // 32-bit step counts
   if (N == 0) return KS_OK;
   KS_CHECK_ARG(phi && alpha && base && h && post_logits && res_logits, "ks_mhc_input: null pointer");
   KS_CHECK_ARG(ks::aligned(x, 16) && ks::aligned(h, 16) && ks::aligned(phi, 4) && ks::aligned(alpha, 4) &&

@@ -42,6 +42,15 @@ def test_host_validation_without_gpu():
     assert lib.ks_rope_inplace(None, None, 1, 1, 1, 128, 4, 64, 0, 10, None) == 1
 
 
+def test_mhc_input_takes_the_widths_of_mhc_pre():
+    # a width that ks_mhc_pre takes gets past the range check (to the null pointers)
+    lib = _lib.load()
+    x = ctypes.c_void_p(4096)
+    for C in (8, 4096, 1 << 28, (1 << 32) - 8):
+        assert lib.ks_mhc_input(x, None, None, None, None, None, None, 1, C, 1e-6, None, 0, None) == 1
+        assert b"null pointer" in lib.ks_last_error(), C
+
+
 def test_workspace_queries():
     lib = _lib.load()
     assert lib.ks_indexer_workspace_size(1, 128, 64, 128, 4096) >= 128 * 4096 * 4  # the fp32 score matrix
