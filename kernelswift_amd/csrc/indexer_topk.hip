@@ -645,7 +645,12 @@ inline SelPlan sel_plan(int64_t rows, int T) {
   return p;
 }
 
-// The selection's regions in its workspace of 64-bit slots: the segments' lists (kRecThreads kpb composites each), the
+// A segment's list, slot i: the composite (key, ~column).  Rows of at most kTopkSelfCount columns, whose scores and bounds
+// every segment's workgroup counts, keep the lists packed in the workspace; longer rows, counted by a launch before, keep
+// them over the segment's own scores (the keys) and bounds (the complemented columns), which no other workgroup reads any
+// more: a row of 32768 columns would otherwise need 256 KiB more workspace (64 queries x 32768 keys: 83.2 -> 83.5 us by the
+// second load of every slot; 4096 columns, 40 us, would pay 0.7 us, which is why short rows' lists stay packed).
+// The selection's regions in its workspace of 64-bit slots: the packed lists (kRecThreads kpb composites each), the
 // slices' bucket counts (2048 x 32 bits each), the segments' states (slots used, largest key) and the rows' (tau, the
 // histogram scale).
 struct SelRegions {
@@ -657,7 +662,8 @@ struct SelRegions {
 inline SelRegions sel_regions(uint64_t *part, int64_t rows, const SelPlan &p) {
   SelRegions r{};
   // one segment of two columns per thread: ranked by the recomputation, no lists
-  const int64_t nl = p.segs == 1 && p.kpb == 2 ? 0 : rows * p.segs * kRecThreads * p.kpb, nh = rows * p.NP * 1024, ns = rows * p.segs;
+  const int64_t nl = (p.segs == 1 && p.kpb == 2) || p.NP > 0 ? 0 : rows * p.segs * kRecThreads * p.kpb;
+  const int64_t nh = rows * p.NP * 1024, ns = rows * p.segs;
   r.slots = nl + nh + ns + rows;
   r.lists = part;
   r.hists = reinterpret_cast<uint32_t *>(part + nl);
@@ -1105,11 +1111,11 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 
 // Workgroup (row, segment) of kRecThreads lanes over columns [c0, c0 + SW) of the row's valid prefix, SW =
 // kRecThreads KPB (column c0 + j kRecThreads + tid in slot j of thread tid):
-//  - tau: the row's bucket counts (NP slices of them summed, or, with NP = 0, counted here from the whole row's scores;
+//  - tau: the row's bucket counts (kRecLong: NP slices of them summed; else counted here from the whole row's scores;
 //    thread t owns the kBPT buckets below 2048 - kBPT t), a block scan from the top bucket finds the bucket holding the
 //    row's k-th largest lower end; tau is its lower edge;
-//  - recomputation of the scores whose upper end reaches tau (recompute_scores); the scores and bounds in memory stay as
-//    they are, since the workgroups of the row's other segments may still be counting them;
+//  - recomputation of the scores whose upper end reaches tau (recompute_scores); but for kRecLong the scores and bounds in
+//    memory stay as they are, since the workgroups of the row's other segments may still be counting them;
 //  - these columns fill the segment's list, in column-slot order: the exact key of each, or 0 where the exact score
 //    fell below tau; the segment's state receives the number of slots and an upper bound of the largest key (the
 //    largest upper end), the row's state tau.
@@ -1120,7 +1126,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_hist_kernel(const flo
 // the score launch at that shape).
 // MODE kRecAllRope: every query row meets one workgroup then, which also rotates it, scales its head weights and forms its
 // statistics on the way into LDS (the pass of its own, 98 MB in and out at that shape: 36 us; the call 349 -> 333 us).
-constexpr int kRecLists = 0, kRecOneSeg = 1, kRecAll = 2, kRecAllRope = 3;
+// MODE kRecLong: lists for rows counted by topk_slice_hist_kernel (NP slices), over the segment's scores and bounds.
+constexpr int kRecLists = 0, kRecOneSeg = 1, kRecAll = 2, kRecAllRope = 3, kRecLong = 4;
 struct RecOut {  // the output of the one-segment modes
   void *out;
   int64_t offset;
@@ -1135,14 +1142,15 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
                                                                     uint2 *__restrict__ sstate,
                                                                     uint2 *__restrict__ rstate) {
   constexpr int SW = kRecThreads * KPB;
-  constexpr bool kAll = MODE >= kRecAll, kRope = MODE == kRecAllRope;
+  constexpr bool kAll = MODE == kRecAll || MODE == kRecAllRope, kRope = MODE == kRecAllRope;
+  constexpr bool kLong = MODE == kRecLong, kLists = MODE == kRecLists || kLong;
   __shared__ RecShared rs;
   __shared__ RecWave rw[kRecWaves];
   __shared__ int32_t list[SW];
   __shared__ uint32_t wsum[kRecWaves];
   __shared__ uint32_t s_tau, s_unc, s_max[kRecWaves];
   __shared__ uint16_t unc[WBF ? SW : 2];  // list positions that certify_scores left open
-  // the row's counts (NP = 0) share the LDS of the recomputation's scratch, which they precede
+  // the row's counts share the LDS of the recomputation's scratch, which they precede
   static_assert(sizeof(RecWave) * kRecWaves >= 2048 * sizeof(uint32_t), "bucket counts fit");
   uint32_t *hist = reinterpret_cast<uint32_t *>(rw);
   // workgroups are dealt to the 8 XCDs round-robin (block id mod 8): the segments of one row are placed on one
@@ -1161,7 +1169,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   const int k_row = k < n_valid ? k : n_valid;
   const int c0 = seg * SW;
   const int nv = n_valid - c0 <= 0 ? 0 : (n_valid - c0 < SW ? n_valid - c0 : SW);
-  if constexpr (MODE != kRecLists) {
+  if constexpr (!kLists) {
     // masked tail: fewer valid columns than k (the -inf ties, in ascending column order)
     const int64_t lim = causal ? (start_pos + s + 1) / ratio : INT64_MAX;
     for (int j = k_row + tid; j < k; j += kRecThreads)
@@ -1199,7 +1207,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   }
   static_assert(kBPT == 4, "one 16-byte read of a slice's buckets per thread");
   uint4 hv0 = make_uint4(0, 0, 0, 0), hv1 = hv0, hv2 = hv0, hv3 = hv0;
-  if (NP > 0) {  // uniform; slice 0 stands in for the slices past NP
+  if constexpr (kLong) {  // slice 0 stands in for the slices past NP
     const uint32_t *hr = hists + row * NP * 2048 + (2048 - kBPT * (tid + 1));
     auto slice = [&](int p) { return *reinterpret_cast<const uint4 *>(hr + (p < NP ? p : 0) * 2048); };
     static_assert(kTopkMaxSlices == 4, "four slices");
@@ -1252,7 +1260,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     for (int i = tid; i < nv; i += kRecThreads) list[i] = i;
   } else {
     // ---- tau: bucket e of the thread's kBPT is 2048 - kBPT (tid + 1) + e (the top one is e = kBPT - 1)
-    if (NP == 0) {  // uniform
+    if constexpr (!kLong) {
       reinterpret_cast<uint4 *>(hist)[tid] = make_uint4(0, 0, 0, 0);
       __syncthreads();
       // eight columns per thread at a time, their loads in flight together
@@ -1305,7 +1313,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     }
     __syncthreads();
     tau = s_tau;
-    if (MODE == kRecLists && seg == 0 && tid == 0) rstate[row].x = tau;
+    if (kLists && seg == 0 && tid == 0) rstate[row].x = tau;
 
     // ---- the segment's candidates: every column whose upper end reaches tau, with U > 0 (a score with U = 0 is exact
     // already and takes its slot as it is); one block scan counts candidates (low 16 bits) and slots (high 16)
@@ -1348,7 +1356,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     recompute_scores<kRecWaves, F8, WBF>(list, unc, nrec, rc, rs, rw[tid >> 6], kbrow0, b * rc.kns, qpmax, n_exact,
                                          n_unres);
   }
-  if constexpr (MODE == kRecLists) {
+  if constexpr (kLists) {
     uint32_t umax = 0, unused = 0;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) umax = ((masks >> (8 + j)) & 1u) && hik[j] > umax ? hik[j] : umax;
@@ -1357,7 +1365,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   }
   __syncthreads();  // every recomputed score is in its list slot
   const int64_t sg = row * segs + seg;
-  if (MODE == kRecLists && tid == 0) {
+  if (kLists && tid == 0) {
     uint32_t m = s_max[0];
 #pragma unroll
     for (int w = 1; w < kRecWaves; ++w) m = s_max[w] > m ? s_max[w] : m;
@@ -1370,7 +1378,7 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   }
 
   const float *listf = reinterpret_cast<const float *>(list);
-  if constexpr (MODE != kRecLists) {
+  if constexpr (!kLists) {
     // ---- ranks of the exact keys (at most two per thread) and the store
     uint64_t v[KPB];
     uint32_t p = bexcl & 0xFFFFu, kmax = 0, kmin = 0;  // kmin: complement of the smallest key
@@ -1417,7 +1425,10 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     }
   } else {
     // ---- the segment's slots: the exact key, or 0 where a recomputed score fell below tau
-    uint64_t *dst = lists + sg * SW;
+    uint64_t *dst = kLong ? nullptr : lists + sg * SW;
+    // (kLong: every score of the segment is in registers since before the barriers above)
+    uint32_t *dk = reinterpret_cast<uint32_t *>(const_cast<float *>(srow)) + c0;
+    uint32_t *dc = reinterpret_cast<uint32_t *>(rc.bounds + row * ld) + c0;
     uint32_t pos = bexcl >> 16, p = bexcl & 0xFFFFu;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) {
@@ -1427,7 +1438,12 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
         p += cj ? 1u : 0u;
         if (key < tau) key = 0u;
         const uint32_t col = static_cast<uint32_t>(c0 + j * kRecThreads + tid);
-        dst[pos++] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
+        if constexpr (kLong) {
+          dk[pos] = key;
+          dc[pos++] = ~col;
+        } else {
+          dst[pos++] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~col);
+        }
       }
     }
   }
@@ -1436,10 +1452,10 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
 // One workgroup per row: the lists of the row's segments (together every column of its top k, each with its exact score;
 // at least k_sel entries) sorted, and the first k_sel stored with the post-processing.  2^tpl = 1024 / (the power of two
 // >= segs) threads read a segment's list; a list longer than those threads hold is first gathered in LDS.  More entries
-// than LDS takes (cap) fall back to the exact selection over the row's keys, spread by column into the row of the bounds
-// (which no launch reads any more).
+// than LDS takes (cap) fall back to the exact selection over the row's keys, spread by column into the row of the bounds, a
+// segment at a time (its list, which may lie there, holds only columns of its own).
 template <int KPT>
-__global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *keys, int64_t ld, int64_t S, int T, int k, int causal,
+__global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(const uint32_t *scores, uint32_t *bounds, int64_t ld, int64_t S, int T, int k, int causal,
                                                                      int64_t start_pos, int ratio, int64_t offset,
                                                                      void *__restrict__ out, int out_i64,
                                                                      const uint64_t *__restrict__ lists, int cap,
@@ -1466,14 +1482,24 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
     const uint2 ss = sstate[row * segs + (lane < nseg ? lane : 0)];
     const uint32_t tau = rstate[row].x;
     const int tps = 1 << tpl, seg = tid >> tpl, i0 = tid & (tps - 1);
-    const uint64_t *src = lists + (row * segs + (seg < nseg ? seg : 0)) * static_cast<int64_t>(SW);
+    constexpr bool kPacked = KPT * kTopkThreads <= kTopkSelfCount;
+    auto entry = [&](int g, uint32_t i) {  // slot i of segment g
+      if constexpr (kPacked) {
+        return lists[(row * segs + g) * static_cast<int64_t>(SW) + i];
+      } else {
+        const int64_t at = row * ld + static_cast<int64_t>(g) * SW + i;
+        return (static_cast<uint64_t>(scores[at]) << 32) | static_cast<uint64_t>(bounds[at]);
+      }
+    };
+    const int rseg = seg < nseg ? seg : 0;
+    const uint32_t room = static_cast<uint32_t>(kPacked ? SW : min(SW, T - rseg * SW));  // slots of its list
     constexpr int kMaxPer = kTopkListCap / kTopkThreads;
     uint64_t v[kMaxPer];
 #pragma unroll
     for (int j = 0; j < kMaxPer; ++j) {
-      const int i = j * tps + i0;
+      const uint32_t i = static_cast<uint32_t>(j * tps + i0);
       v[j] = 0;
-      if (j < spec) v[j] = src[i < SW ? i : 0];  // uniform
+      if (j < spec) v[j] = entry(rseg, i < room ? i : 0u);  // uniform
     }
     const uint32_t c = lane < nseg ? ss.x : 0u;
     const uint32_t incl = wave_incl_scan(c);
@@ -1484,8 +1510,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
     auto gather = [&]() {  // the lists one after the other in LDS
       for (int g = tid >> 6; g < nseg; g += kTopkWaves) {
         const uint32_t len = __shfl(c, g, 64), at = __shfl(incl, g, 64) - len;
-        const uint64_t *gs = lists + (row * segs + g) * static_cast<int64_t>(SW);
-        for (uint32_t i = lane; i < len; i += 64) cand[at + i] = gs[i];
+        for (uint32_t i = lane; i < len; i += 64) cand[at + i] = entry(g, i);
       }
       __syncthreads();
     };
@@ -1494,7 +1519,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
 #pragma unroll
         for (int j = 0; j < kMaxPer; ++j) {
           const uint32_t i = static_cast<uint32_t>(j * tps + i0);
-          if (j >= spec && static_cast<uint32_t>(j * tps) < most) v[j] = src[i < static_cast<uint32_t>(SW) ? i : 0];  // uniform
+          if (j >= spec && static_cast<uint32_t>(j * tps) < most) v[j] = entry(rseg, i < room ? i : 0u);  // uniform
           if (i >= mine || seg >= nseg) v[j] = 0;
         }
       } else {
@@ -1538,18 +1563,23 @@ __global__ __launch_bounds__(kTopkThreads) void topk_collected_kernel(uint32_t *
         sort_merge_store(cand, P, static_cast<int>(n), k_sel, row, k, out, out_i64, causal, limit, offset, nullptr);
       }
     } else {
-      uint32_t *kr = keys + row * ld;
-      for (int i = tid; i < n_valid; i += kTopkThreads) kr[i] = 0u;
-      __syncthreads();
-      for (int g = tid >> 6; g < nseg; g += kTopkWaves) {
-        const uint32_t len = __shfl(c, g, 64);
-        const uint64_t *gs = lists + (row * segs + g) * static_cast<int64_t>(SW);
-        for (uint32_t i = lane; i < len; i += 64) {
-          const uint64_t e = gs[i];
-          kr[~static_cast<uint32_t>(e)] = static_cast<uint32_t>(e >> 32);
+      uint32_t *kr = bounds + row * ld;
+      constexpr int kMaxSeg = kRecThreads * 8 / kTopkThreads;  // entries of a segment per thread, at most
+      for (int g = 0; g < nseg; ++g) {
+        const uint32_t len = __builtin_amdgcn_readlane(c, g);
+        uint64_t e[kMaxSeg];
+#pragma unroll
+        for (int j = 0; j < kMaxSeg; ++j) {
+          const uint32_t i = static_cast<uint32_t>(j * kTopkThreads + tid);
+          e[j] = i < len ? entry(g, i) : 0ull;
         }
+        __syncthreads();
+        for (int i = g * SW + tid; i < min((g + 1) * SW, n_valid); i += kTopkThreads) kr[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kMaxSeg; ++j)
+          if (e[j] != 0ull) kr[~static_cast<uint32_t>(e[j])] = static_cast<uint32_t>(e[j] >> 32);
       }
-      __threadfence_block();
       __syncthreads();
       uint32_t key[KPT];
 #pragma unroll
@@ -1667,6 +1697,9 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
     }
     if (all) rec(topk_recompute_kernel<2, f, wb, kRecAll>);
     else if (one) rec(topk_recompute_kernel<2, f, wb, kRecOneSeg>);
+    else if (NP > 0 && kpb == 2) rec(topk_recompute_kernel<2, f, wb, kRecLong>);
+    else if (NP > 0 && kpb == 4) rec(topk_recompute_kernel<4, f, wb, kRecLong>);
+    else if (NP > 0) rec(topk_recompute_kernel<8, f, wb, kRecLong>);
     else if (kpb == 2) rec(topk_recompute_kernel<2, f, wb, kRecLists>);
     else if (kpb == 4) rec(topk_recompute_kernel<4, f, wb, kRecLists>);
     else rec(topk_recompute_kernel<8, f, wb, kRecLists>);
@@ -1689,7 +1722,7 @@ int ks::launch_indexer_topk_bounded(float *scores, int64_t ld, int64_t B, int64_
   const int spec = static_cast<int>(share < kRecThreads * kpb ? ceil_div(share, tps) : ceil_div(kRecThreads * kpb, tps));
 #define KS_COLL(KPT_)                                                                                                \
   hipLaunchKernelGGL(topk_collected_kernel<KPT_>, dim3(static_cast<unsigned>(rows)), dim3(kTopkThreads), shmem, st, \
-                     reinterpret_cast<uint32_t *>(rc.bounds), ld, S, Ti, ki, c, start_pos, ratio, offset, out, o,    \
+                     reinterpret_cast<uint32_t *>(scores), reinterpret_cast<uint32_t *>(rc.bounds), ld, S, Ti, ki, c, start_pos, ratio, offset, out, o,    \
                      rg.lists, cap, spec, segs, kRecThreads * kpb, tpl, rg.sstate,                                  \
                      rg.rstate)
   if (Ti <= 1024) KS_COLL(1);

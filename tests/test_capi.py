@@ -63,6 +63,14 @@ def test_workspace_queries():
     assert lib.ks_mhc_input_workspace_size(1, 8) == 32 * 4 and lib.ks_mhc_input_workspace_size(1000, 4096) > 0
 
 
+def test_bounded_selection_workspace_is_bounded():
+    # beside the scores and bounds a row needs at most 8192 list slots, or four slices' bucket counts
+    lib = _lib.load()
+    for rows in (1, 3, 64, 255, 256, 2048, 100000):
+        for T in (1, 300, 1024, 1025, 4096, 5000, 8191, 8192, 8193, 12000, 16382, 20000, 32768):
+            assert 0 < lib.ks_dbg_topk_bounded_slots(rows, T) <= rows * (8192 + 64), (rows, T)
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     from kernelswift_amd import ops

@@ -201,3 +201,25 @@ def test_subnormal_dots_large_weights(device, wbf, S, T):
     k[0, 300:300 + 2 * n, 64], k[0, 300:300 + 2 * n, 66] = 4.0 * 2.0 ** -67, 2.0 ** -67
     print(f"[case] subnormal dots, large weights S={S} T={T} bf16={wbf}", flush=True)
     _check(device, q.bfloat16(), k.bfloat16(), w.bfloat16() if wbf else w, n, False, 0)
+
+
+# more tied scores than the ranking takes in LDS: the whole-row selection over the lists, in the workspace (at most 8192
+# columns) and over the rows' own scores and bounds (more); a ragged last segment, causal prefixes inside a segment
+@pytest.mark.parametrize("S,T,k_top,causal,start", [
+    (5, 8192, 700, False, 0), (6, 9001, 2048, False, 0), (5, 20000, 1000, True, 17300), (3, 32768, 2048, False, 0),
+    (300, 8200, 64, False, 0)])
+def test_long_lists_of_ties(device, S, T, k_top, causal, start):
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(1, S, 64, 128, generator=g).abs().bfloat16()
+    k = torch.randn(1, T, 128, generator=g)
+    tied = torch.rand(T, generator=g) < 0.7
+    k[0, tied] = torch.randn(1, 128, generator=g).abs() * 3  # ahead of most others
+    k[0, :, :64] = 0.0                                       # nothing that the rotation changes
+    w = torch.rand(1, S, 64, generator=g) / 8
+    rows = slice(0, 6)
+    print(f"[case] long lists of ties S={S} T={T} k={k_top} causal={causal}", flush=True)
+    tab = workloads.freqs_table(64, T + 1)
+    k = k.bfloat16()
+    got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), k_top, causal, start, 1, 0, 0, 64, True)
+    want = oracle.indexer(_u16(q[:, rows]), _u16(k), w[:, rows].numpy(), tab.numpy(), k_top, causal, start, 1, 0, 0, 64, True)
+    np.testing.assert_array_equal(got[:, rows].cpu().numpy().astype(np.int64), want)
