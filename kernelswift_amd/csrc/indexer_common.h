@@ -17,13 +17,13 @@ __device__ __forceinline__ uint32_t score_key(float f) {
 // row's scores rarely exceed; any value is correct): positive values 1024 .. 2047, negative ones 1023 .. 0, larger
 // magnitudes clamped to the outermost bucket, smaller ones to the two middle ones.  The key's own top bits would give
 // 4 buckets per octave in 11 bits, which at N(0, 1) inputs puts a tenth more keys above the threshold.
-__device__ __forceinline__ uint32_t bound_digit(float lo, uint32_t M) {
+__host__ __device__ __forceinline__ uint32_t bound_digit(float lo, uint32_t M) {
   const uint32_t u = __builtin_bit_cast(uint32_t, lo), m = u & 0x7FFFFFFFu;
-  const uint32_t d = min(M > m ? (M - m) >> 17 : 0u, 1023u);
+  const uint32_t b = M > m ? (M - m) >> 17 : 0u, d = b < 1023u ? b : 1023u;
   return (u >> 31) ? d : 2047u - d;
 }
 // The smallest nonzero key that a value of bucket d can have (so that no value of bucket d or above lies below it).
-__device__ __forceinline__ uint32_t bound_digit_edge(uint32_t d, uint32_t M) {
+__host__ __device__ __forceinline__ uint32_t bound_digit_edge(uint32_t d, uint32_t M) {
   if (d >= 1024u) {  // m > M - ((dd + 1) << 17), or any m down to zero in the last bucket
     const uint32_t dd = 2047u - d, low = (dd + 1u) << 17;
     return 0x80000000u | (dd < 1023u && M >= low ? M - low + 1u : 0u);

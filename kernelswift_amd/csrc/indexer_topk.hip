@@ -1785,6 +1785,13 @@ extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const f
 
 extern "C" int64_t ks_dbg_topk_bounded_slots(int64_t rows, int64_t T) { return ks::topk_bounded_part_capacity(rows, T); }
 
+// The threshold histogram's buckets of n values at row scale M, and the edges of the 2048 buckets, on the host (the device's
+// own functions).
+extern "C" void ks_dbg_bound_digits(const float *x, int64_t n, uint32_t M, uint32_t *digits, uint32_t *edges) {
+  for (int64_t i = 0; i < n; ++i) digits[i] = ks::bound_digit(x[i], M);
+  for (uint32_t d = 0; d < 2048u; ++d) edges[d] = ks::bound_digit_edge(d, M);
+}
+
 // The rank buckets of n keys over [kmin, kmax], on the host (the device's own functions).
 extern "C" void ks_dbg_rank_buckets(const uint32_t *keys, int64_t n, uint32_t kmin, uint32_t kmax, uint32_t *out) {
   const ks::RankScale rk(kmin, kmax);
