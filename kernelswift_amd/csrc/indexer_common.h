@@ -362,7 +362,7 @@ int launch_indexer_scores(const uint16_t *q, const uint16_t *k, const void *w, i
 // (64 heads, D = 128), w [B, S, 64]; with kc / ks set, the keys are e4m3 codes and row scales (the statistics
 // those of the dequantised rows), read directly and dequantised in registers.
 struct TopkRecompute {
-  float *bounds;  // overwritten where a row's list outgrows LDS
+  float *bounds;  // overwritten: lists of rows past 8192 columns, and where a row's lists outgrow LDS
   const uint16_t *q;
   const uint16_t *k;
   const void *w;  // fp32, or bf16 (w_bf16)

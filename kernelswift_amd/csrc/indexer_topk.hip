@@ -1253,8 +1253,8 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   if constexpr (!kRope) query_max(qnv);
 
   if (tid == 0) s_unc = 0u;
-  uint32_t hik[KPB], masks = 0;  // bit j: column j is a candidate; bit 8 + j: it has a slot
-  uint32_t tau = 1u, ncand = 0, nres = 0, bexcl = 0;
+  uint32_t masks = 0;  // bit j: column j is a candidate
+  uint32_t tau = 1u, ncand = 0, bexcl = 0;
   if constexpr (kAll) {
     ncand = static_cast<uint32_t>(nv);
     for (int i = tid; i < nv; i += kRecThreads) list[i] = i;
@@ -1315,28 +1315,27 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     tau = s_tau;
     if (kLists && seg == 0 && tid == 0) rstate[row].x = tau;
 
-    // ---- the segment's candidates: every column whose upper end reaches tau, with U > 0 (a score with U = 0 is exact
-    // already and takes its slot as it is); one block scan counts candidates (low 16 bits) and slots (high 16)
-    // (few registers stay live across the recomputation: the masks share one word, the bases another, and the
-    // largest upper end is taken from hik afterwards)
+    // ---- the segment's candidates: every column whose upper end reaches tau (no bound is zero, so each of them is
+    // recomputed and takes a slot); a block scan gives their places, and the largest upper end bounds the segment's keys
     static_assert(KPB <= 8, "masks of up to 8 columns per thread");
+    uint32_t umax = 0;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) {
-      const bool v = j * kRecThreads + tid < nv;
-      const uint32_t lo = score_key(uv[j] > 0.f ? sv[j] - uv[j] : sv[j]);
-      hik[j] = v ? score_key(uv[j] > 0.f ? sv[j] + uv[j] : sv[j]) : 0u;
-      if (v && hik[j] >= tau) masks |= (lo != hik[j] ? 0x101u : 0x100u) << j;
+      const uint32_t hi = j * kRecThreads + tid < nv ? score_key(sv[j] + uv[j]) : 0u;
+      if (hi >= tau) masks |= 1u << j;  // tau > 0
+      umax = hi > umax ? hi : umax;
     }
-    static_assert(SW < 65536, "candidate and slot counts share a 32-bit scan");
-    const uint32_t both = __builtin_popcount(masks & 0xFFu) | (__builtin_popcount(masks >> 8) << 16);
-    bexcl = block_inclusive_scan<true, kRecWaves>(both, wsum) - both;  // slots << 16 | candidates
+    if constexpr (kLists) {
+      uint32_t unused = 0;
+      wave_max2(unused, umax);
+      if ((tid & 63) == 0) s_max[tid >> 6] = umax;
+    }
+    const uint32_t mc = __builtin_popcount(masks);
+    bexcl = block_inclusive_scan<true, kRecWaves>(mc, wsum) - mc;
 #pragma unroll
-    for (int w = 0; w < kRecWaves; ++w) {
-      ncand += wsum[w] & 0xFFFFu;
-      nres += wsum[w] >> 16;
-    }
+    for (int w = 0; w < kRecWaves; ++w) ncand += wsum[w];
     {
-      uint32_t p = bexcl & 0xFFFFu;
+      uint32_t p = bexcl;
 #pragma unroll
       for (int j = 0; j < KPB; ++j)
         if ((masks >> j) & 1u) list[p++] = c0 + j * kRecThreads + tid;
@@ -1356,20 +1355,13 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     recompute_scores<kRecWaves, F8, WBF>(list, unc, nrec, rc, rs, rw[tid >> 6], kbrow0, b * rc.kns, qpmax, n_exact,
                                          n_unres);
   }
-  if constexpr (kLists) {
-    uint32_t umax = 0, unused = 0;
-#pragma unroll
-    for (int j = 0; j < KPB; ++j) umax = ((masks >> (8 + j)) & 1u) && hik[j] > umax ? hik[j] : umax;
-    wave_max2(unused, umax);
-    if ((tid & 63) == 0) s_max[tid >> 6] = umax;
-  }
   __syncthreads();  // every recomputed score is in its list slot
   const int64_t sg = row * segs + seg;
   if (kLists && tid == 0) {
     uint32_t m = s_max[0];
 #pragma unroll
     for (int w = 1; w < kRecWaves; ++w) m = s_max[w] > m ? s_max[w] : m;
-    sstate[sg] = make_uint2(nres, m);
+    sstate[sg] = make_uint2(ncand, m);
   }
   if (rc.stats != nullptr) {
     if (n_exact) atomicAdd(&rc.stats[0], n_exact);
@@ -1381,17 +1373,15 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
   if constexpr (!kLists) {
     // ---- ranks of the exact keys (at most two per thread) and the store
     uint64_t v[KPB];
-    uint32_t p = bexcl & 0xFFFFu, kmax = 0, kmin = 0;  // kmin: complement of the smallest key
+    uint32_t p = bexcl, kmax = 0, kmin = 0;  // kmin: complement of the smallest key
 #pragma unroll
     for (int j = 0; j < KPB; ++j) {
       const int col = j * kRecThreads + tid;
       uint32_t key = 0u;
       if constexpr (kAll) {
         if (col < nv) key = score_key(listf[col]);
-      } else if ((masks >> (8 + j)) & 1u) {
-        const bool cj = (masks >> j) & 1u;
-        key = cj ? score_key(listf[p]) : hik[j];
-        p += cj ? 1u : 0u;
+      } else if ((masks >> j) & 1u) {
+        key = score_key(listf[p++]);
         if (key < tau) key = 0u;
       }
       v[j] = key == 0u ? 0ull : (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(~static_cast<uint32_t>(col));
@@ -1429,13 +1419,11 @@ __global__ __launch_bounds__(kRecThreads, 4) void topk_recompute_kernel(const fl
     // (kLong: every score of the segment is in registers since before the barriers above)
     uint32_t *dk = reinterpret_cast<uint32_t *>(const_cast<float *>(srow)) + c0;
     uint32_t *dc = reinterpret_cast<uint32_t *>(rc.bounds + row * ld) + c0;
-    uint32_t pos = bexcl >> 16, p = bexcl & 0xFFFFu;
+    uint32_t pos = bexcl;
 #pragma unroll
     for (int j = 0; j < KPB; ++j) {
-      if ((masks >> (8 + j)) & 1u) {
-        const bool cj = (masks >> j) & 1u;
-        uint32_t key = cj ? score_key(listf[p]) : hik[j];
-        p += cj ? 1u : 0u;
+      if ((masks >> j) & 1u) {
+        uint32_t key = score_key(listf[pos]);
         if (key < tau) key = 0u;
         const uint32_t col = static_cast<uint32_t>(c0 + j * kRecThreads + tid);
         if constexpr (kLong) {
@@ -1763,8 +1751,8 @@ int64_t ks::topk_bounded_part_capacity(int64_t rows, int64_t T) {
 }
 
 // Diagnostic entry (not part of the public header) of the bounded top-k, for timing it alone: scores and
-// bounds from ks_dbg_indexer_scores_bounded over rotated q / k (with their row statistics); the scores that
-// are recomputed are rewritten in place (bound 0).  ratio 1, int32 output.  part: part_cap 64-bit slots, at
+// bounds from ks_dbg_indexer_scores_bounded over rotated q / k (with their row statistics); both are overwritten
+// (rows past 8192 columns, and rows whose lists outgrow LDS).  ratio 1, int32 output.  part: part_cap 64-bit slots, at
 // least ks_dbg_topk_bounded_slots(B S, T) of them, as ks_dbg_indexer_scores_bounded left them (the rows' histogram
 // scales).  kmax is not read.
 extern "C" int ks_dbg_indexer_topk_bounded(float *scores, float *bounds, const float *kmax, const uint16_t *q,
