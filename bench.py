@@ -220,8 +220,8 @@ def run_indexer(cfg, steps, warmup, do_cpu, cpu_budget):
     kmax = torch.empty(B, (T + 255) // 256, dtype=torch.float32, device="cuda")
     idx = torch.empty(B, S, min(p["k_top"], T), dtype=torch.int32, device="cuda")
     lib = _lib.load()
-    # the bounded selection's workspace: lists, bucket counts, list lengths; where the fused call counts the
-    # rows in the score kernel (a one-round score grid), so does the diagnostic one, into this zeroed region
+    # the bounded selection's workspace: lists, bucket counts, states (the score kernel leaves the rows' histogram
+    # scales in it); kmax is not read
     part = torch.zeros(lib.ks_dbg_topk_bounded_slots(B * S, T), dtype=torch.int64, device="cuda")
     (qn, qs), (kn, ks_) = stats
     stream = torch.cuda.current_stream().cuda_stream
@@ -245,9 +245,8 @@ def run_indexer(cfg, steps, warmup, do_cpu, cpu_budget):
                                          T, 1, p["start_pos"], 1, stream), "scores")
 
     score_us = _events_avg(scores_bounded, steps, warmup)
-    # the bounded top-k writes its recomputed scores back (bound 0) and appends to its lists, so every timed
-    # call starts from a fresh copy of one score kernel call's output (scores, bounds, counts on a zeroed
-    # workspace); the copies are timed alone and subtracted
+    # the bounded top-k may overwrite scores, bounds and its workspace, so every timed call starts from a fresh
+    # copy of one score kernel call's output; the copies are timed alone and subtracted
     part.zero_()
     scores_bounded()
     out0, bnd0, part0 = out.clone(), bnd.clone(), part.clone()

@@ -675,23 +675,17 @@ __global__ __launch_bounds__(64 * NW, 1) void sparse_attn_mla_kernel(
   const uint32_t kb_lds = __builtin_amdgcn_readfirstlane(lds_addr(&kb[0][0]));
   auto issue = [&](int c) {
     const int buf = c % NBUF;
-    // index reads together: one LDS latency
-    constexpr int BATCH = NJ <= 12 ? NJ : 9;
-    static_assert(NJ % BATCH == 0, "every batch lies inside the wave's NJ gathers");
+    int32_t r[NJ];  // the index reads together: one LDS latency
 #pragma unroll
-    for (int i0 = 0; i0 < NJ; i0 += BATCH) {
-      int32_t r[BATCH];
+    for (int i = 0; i < NJ; ++i) r[i] = sidx[c * kKC + (64 * (wave + NW * i) + lane) / UPR];
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) r[i] = sidx[c * kKC + (64 * (wave + NW * (i0 + i)) + lane) / UPR];
-#pragma unroll
-      for (int i = 0; i < BATCH; ++i) {
-        const int jj = wave + NW * (i0 + i);
-        const int sl = 64 * jj + lane;
-        const int key = sl / UPR;
-        const uint32_t voff =
-            static_cast<uint32_t>(r[i] < 0 ? 0 : r[i]) * (Sh::DQK * 2) + ((sl % UPR) ^ (key & 7)) * 16;
-        dma16((const void *)kvb, voff, kb_lds + (buf * Sh::BUF + 64 * jj * 8) * 2);
-      }
+    for (int i = 0; i < NJ; ++i) {
+      const int jj = wave + NW * i;
+      const int sl = 64 * jj + lane;
+      const int key = sl / UPR;
+      const uint32_t voff =
+          static_cast<uint32_t>(r[i] < 0 ? 0 : r[i]) * (Sh::DQK * 2) + ((sl % UPR) ^ (key & 7)) * 16;
+      dma16((const void *)kvb, voff, kb_lds + (buf * Sh::BUF + 64 * jj * 8) * 2);
     }
   };
   const int npre = nch < NBUF - 1 ? nch : NBUF - 1;

@@ -25,7 +25,7 @@ def _check(device, q, k, w, k_top, causal, start_pos, ratio=1, offset=0, rows=No
 
 # one to five queries (the few-queries form up to four); one key, a partial group of 64, a partial last workgroup;
 # 8192 and 8193 columns (counted by the recomputation / by the histogram launch); causal limits inside a group and before
-# the row's later groups; several groups per wave (B 9 x S 4 x T 16000)
+# the row's later groups
 @pytest.mark.parametrize("B,S,T,k_top,causal,start,ratio", [
     (1, 1, 1, 1, False, 0, 1), (2, 1, 63, 64, False, 0, 1), (3, 2, 65, 32, True, 30, 1), (1, 4, 511, 100, True, 508, 1),
     (2, 3, 1025, 512, False, 700, 1), (1, 1, 8192, 512, False, 8191, 1), (1, 2, 8193, 2048, True, 8191, 1),
