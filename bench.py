@@ -279,8 +279,7 @@ def run_indexer(cfg, steps, warmup, do_cpu, cpu_budget):
                        "topk_rows_kernel (plain, other shapes)": round(topk_us, 3)},
         "roofline": {"bound": "mfma", "kernel": "indexer_scores_kernel (bounded)", "achieved": round(achieved, 2),
                      "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
-                     "traffic": _traffic(f"indexer_scores_kernel<4, 128, false, true, true, false>@{cfg}")
-                     or _traffic(f"indexer_scores_kernel<4, 128, false, true, false, false>@{cfg}")},
+                     "traffic": _traffic(f"indexer_scores_kernel<4, 128, false, true, false, false>@{cfg}")},
         # the product's bounded top-k reads a score and a bound (8 B) per column; the plain one 4 B
         "topk_bounded_GBps": round(S * T * 8 / (topkb_us * 1e-6) / 1e9, 1),
         "topk_plain_GBps": round(S * T * 4 / (topk_us * 1e-6) / 1e9, 1),
