@@ -582,8 +582,7 @@ def _bounded_scores_gpu(q, k, w, start_pos):
 def test_bounded_scores_contain_exact(device, dist, S, T):
     # the bound-mode score kernel's contract, checked score by score against the oracle's exact scores on the
     # valid (unmasked) columns: U >= 0, the stored score exact (bit for bit) where U = 0, |exact - S| <= U elsewhere.  The last
-    # shape's grid (17 query groups x 16 key blocks) exceeds one round of the GPU, so it runs the non-counting
-    # form of the kernel; the others run the counting form.
+    # shape's grid (17 query groups x 16 key blocks) exceeds one round of the GPU.
     g = torch.Generator().manual_seed(41 + S)
     q = torch.randn(1, S, 64, 128, generator=g)
     k = torch.randn(1, T, 128, generator=g)

@@ -7,6 +7,7 @@ import torch
 
 import oracle
 from kernelswift_amd import ops, workloads
+from tests.test_gpu_indexer import _bounded_scores_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -223,3 +224,26 @@ def test_long_lists_of_ties(device, S, T, k_top, causal, start):
     got = ops.indexer(q.to(device), k.to(device), w.to(device), tab.to(device), k_top, causal, start, 1, 0, 0, 64, True)
     want = oracle.indexer(_u16(q[:, rows]), _u16(k), w[:, rows].numpy(), tab.numpy(), k_top, causal, start, 1, 0, 0, 64, True)
     np.testing.assert_array_equal(got[:, rows].cpu().numpy().astype(np.int64), want)
+
+
+# the bound itself, score by score, in the few-queries form (up to four queries) and the other one: |exact - S| <= U with
+# U > 0; "subnormal": dots around the smallest bf16 steps under large weights
+@pytest.mark.parametrize("dist", ["normal", "midpoints", "scaled", "subnormal"])
+@pytest.mark.parametrize("S,T", [(1, 700), (4, 1100), (40, 1200)])
+def test_bounds_contain_exact_scores(device, dist, S, T):
+    g = torch.Generator().manual_seed(S + T)
+    q, k = torch.randn(1, S, 64, 128, generator=g), torch.randn(1, T, 128, generator=g)
+    w = torch.randn(1, S, 64, generator=g) / 8
+    if dist == "midpoints":
+        q, k = torch.randint(-3, 4, q.shape, generator=g).float(), torch.randint(-3, 4, k.shape, generator=g).float()
+    elif dist == "scaled":
+        q = q * torch.exp2(torch.randint(-8, 9, (1, S, 64, 1), generator=g).float())
+        w = w * torch.exp2(torch.randint(-100, 60, (1, S, 64), generator=g).float())
+    elif dist == "subnormal":
+        q, k, w = q * 2.0 ** -66, k * 2.0 ** -69, w * 2.0 ** 33
+    q, k = q.bfloat16(), k.bfloat16()
+    print(f"[case] bounds contain exact scores {dist} S={S} T={T}", flush=True)
+    got, u = _bounded_scores_gpu(q, k, w, T)  # every column is live
+    want = oracle.indexer_scores(_u16(q), _u16(k), w.numpy(), True, T).astype(np.float64)
+    assert (u > 0).all() and np.isfinite(u).all()
+    assert (np.abs(want - got) <= u).all()
