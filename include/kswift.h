@@ -290,8 +290,11 @@ int ks_mhc_post(const uint16_t *x, const uint16_t *f, const float *res_logits,
  *   res = alpha[2] z[8..23] + base[8..23],
  * then h as ks_mhc_pre.  phi: f32 [4 C, 24]; alpha: f32 [3]; base: f32 [24];
  * post_logits f32 [N, 4] and res_logits f32 [N, 4, 4] are written for
- * ks_mhc_post.  fp32 sums of exact products; x and h 16-byte aligned.
- * workspace: ks_mhc_input_workspace_size(N, C) bytes. */
+ * ks_mhc_post.  fp32 sums of exact products (of the plain streams, scaled
+ * afterwards; tokens whose products leave the fp32 range are normalised
+ * first); x and h 16-byte aligned.
+ * workspace: ks_mhc_input_workspace_size(N, C) bytes (0 for an N or C that
+ * ks_mhc_input refuses). */
 size_t ks_mhc_input_workspace_size(int64_t N, int64_t C);
 int ks_mhc_input(const uint16_t *x, const float *phi, const float *alpha,
                  const float *base, uint16_t *h, float *post_logits,
