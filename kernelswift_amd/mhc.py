@@ -47,21 +47,22 @@ class HyperConnection(nn.Module):
 
     def _fused(self, x: torch.Tensor) -> bool:
         """Whether `pre` may form the logits inside the kernel: plain contiguous tensors of the kernel's types on one
-        GPU, with no gradient (reverse or forward mode), autocast, vmap or trace that has to see the torch operations,
-        and no `logits` of a subclass's or the instance's own."""
+        GPU, with no gradient (reverse or forward mode), autocast, vmap, trace or dispatch mode that has to see the torch
+        operations, and no `logits` of a subclass's or the instance's own."""
         if type(self).logits is not HyperConnection.logits or "logits" in self.__dict__:
             return False
         if not isinstance(self.norm_eps, (int, float)):
             return False
         ts = (x, self.phi, self.alpha, self.base)
+        if any(type(t) not in (torch.Tensor, nn.Parameter) for t in ts):  # a tracer's proxies too, before any is asked
+            return False
         if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.maybe_current_level() is not None:
             return False
-        if torch.is_autocast_enabled() or forward_ad._current_level >= 0:
+        if torch.is_autocast_enabled() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0:
             return False
         if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
             return False
-        return (all(type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.device == x.device and t.is_contiguous()
-                    for t in ts)
+        return (all(t.is_cuda and t.device == x.device and t.is_contiguous() for t in ts)
                 and x.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[0] > 0 and x.shape[1:] == (4, self.dim)
                 and self.dim % 8 == 0 and all(t.dtype == torch.float32 for t in ts[1:])
                 and self.phi.shape == (4 * self.dim, 24) and self.alpha.shape == (3,) and self.base.shape == (24,))

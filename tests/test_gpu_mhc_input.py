@@ -136,6 +136,24 @@ def test_own_logits_are_used(device):
             torch.testing.assert_close(r, res + 3.0, rtol=1e-5, atol=1e-5)
 
 
+def test_dispatch_modes_see_the_logits(device):
+    from torch.utils._python_dispatch import TorchDispatchMode
+    seen = []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    hc = _block(device, 64, 7)
+    x = torch.randn(4, 4, 64).bfloat16().to(device)
+    want = hc.pre(x)
+    with torch.no_grad(), Seen():
+        got = hc.pre(x)
+    assert any("mm" in f for f in seen) and not any("mhc_input" in f for f in seen)
+    torch.testing.assert_close(got[1], want[1], rtol=1e-5, atol=1e-5)
+
+
 def test_mhc_input_errors(device):
     hc = _block(device, 64, 4)
     x = torch.zeros(2, 4, 64, dtype=torch.bfloat16, device=device)
